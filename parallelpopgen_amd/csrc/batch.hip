@@ -42,6 +42,7 @@
  * result is bit for bit the result gf_run gives for it alone.
  */
 #include "gf_kernels.hpp"
+#include "gf_const_drift.hpp"
 #include "gf_runtime.hpp"
 #include "gf_spectrum.hpp"
 
@@ -91,6 +92,8 @@ struct alignas(16) BSim {
     /* this block (k_bt_rows) */
     int Kb, nnew, tiles;
     int need;     /* tiles a stalled simulation's block needs */
+    int counted;  /* Nc is in const_drift's range */
+    int resized;  /* the start is counted in another number of chromosomes */
 };
 
 /* device pointers of a layout (kernel argument, fixed while a graph lives) */
@@ -102,6 +105,7 @@ struct BBufs {
     unsigned int *cnt;            /* survivors per output tile */
     GenRow<1> *rows;              /* [S][BK_MAX] */
     const int *tile_sim;          /* tile -> simulation */
+    const PoisTable *pois;        /* [S] draw tables */
     unsigned long long *live;     /* 64 partial sums of live mutation-generations */
     int *K;                       /* block length (device word: the tuner changes it between replays) */
     int ntiles, S;
@@ -115,8 +119,16 @@ __device__ __forceinline__ BSim load_bsim(const BSim *p) {
     b.F = c.F; b.h = c.h; b.mu = c.mu; b.s = c.s; b.L = c.L; b.c1 = c.c1; b.c2 = c.c2;
     b.newfreq = c.newfreq; b.fN = c.fN; b.k0 = c.k0; b.k1 = c.k1;
     b.t0 = c.t0; b.nt = c.nt; b.p0 = c.p0; b.g = c.g; b.M = c.M; b.T = c.T; b.cur = c.cur;
-    b.status = c.status; b.Kb = c.Kb; b.nnew = c.nnew; b.tiles = c.tiles;
+    b.counted = c.counted; b.resized = c.resized; b.status = c.status; b.Kb = c.Kb; b.nnew = c.nnew; b.tiles = c.tiles;
     return b;
+}
+
+/* ---- draw tables, one wave per simulation (once per batch) ---- */
+static __global__ __launch_bounds__(WG) void k_bt_pois(const BSim *__restrict__ sims, int S, PoisTable *__restrict__ out) {
+    const int s = (int)blockIdx.x * (WG / 64) + ((int)threadIdx.x >> 6);
+    if (s >= S || !sims[s].counted) return;   /* the whole wave */
+    const BSim &b = sims[s];
+    pois_table_build(ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral}, out + s);
 }
 
 /* ---- 1. rows and new-mutation counts of the next block, one thread per simulation ---- */
@@ -161,7 +173,10 @@ static __global__ void k_bt_rows(BSim *__restrict__ sims, BBufs B) {
     b.tiles = tiles;
 }
 
-/* ---- 2. drift + new mutations + tile-local compaction of every simulation's block ---- */
+/* ---- 2. drift + new mutations + tile-local compaction of every simulation's block ----
+ * CONST: the simulations whose chromosome number const_drift covers; the
+ * others run in the second instance, launched only for a batch that has any. */
+template <bool CONST>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_bt_advance(const BSim *__restrict__ sims,
                                                                                           const BBufs B) {
     const int lane = threadIdx.x & 63;
@@ -170,6 +185,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     __shared__ int sh_pre[WG + 1];
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
     __shared__ ExpSeg sh_eneg[GF_EXPNEG_SEGMENTS];
+    __shared__ uint4 sh_pois[CONST ? POIS_ROWS * POIS_ROW_VECS : 1];
     load_draw_tables(sh_ncdf, sh_eneg);   /* published by the tile loop's first barrier */
     uint64_t live = 0;          /* this thread's slots' live mutation-generations */
     for (int gt = blockIdx.x;; gt += gridDim.x) {
@@ -178,7 +194,11 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const int s = *as_const(B.tile_sim + gt);
         const BSim S = load_bsim(sims + s);
         const int j = gt - S.t0;
-        if (j >= S.tiles) continue;
+        if (j >= S.tiles || (bool)S.counted != CONST) continue;
+        if constexpr (CONST) {
+            if (threadIdx.x < POIS_ROWS * POIS_ROW_VECS) sh_pois[threadIdx.x] = B.pois[s].v[threadIdx.x];
+        }
+        const int jn = CONST ? as_const(B.pois + s)->jn : 1;
         /* the two buffers by selects (indexing the argument's arrays with
          * a run-time value would put them in scratch memory) */
         const bool c1 = S.cur != 0;
@@ -196,51 +216,62 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const GenRow<1> *rows = B.rows + (size_t)s * BK_MAX;
         int s0 = 0;
         if (!dense && j * WG < M0) s0 = load_frag_window(j, src0_in, pre_in, S.T, sh_pre);
+        else if (CONST) __syncthreads();   /* sh_pois */
         float x = 0.0f;
-        int ogen = 0, opop = 0, born = -1;
+        int jc = 0, born = -1;
         uint32_t tid = 0;
         gf_mutid id;
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
+        const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral};
+        /* the start is counted in generation 0's chromosomes */
+        const bool first_freq = S.g == 0 && S.resized;
         if (valid) {
             if (li < M0) {
                 const int64_t src = base + (dense ? (int64_t)li : frag_slot(li, s0, sh_pre, pre_in, S.T));
                 x = freq_in[src];
                 id = ids_in[src];
-                ogen = id.origin_generation;
-                opop = id.origin_population;
                 tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
+                jc = const_count(x, first_freq, C);
             } else {
                 const int rel = li - M0;
                 int tb, pb;
                 find_birth<1>(rows, S.Kb, rel, tb, pb);
                 born = tb;
-                ogen = S.g + 1 + tb;
-                opop = pb;
-                tid = (uint32_t)(rel - rows[tb].newcum[pb] + 1);
-                x = rows[tb].newfreq[0];
-                id.origin_generation = ogen;
-                id.origin_population = opop;
+                tid = (uint32_t)(rel - rows[tb].newcum[0] + 1);
+                id.origin_generation = S.g + 1 + tb;
                 id.origin_threadID = (int32_t)tid;
-                id.reserved = 0;
+                jc = 1;
+                x = S.newfreq;
             }
         }
-        const auto *crows = as_const(rows);
-        u32x4 rc[1];
-        bool keep = false;
-        int kfirst = KMAX, klast = -1;
-        for (int t = 0; t < S.Kb; t++) {
-            const auto &R = crows[t];
-            const int g = S.g + 1 + t;
-            if (valid && born < t) {
-                const bool refresh = ((g & 3) == 0) || (t == born + 1);
-                generation_update<1>(&x, R, g, refresh, rc, S.k0, S.k1, tid, ogen, opop, LinearSel(), sh_ncdf, sh_eneg);
+        bool keep;
+        if constexpr (CONST) {
+            int klast;
+            const_drift(jc, klast, x, first_freq, born, S.Kb, S.g, S.k0, S.k1, tid, id.origin_generation, 0, C, jn,
+                        sh_pois, sh_ncdf, sh_eneg);
+            if (klast >= 0) live += (uint64_t)(klast - (born < 0 ? 0 : born) + 1);
+            keep = klast == S.Kb - 1;
+            x = quot_count((float)jc, C.N, C.r);
+        } else {
+            const auto *crows = as_const(rows);
+            u32x4 rc[1];
+            keep = false;
+            int kfirst = KMAX, klast = -1;
+            for (int t = 0; t < S.Kb; t++) {
+                const auto &R = crows[t];
+                const int g = S.g + 1 + t;
+                if (valid && born < t) {
+                    const bool refresh = ((g & 3) == 0) || (t == born + 1);
+                    generation_update<1>(&x, R, g, refresh, rc, S.k0, S.k1, tid, id.origin_generation, 0, LinearSel(),
+                                         sh_ncdf, sh_eneg);
+                }
+                keep = valid && born <= t && keep_rule<1>(&x, R.present_mask, false);
+                /* one population: kept over one run of generations (lost and
+                 * fixed are absorbing) */
+                if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
             }
-            keep = valid && born <= t && keep_rule<1>(&x, R.present_mask, false);
-            /* one population: kept over one run of generations (lost and
-             * fixed are absorbing) */
-            if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
+            if (klast >= 0) live += (uint64_t)(klast - kfirst + 1);
         }
-        if (klast >= 0) live += (uint64_t)(klast - kfirst + 1);
         /* tile-local stable packing into the other buffer */
         const uint64_t kb = __ballot(keep);
         if (lane == 0) sh_wcount[w] = (unsigned int)__popcll(kb);
@@ -522,6 +553,8 @@ struct BatchRun {
     DevBuf<int> pre[2], src0[2], tile_sim, d_K;
     DevBuf<unsigned int> cnt;
     DevBuf<GenRow<1>> rows;
+    DevBuf<PoisTable> pois;
+    bool any_counted = false, any_general = false;
     DevBuf<unsigned long long> live;
     DevBuf<float *> d_fptr;
     DevBuf<gf_mutid *> d_iptr;
@@ -569,6 +602,10 @@ struct BatchRun {
             d.c2 = (b.F + (2.0f * b.h)) - ((2.0f * b.h) * b.F);
             d.newfreq = d.Nc > 0 ? 1.0f / (float)d.Nc : 0.0f;
             d.neutral = b.s == 0.0f;
+            d.counted = const_drift_range(d.Nc);
+            d.resized = d.Nc != (b.N > 0 ? nchrom(b.N, b.F) : 0);
+            any_counted |= d.counted != 0;
+            any_general |= d.counted == 0;
             d.T = -1;
             d.status = d.G > 0 ? BS_ACTIVE : BS_DONE;
             if (b.N < 0 || N1 < 0 || b.F < 0 || b.F > 1 || b.mu < 0 || b.num_generations < 0) {
@@ -677,6 +714,10 @@ struct BatchRun {
             GF_HIP(hipGetLastError());
         }
         GF_HIP(hipMemcpyAsync(d_sims.p, host.data(), (size_t)S * sizeof(BSim), hipMemcpyHostToDevice, st));
+        GF_TRY(pois.alloc(S));
+        if (any_counted)
+            hipLaunchKernelGGL(k_bt_pois, dim3((S + 3) / 4), dim3(WG), 0, st, (const BSim *)d_sims.p, S, pois.p);
+        GF_HIP(hipGetLastError());
         GF_HIP(hipStreamSynchronize(st));
         return GF_OK;
     }
@@ -715,6 +756,7 @@ struct BatchRun {
         B.cnt = cnt.p;
         B.rows = rows.p;
         B.tile_sim = tile_sim.p;
+        B.pois = pois.p;
         B.live = live.p;
         B.K = d_K.p;
         B.ntiles = (int)ntiles;
@@ -730,7 +772,8 @@ struct BatchRun {
         const int grid = std::max(1, std::min<int>((int)ntiles, num_cus() * 8));
         GF_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
         hipLaunchKernelGGL(k_bt_rows, dim3((S + 127) / 128), dim3(128), 0, st, d_sims.p, B);
-        hipLaunchKernelGGL(k_bt_advance, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
+        if (any_counted) hipLaunchKernelGGL(k_bt_advance<true>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
+        if (any_general) hipLaunchKernelGGL(k_bt_advance<false>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
         hipLaunchKernelGGL(k_bt_scan, dim3(S), dim3(256), 0, st, d_sims.p, B);
         hipLaunchKernelGGL(k_bt_status, dim3(1), dim3(1024), 0, st, (const BSim *)d_sims.p, B, h_status.p);
         const hipError_t e = hipStreamEndCapture(st, &graph);

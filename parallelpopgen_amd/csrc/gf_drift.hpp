@@ -114,6 +114,16 @@ struct FunctorSel {
     __device__ __forceinline__ float operator()(int p, int g, float x, const Row &) const { return f(p, g, x); }
 };
 
+/* Eq. 13: (x + s x (x + c1 (1-x))) / (1 + s x (x + c2 (1-x))), s >= -1 */
+GF_HD float selected_freq(float x, float s, float c1, float c2) {
+    GF_STRICT_FP
+    const float om = 1.0f - x;
+    const float sx = s * x;
+    const float num = __builtin_fmaf(sx, __builtin_fmaf(c1, om, x), x);
+    const float den = __builtin_fmaf(sx, __builtin_fmaf(c2, om, x), 1.0f);
+    return num / den;
+}
+
 /* ---------------- migration, selection and drift of one generation ----------------
  * Reference migration_selection_drift (go_fish_impl.cuh:93-124): each
  * population's frequency after migration (weighted sum over the source
@@ -151,12 +161,7 @@ __device__ __forceinline__ void generation_update(float *x, const Row &R, int g,
         } else {
             float s = sel(p, g, im, R);
             s = s > -1.0f ? s : -1.0f;
-            /* Eq. 13: (x + s x (x + c1 (1-x))) / (1 + s x (x + c2 (1-x))) */
-            const float om = 1.0f - im;
-            const float sx = s * im;
-            const float num = __builtin_fmaf(sx, __builtin_fmaf(R.c1[p], om, im), im);
-            const float den = __builtin_fmaf(sx, __builtin_fmaf(R.c2[p], om, im), 1.0f);
-            xs = num / den;
+            xs = selected_freq(im, s, R.c1[p], R.c2[p]);
         }
         const float N = R.fN[p];
         const float mean = xs * N;

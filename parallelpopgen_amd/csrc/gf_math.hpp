@@ -403,6 +403,16 @@ GF_HD int round_away_nonneg(float v) {
     return f2i_sat(v) + (d >= 0.5f ? 1 : 0);
 }
 
+/* the rounded normal approximation of the binomial draw, for the caller's
+ * clamp to [0, N].  u01 gives 2^-33 <= u <= 1 (never NaN): of
+ * normcdfinv_tab's clamps only the top one can act. */
+GF_HD float u01_top(float u) { return u > 0.99999994039535522f ? 0.99999994039535522f : u; }
+
+GF_HD int binom_normal(float u, float mean, float var, const NcdfSeg *ncdf) {
+    GF_STRICT_FP
+    return round_away_nonneg(normcdfinv_core(ncdf, u01_top(u)) * sqrt_pos(var) + mean);
+}
+
 /* approximate binomial draw (reference shared.cu:10-18): the two Poisson
  * (or binomial, N < 100) tails share one CDF inversion; the rest is the
  * rounded normal approximation.  A mean of exactly 0 or N (lost or fixed:
@@ -422,10 +432,7 @@ GF_HD int binom_draw(uint32_t bits, float mean, float var, float N, const NcdfSe
         if (m != 0.0f) k = (N < 100.0f) ? binomcdfinv(u, m, m / N, N) : poiscdfinv_tail(u, m, etab);
         return lo ? k : f2i_sat(N - (float)k);
     }
-    /* u01 gives 2^-33 <= u <= 1 (never NaN): of normcdfinv_tab's clamps
-     * only the top one can act, and the result is the same */
-    return round_away_nonneg(normcdfinv_core(ncdf, u > 0.99999994039535522f ? 0.99999994039535522f : u) *
-                                 sqrt_pos(var) + mean);
+    return binom_normal(u, mean, var, ncdf);
 }
 
 /* approximate Poisson draw (reference shared.cuh:251-256) */

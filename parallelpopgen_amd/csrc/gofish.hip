@@ -11,6 +11,7 @@
  * and at time samples (device-to-host copy).
  */
 #include "gf_kernels.hpp"
+#include "gf_const_drift.hpp"
 #include "gf_runtime.hpp"
 #include "gf_spectrum.hpp"
 
@@ -205,6 +206,8 @@ struct PlainRun {
     int64_t launches = 0;
     int64_t M_bound = 0;                /* upper bound of the current slot count */
     int64_t last_new = 0;               /* new slots of the most recent launch */
+    DevBuf<PoisTable> d_pois;           /* draw table of row pois_row's model (k_advance_const) */
+    int pois_row = -1;
 
     int plan() {
         const int Pn = d->num_populations;
@@ -520,6 +523,38 @@ struct PlainRun {
         return ensure_capacity(need);
     }
 
+    static bool same_model(const GenRow<P> &a, const GenRow<P> &b) {
+        return a.Nc[0] == b.Nc[0] && a.neutral_mask == b.neutral_mask && a.sa[0] == b.sa[0] && a.sb[0] == b.sb[0] &&
+               a.c1[0] == b.c1[0] && a.c2[0] == b.c2[0];
+    }
+
+    /* whether generations t_first .. t_first+K-1 run as k_advance_const: one
+     * population, the library's own selection form, one model throughout,
+     * and a state counted in some number of chromosomes (every state but a
+     * previous run's, whose frequencies are the caller's) */
+    bool const_model(int t_first, int K) const {
+        if (P != 1 || hooks || (t_first == 1 && d->init_mode == GF_INIT_PREV)) return false;
+        if (!const_drift_range(rows[t_first].Nc[0]) || !(rows[t_first].present_mask & 1)) return false;
+        for (int t = t_first + 1; t < t_first + K; t++)
+            if (!same_model(rows[t], rows[t_first])) return false;
+        return true;
+    }
+
+    int advance_const(const FusedLaunch &F, const SegLaunch<P> &sl, int t_first, int grid) {
+        if constexpr (P == 1) {
+            if (pois_row < 0 || !same_model(rows[pois_row], rows[t_first])) {
+                GF_TRY(d_pois.alloc(1));
+                hipLaunchKernelGGL(k_pois_table, dim3(1), dim3(64), 0, st, d_rows.p + t_first, d_pois.p);
+                GF_HIP(hipGetLastError());
+                pois_row = t_first;
+            }
+            const int Nc_prev = t_first > 1 ? rows[t_first - 1].Nc[0] : nchrom(d->params[0].N, d->params[0].F);
+            hipLaunchKernelGGL(k_advance_const, dim3(grid), dim3(WG), 0, st, F, sl, d_pois.p,
+                               Nc_prev == rows[t_first].Nc[0] ? 0 : 1);
+        }
+        return GF_OK;
+    }
+
     /* Advance generations t_first .. t_first+K-1 in one fused launch
      * (reference migration_selection_drift + add_new_mutations per
      * generation, go_fish_impl.cuh:645-684, and, when `compact`,
@@ -564,6 +599,8 @@ struct PlainRun {
         if (hooks) {
             const int32_t rc = hooks->advance(hooks->user, P, &F, &sl, grid, (void *)st);
             if (rc != GF_OK) { set_error("run_sim: selection advance hook failed"); return rc; }
+        } else if (const_model(t_first, K)) {
+            GF_TRY(advance_const(F, sl, t_first, grid));
         } else {
             hipLaunchKernelGGL((k_advance_fused<P, LinearSel>), dim3(grid), dim3(WG), 0, st, F, sl, LinearSel());
         }
