@@ -81,7 +81,7 @@ struct alignas(16) BSim {
     int Nc, N, G, neutral;
     float F, h, mu, s, L, c1, c2, newfreq, fN;
     uint32_t k0, k1;
-    /* layout: tiles [t0, t0 + nt) of both buffers, prefix entries [p0, p0 + nt] */
+    /* layout: tiles [t0, t0 + nt) of both buffers, prefix entries [p0, p0 + nt + PRE_PAD) */
     int t0, nt, p0;
     /* progress */
     int g;        /* generations done */
@@ -92,6 +92,7 @@ struct alignas(16) BSim {
     /* this block (k_bt_rows) */
     int Kb, nnew, tiles;
     int need;     /* tiles a stalled simulation's block needs */
+    int mid;      /* mid_selection of the model */
     int counted;  /* Nc is in const_drift's range */
     int resized;  /* the start is counted in another number of chromosomes */
 };
@@ -100,7 +101,7 @@ struct alignas(16) BSim {
 struct BBufs {
     float *freq[2];
     gf_mutid *ids[2];
-    int *pre[2];                  /* per simulation nt + 1 entries from p0 */
+    int *pre[2];                  /* per simulation nt + PRE_PAD entries from p0 */
     int *src0[2];                 /* per simulation nt entries from t0 */
     unsigned int *cnt;            /* survivors per output tile */
     GenRow<1> *rows;              /* [S][BK_MAX] */
@@ -119,7 +120,7 @@ __device__ __forceinline__ BSim load_bsim(const BSim *p) {
     b.F = c.F; b.h = c.h; b.mu = c.mu; b.s = c.s; b.L = c.L; b.c1 = c.c1; b.c2 = c.c2;
     b.newfreq = c.newfreq; b.fN = c.fN; b.k0 = c.k0; b.k1 = c.k1;
     b.t0 = c.t0; b.nt = c.nt; b.p0 = c.p0; b.g = c.g; b.M = c.M; b.T = c.T; b.cur = c.cur;
-    b.counted = c.counted; b.resized = c.resized; b.status = c.status; b.Kb = c.Kb; b.nnew = c.nnew; b.tiles = c.tiles;
+    b.mid = c.mid; b.counted = c.counted; b.resized = c.resized; b.status = c.status; b.Kb = c.Kb; b.nnew = c.nnew; b.tiles = c.tiles;
     return b;
 }
 
@@ -128,7 +129,7 @@ static __global__ __launch_bounds__(WG) void k_bt_pois(const BSim *__restrict__ 
     const int s = (int)blockIdx.x * (WG / 64) + ((int)threadIdx.x >> 6);
     if (s >= S || !sims[s].counted) return;   /* the whole wave */
     const BSim &b = sims[s];
-    pois_table_build(ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral}, out + s);
+    pois_table_build(ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral, b.mid}, out + s);
 }
 
 /* ---- 1. rows and new-mutation counts of the next block, one thread per simulation ---- */
@@ -180,9 +181,8 @@ template <bool CONST>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_bt_advance(const BSim *__restrict__ sims,
                                                                                           const BBufs B) {
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
+    const int w = wave_index();
     __shared__ unsigned int sh_wcount[WG / 64];
-    __shared__ int sh_pre[WG + 1];
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
     __shared__ ExpSeg sh_eneg[GF_EXPNEG_SEGMENTS];
     __shared__ uint4 sh_pois[CONST ? POIS_ROWS * POIS_ROW_VECS : 1];
@@ -214,22 +214,22 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const int li = j * WG + (int)threadIdx.x;
         const bool valid = li < Mend;
         const GenRow<1> *rows = B.rows + (size_t)s * BK_MAX;
-        int s0 = 0;
-        if (!dense && j * WG < M0) s0 = load_frag_window(j, src0_in, pre_in, S.T, sh_pre);
-        else if (CONST) __syncthreads();   /* sh_pois */
+        const int first = j * WG + w * 64;   /* the wave's first index */
+        int64_t src = li;
+        if (!dense && first < M0) src = frag_slot(li, first, j, src0_in, pre_in, S.T);
+        if (CONST) __syncthreads();   /* sh_pois */
         float x = 0.0f;
         int jc = 0, born = -1;
         uint32_t tid = 0;
         gf_mutid id;
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
-        const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral};
+        const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral, S.mid};
         /* the start is counted in generation 0's chromosomes */
         const bool first_freq = S.g == 0 && S.resized;
         if (valid) {
             if (li < M0) {
-                const int64_t src = base + (dense ? (int64_t)li : frag_slot(li, s0, sh_pre, pre_in, S.T));
-                x = freq_in[src];
-                id = ids_in[src];
+                x = freq_in[base + src];
+                id = ids_in[base + src];
                 tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
                 jc = const_count(x, first_freq, C);
             } else {
@@ -348,7 +348,7 @@ static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims,
         __syncthreads();
     }
     if (threadIdx.x == 0) {
-        pre[T] = carry;
+        for (int k = 0; k < PRE_PAD; k++) pre[T + k] = carry;
         BSim &r = sims[s];
         r.M = carry;
         r.T = T;
@@ -399,9 +399,8 @@ static __global__ __launch_bounds__(WG) void k_bt_move(const BMove *__restrict__
                                                        float *const *__restrict__ freq_old,
                                                        gf_mutid *const *__restrict__ ids_old,
                                                        float *__restrict__ freq_new, gf_mutid *__restrict__ ids_new) {
-    __shared__ int sh_pre[WG + 1];
+    const int w = wave_index();
     for (int gt = blockIdx.x; gt < ntiles; gt += gridDim.x) {
-        __syncthreads();
         int lo = 0, hi = nmv - 1;   /* last move whose first tile <= gt */
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -410,10 +409,11 @@ static __global__ __launch_bounds__(WG) void k_bt_move(const BMove *__restrict__
         const BMove m = mv[lo];
         const int j = gt - m.tile_first;
         const int li = j * WG + (int)threadIdx.x;
-        int s0 = 0;
-        if (m.pre && j * WG < m.M) s0 = load_frag_window(j, m.src0, m.pre, m.T, sh_pre);
+        const int first = j * WG + w * 64;
+        int64_t src = li;
+        if (m.pre && first < m.M) src = frag_slot(li, first, j, m.src0, m.pre, m.T);
         if (li < m.M) {
-            const int64_t src = m.src_base + (m.pre ? frag_slot(li, s0, sh_pre, m.pre, m.T) : (int64_t)li);
+            src += m.src_base;
             freq_new[m.dst_base + li] = freq_old[m.cur][src];
             ids_new[m.dst_base + li] = ids_old[m.cur][src];
         }
@@ -602,6 +602,7 @@ struct BatchRun {
             d.c2 = (b.F + (2.0f * b.h)) - ((2.0f * b.h) * b.F);
             d.newfreq = d.Nc > 0 ? 1.0f / (float)d.Nc : 0.0f;
             d.neutral = b.s == 0.0f;
+            d.mid = mid_selection(0.0f, b.s, b.F, b.h);
             d.counted = const_drift_range(d.Nc);
             d.resized = d.Nc != (b.N > 0 ? nchrom(b.N, b.F) : 0);
             any_counted |= d.counted != 0;
@@ -689,7 +690,7 @@ struct BatchRun {
             const int nt = (int)std::ceil((double)g_region_scale * tiles_for(d.M, lam, Kmax + grow));
             d.nt = std::max(nt, (int)((d.M + WG - 1) / WG));
             t += d.nt;
-            pcount++;
+            pcount += PRE_PAD;
             layout.push_back(s);
             if (t > 2000000000LL / WG) { set_error("gf_batch_run: more than 2e9 slots"); return GF_ERR_UNSUPPORTED; }
         }
@@ -729,7 +730,7 @@ struct BatchRun {
         for (int b = 0; b < 2; b++) {
             GF_TRY(freq[b].alloc(slots));
             GF_TRY(ids[b].alloc(slots));
-            GF_TRY(pre[b].alloc((size_t)t + layout.size() + 1));
+            GF_TRY(pre[b].alloc((size_t)t + PRE_PAD * std::max<size_t>(layout.size(), 1)));
             GF_TRY(src0[b].alloc((size_t)std::max<int64_t>(t, 1)));
         }
         GF_TRY(cnt.alloc((size_t)std::max<int64_t>(t, 1)));
@@ -889,7 +890,7 @@ struct BatchRun {
             }
             b.nt = nt;
             b.t0 = (int)t;
-            b.p0 = (int)(t + k);
+            b.p0 = (int)(t + (int64_t)PRE_PAD * k);
             BMove m;
             m.src_base = (int64_t)old[s].t0 * WG;
             m.dst_base = (int64_t)b.t0 * WG;

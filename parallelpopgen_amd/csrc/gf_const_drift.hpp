@@ -16,8 +16,10 @@
  *
  * Bound: vector-ALU issue.  2.0e6 mutations of N = 1e5, gamma = -10, ten
  * generations a launch: 6.9e7 vector instructions by k_advance_fused, 5.2e7
- * here; the whole 5,000-generation run 64.1 -> 51.2 ms, a run of 8.4e3
- * mutations 2.14 -> 1.81 ms, a batch of 64 uneven simulations 566 -> 372 ms.
+ * with the table, 4.5e7 with the arithmetic of gf_math.hpp (div_mid,
+ * sqrt_pos, round_count) and the scalar gather (frag_slot) besides.  The
+ * 5,000-generation run: 64.1 -> 51.2 -> 46.3 ms; a run of 8.4e3 mutations
+ * 2.14 -> 1.81 -> 1.74 ms; a batch of 64 uneven simulations 428 -> 261 ms.
  */
 #ifndef GF_CONST_DRIFT_HPP_
 #define GF_CONST_DRIFT_HPP_
@@ -28,7 +30,7 @@ namespace gf {
 
 constexpr int POIS_ROWS = 8;    /* counts 1..8 */
 constexpr int POIS_TERMS = 24;  /* the inversion stops at term 24 at the latest for means up to 6 */
-constexpr int POIS_ROW_VECS = 6;
+constexpr int POIS_ROW_VECS = 8; /* 6 in use: a power of two, so a row's address is a shift */
 
 /* Row j - 1, with T[k] = the largest random word w with u01(w) <= S_k (the
  * k-th partial sum), 2^32 - 1 past the row's early exit: vector 0 = T[4],
@@ -44,7 +46,7 @@ struct ConstModel {
     int Nc;
     float N, r;      /* (float)Nc, RN(1/N) */
     float sa, sb, c1, c2;
-    int neutral;
+    int neutral, mid;   /* mid: selected_freq's */
 };
 
 /* chromosome numbers the count form covers: from 100 (below, the tails are
@@ -55,9 +57,10 @@ GF_HD bool const_drift_range(int Nc) { return Nc >= 100 && Nc <= (1 << 21); }
 GF_HD float const_selected(float x, const ConstModel &C) {
     GF_STRICT_FP
     if (C.neutral) return x;   /* s == 0: Eq. 13 reduces exactly to x */
-    float s = C.sa == 0.0f ? C.sb : C.sa * x + C.sb;
+    float s = C.sb;
+    if (C.sa != 0.0f) s = C.sa * x + C.sb;   /* 0 * x + sb is sb */
     s = s > -1.0f ? s : -1.0f;
-    return selected_freq(x, s, C.c1, C.c2);
+    return selected_freq(x, s, C.c1, C.c2, C.mid != 0);
 }
 
 /* row `row` of the table; true if its mean is in [0, 6] */
@@ -136,16 +139,15 @@ __device__ __forceinline__ void const_drift(int &j, int &klast, float x, bool fi
                 const float mean = xs * C.N;
                 const float var = (1.0f - xs) * mean;
                 const float u = u01(bits);
-                int d;
-                if (mean > 6.0f && mean < C.N - 6.0f) {
-                    d = binom_normal(u, mean, var, ncdf);
-                } else {   /* binom_draw's tails (N >= 100) outside the table: close to fixation, or from a frequency */
-                    const bool lo = mean <= 6.0f;
+                const bool lo = mean <= 6.0f;
+                if (lo || mean >= C.N - 6.0f) {   /* outside the table: close to fixation, or from a frequency */
                     const float m = lo ? mean : C.N - mean;
-                    const int k = m != 0.0f ? poiscdfinv_tail(u, m, etab) : 0;
-                    d = lo ? k : f2i_sat(C.N - (float)k);
+                    const int k = m != 0.0f ? poiscdfinv_tail(u, m, etab) : 0;   /* N >= 100 */
+                    const int d = lo ? k : f2i_sat(C.N - (float)k);
+                    j = min(max(d, 0), C.Nc);
+                } else {
+                    j = round_count(binom_normal(u, mean, var, ncdf), C.N);
                 }
-                j = min(max(d, 0), C.Nc);
             }
             if ((unsigned)(j - 1) < inner) klast = t;
         }
@@ -162,9 +164,10 @@ __device__ __forceinline__ int const_count(float x, bool first_freq, const Const
 }
 
 /* the table of rows[0]'s model, one wave */
-static __global__ __launch_bounds__(64) void k_pois_table(const GenRow<1> *__restrict__ row, PoisTable *__restrict__ out) {
+static __global__ __launch_bounds__(64) void k_pois_table(const GenRow<1> *__restrict__ row, int mid,
+                                                           PoisTable *__restrict__ out) {
     const auto &R = *as_const(row);
-    pois_table_build(ConstModel{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1}, out);
+    pois_table_build(ConstModel{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1, mid}, out);
 }
 
 /* k_advance_fused for one population and a launch whose model rows are all
@@ -172,11 +175,10 @@ static __global__ __launch_bounds__(64) void k_pois_table(const GenRow<1> *__res
 static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_advance_const(const FusedLaunch F,
                                                                                               const SegLaunch<1> S,
                                                                                               const PoisTable *__restrict__ ptab,
-                                                                                              int first_freq) {
+                                                                                              int mid, int first_freq) {
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
+    const int w = wave_index();
     __shared__ unsigned int sh_wcount[WG / 64];
-    __shared__ int sh_pre[WG + 1];
     __shared__ int sh_diff[KMAX + 1];
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
     __shared__ ExpSeg sh_eneg[GF_EXPNEG_SEGMENTS];
@@ -192,7 +194,7 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
     if (blockIdx.x == 0 && threadIdx.x == 0 && need_tiles > F.ntiles) *F.error = 2;   /* slots would be dropped */
     const GenRow<1> *rows = S.rows;
     const auto &R = *as_const(rows);
-    const ConstModel C{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1};
+    const ConstModel C{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1, mid};
     const int K = S.K;
     const int last_tile = need_tiles < F.ntiles ? need_tiles : F.ntiles;
     for (int tile = (int)blockIdx.x;; tile += (int)gridDim.x) {
@@ -200,8 +202,9 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
         if (tile >= last_tile) break;
         const int li = tile * WG + (int)threadIdx.x;
         const bool valid = li < Mend;
-        int s0 = 0;
-        if (!F.dense && tile * WG < M0) s0 = load_frag_window(tile, F.src0_in, F.pre_in, T_in, sh_pre);
+        const int first = tile * WG + w * 64;   /* the wave's first index */
+        int64_t src = li;
+        if (!F.dense && first < M0) src = frag_slot(li, first, tile, F.src0_in, F.pre_in, T_in);
         float x = 0.0f;
         int j = 0, born = -1;
         uint32_t tid = 0;
@@ -209,7 +212,6 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
         if (valid) {
             if (li < M0) {
-                const int64_t src = F.dense ? (int64_t)li : frag_slot(li, s0, sh_pre, F.pre_in, T_in);
                 x = F.freq_in[src];
                 id = F.ids_in[src];
                 tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);

@@ -114,14 +114,27 @@ struct FunctorSel {
     __device__ __forceinline__ float operator()(int p, int g, float x, const Row &) const { return f(p, g, x); }
 };
 
-/* Eq. 13: (x + s x (x + c1 (1-x))) / (1 + s x (x + c2 (1-x))), s >= -1 */
-GF_HD float selected_freq(float x, float s, float c1, float c2) {
+/* Eq. 13: (x + s x (x + c1 (1-x))) / (1 + s x (x + c2 (1-x))), s >= -1;
+ * mid: the quotient's operands are known to lie in div_mid's range */
+GF_HD float selected_freq(float x, float s, float c1, float c2, bool mid) {
     GF_STRICT_FP
     const float om = 1.0f - x;
     const float sx = s * x;
     const float num = __builtin_fmaf(sx, __builtin_fmaf(c1, om, x), x);
     const float den = __builtin_fmaf(sx, __builtin_fmaf(c2, om, x), 1.0f);
-    return num / den;
+    return mid ? div_mid(num, den) : num / den;
+}
+
+/* Whether a linear selection s(x) = sa x + sb with inbreeding F and
+ * dominance h keeps Eq. 13's operands in div_mid's range for x in [0, 1]:
+ * |s| <= 1/2 and F, h in [0, 1] give 0 <= x + c1 (1-x) <= 1 and x (x + c2
+ * (1-x)) <= 1, so 1/2 <= den <= 3/2 and x/2 <= num <= 3x/2 (to rounding).
+ * The caller sees to x = 0 or x >= 2^-79.  Used by the count form (gf_const_drift.hpp);
+ * in k_advance_fused the choice between the two quotients cost more scalar
+ * instructions than it saved (three populations 4 % slower). */
+GF_HD bool mid_selection(float sa, float sb, float F, float h) {
+    const float s = (sa < 0.0f ? -sa : sa) + (sb < 0.0f ? -sb : sb);
+    return s <= 0.5f && F >= 0.0f && F <= 1.0f && h >= 0.0f && h <= 1.0f;
 }
 
 /* ---------------- migration, selection and drift of one generation ----------------
@@ -161,13 +174,12 @@ __device__ __forceinline__ void generation_update(float *x, const Row &R, int g,
         } else {
             float s = sel(p, g, im, R);
             s = s > -1.0f ? s : -1.0f;
-            xs = selected_freq(im, s, R.c1[p], R.c2[p]);
+            xs = selected_freq(im, s, R.c1[p], R.c2[p], false);
         }
         const float N = R.fN[p];
         const float mean = xs * N;
         const float var = (1.0f - xs) * mean;
-        int j = binom_draw(lane_of(rc[p], g & 3), mean, var, N, ncdf, etab);
-        j = min(max(j, 0), Nc);
+        const int j = binom_count(lane_of(rc[p], g & 3), mean, var, N, Nc, ncdf, etab);
         /* (float)j / N, correctly rounded: up to N = 2^22 in three float
          * operations with r = RN(1/N), the row's newfreq (quot_count),
          * above through double (invN); the test is on the integer Nc, a
@@ -251,47 +263,51 @@ struct FusedLaunch {
     int preserve;
 };
 
-/* Slot of compacted index li (< M_in) in a fragmented input, for every lane
- * of one tile.  sh_pre is a 257-entry LDS window pre[s0 .. s0 + 256] filled
- * by the caller (INT_MAX past the end); s0 = the input tile holding the
- * tile's first compacted index, so sh_pre[0] <= li for every lane. */
-__device__ __forceinline__ int64_t frag_slot(int li, int s0, const int *sh_pre, const int *__restrict__ pre, int T_in) {
-    int lo = 0, hi = WG;                 /* last k with sh_pre[k] <= li */
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (sh_pre[mid] <= li) lo = mid; else hi = mid - 1;
-    }
-    int s = s0 + lo;
-    if (lo == WG) {                      /* more than 256 input tiles before li: search the rest */
-        int l2 = s, h2 = T_in - 1;
-        while (l2 < h2) {
-            const int mid = (l2 + h2 + 1) >> 1;
-            if (pre[mid] <= li) l2 = mid; else h2 = mid - 1;
+/* Slot of compacted index li in a fragmented input: tile s = the last one
+ * whose first survivor's index pre[s] is at most li, at offset li - pre[s].
+ * Called by a whole wave, whose lanes hold first .. first + 63 (all at least
+ * 256 `tile`, whose input tile is src0[tile]; lanes past the input's last
+ * index get a slot that is not read).  A wave's 64 indices span a few input
+ * tiles (2 to 7), so their boundaries are read through scalar loads, eight at
+ * a time, and each lane counts the ones it has passed: three vector
+ * instructions a boundary, no LDS and no barrier, where the binary search of
+ * a 257-entry LDS window it replaced took about fifty and a barrier.  The
+ * PRE_PAD entries from pre[T_in] on hold the total. */
+constexpr int PRE_PAD = 8;
+
+/* entries a prefix over `tiles` tiles takes, a multiple of 4 for 16-byte stores */
+__host__ __device__ constexpr int64_t pre_entries(int64_t tiles) { return (tiles + PRE_PAD + 3) & ~(int64_t)3; }
+
+__device__ __forceinline__ int64_t frag_slot(int li, int first, int tile, const int *__restrict__ src0,
+                                             const int *__restrict__ pre, int T_in) {
+    const auto *cpre = as_const(pre);
+    const int s0 = as_const(src0)[tile];
+    int s = s0, at = cpre[s0];
+    for (int k = s0 + 1; k < T_in; k += PRE_PAD) {
+        int v[PRE_PAD];
+#pragma unroll
+        for (int i = 0; i < PRE_PAD; i++) v[i] = cpre[k + i];
+#pragma unroll
+        for (int i = 0; i < PRE_PAD; i++) {
+            const bool passed = v[i] <= li;
+            s += passed ? 1 : 0;
+            at = passed ? v[i] : at;
         }
-        s = l2;
-        return (int64_t)s * WG + (li - pre[s]);
+        if (v[PRE_PAD - 1] > first + 63) break;
     }
-    return (int64_t)s * WG + (li - sh_pre[lo]);
+    return (int64_t)s * WG + (li - at);
 }
 
-/* loads the LDS window of frag_slot for tile `tile` (all threads; ends with
- * a barrier) */
-__device__ __forceinline__ int load_frag_window(int tile, const int *__restrict__ src0, const int *__restrict__ pre,
-                                                int T_in, int *sh_pre) {
-    const int s0 = src0[tile];
-    for (int k = threadIdx.x; k <= WG; k += WG) sh_pre[k] = (s0 + k <= T_in) ? pre[s0 + k] : 0x7fffffff;
-    __syncthreads();
-    return s0;
-}
+/* the wave's index in its workgroup, as a scalar */
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 
 template <int P, typename Sel>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_advance_fused(const FusedLaunch F, const SegLaunch<P> S,
                                                                                           const Sel sel) {
     const int lane = threadIdx.x & 63;
-    const int w = threadIdx.x >> 6;
+    const int w = wave_index();
     __shared__ int sh_tile;
     __shared__ unsigned int sh_wcount[WG / 64];
-    __shared__ int sh_pre[WG + 1];
     __shared__ unsigned long long sh_live[64];
     __shared__ int sh_diff[KMAX + 1];
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
@@ -319,13 +335,14 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         } else {
             if (threadIdx.x == 0) sh_tile = (int)atomicAdd(F.ticket, 1u);
             __syncthreads();
-            tile = sh_tile;
+            tile = __builtin_amdgcn_readfirstlane(sh_tile);
         }
         if (tile >= last_tile) break;
         const int li = tile * WG + (int)threadIdx.x;
         const bool valid = li < Mend;
-        int s0 = 0;
-        if (!F.dense && tile * WG < M0) s0 = load_frag_window(tile, F.src0_in, F.pre_in, T_in, sh_pre);
+        const int first = tile * WG + w * 64;   /* the wave's first index */
+        int64_t src = li;
+        if (!F.dense && first < M0) src = frag_slot(li, first, tile, F.src0_in, F.pre_in, T_in);
         float x[P];
         int ogen = 0, opop = 0, born = -1;
         uint32_t tid = 0;
@@ -336,7 +353,6 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
         if (valid) {
             if (li < M0) {
-                const int64_t src = F.dense ? (int64_t)li : frag_slot(li, s0, sh_pre, F.pre_in, T_in);
 #pragma unroll
                 for (int p = 0; p < P; p++) x[p] = F.freq_in[p * F.pitch + src];
                 id = F.ids_in[src];

@@ -13,7 +13,8 @@ namespace gf {
 
 /* ---------------- prefix of the fused launch's tile counts ----------------
  * T = tiles of the launch (from the device slot count M_in + new);
- * pre[s] = survivors of tiles before s, pre[T] = total = *M_out; for every
+ * pre[s] = survivors of tiles before s, pre[T .. T + PRE_PAD) = total =
+ * *M_out; for every
  * tile j of the next launch (256 j < total) src0[j] = the tile holding
  * compacted index 256 j.
  * One workgroup walks the counts in chunks of SCAN_CHUNK.  For large
@@ -117,7 +118,8 @@ static __global__ __launch_bounds__(1024) void k_tile_scan(const unsigned int *_
             /* the last round: the totals are known, and their stores (one
              * of them to host memory) overlap the prefix stores below */
             const int total = carry + sh_w[15];
-            pre[T] = total;
+#pragma unroll
+            for (int k = 0; k < PRE_PAD; k++) pre[T + k] = total;
             *M_out = total;
             *T_out = T;
             if (M_host) *M_host = total;   /* pinned host word: the host reads it after the launch's event */
@@ -148,7 +150,7 @@ static __global__ __launch_bounds__(1024) void k_tile_scan(const unsigned int *_
         __syncthreads();
     }
     if (T == 0 && threadIdx.x == 0 && blockIdx.x == 0) {
-        pre[0] = 0;
+        for (int k = 0; k < PRE_PAD; k++) pre[k] = 0;
         *M_out = 0;
         *T_out = 0;
         if (M_host) *M_host = 0;
@@ -174,14 +176,13 @@ __global__ __launch_bounds__(WG) void k_densify(const float *__restrict__ freq_i
                                                 float *__restrict__ freq_out, gf_mutid *__restrict__ ids_out, int64_t pitch,
                                                 const int *__restrict__ pre, const int *__restrict__ src0,
                                                 const int *__restrict__ T_in, const int *__restrict__ M_in) {
-    __shared__ int sh_pre[WG + 1];
     const int M = *M_in, T = *T_in;
+    const int w = wave_index();
     for (int tile = blockIdx.x; tile * WG < M; tile += gridDim.x) {
-        __syncthreads();
-        const int s0 = load_frag_window(tile, src0, pre, T, sh_pre);
-        const int li = tile * WG + (int)threadIdx.x;
+        const int li = tile * WG + (int)threadIdx.x, first = tile * WG + w * 64;
+        if (first >= M) continue;
+        const int64_t src = frag_slot(li, first, tile, src0, pre, T);
         if (li < M) {
-            const int64_t src = frag_slot(li, s0, sh_pre, pre, T);
 #pragma unroll
             for (int p = 0; p < P; p++) freq_out[p * pitch + li] = freq_in[p * pitch + src];
             ids_out[li] = ids_in[src];

@@ -64,9 +64,8 @@ GF_HD uint32_t lane_of(const u32x4 &r, int i) {
 /* u * 2^-32 + 2^-33 in (0, 1] (reference shared.cuh:59-64) */
 GF_HD float u01(uint32_t u) {
     GF_STRICT_FP
-    float f = (float)u;
-    f = f * 2.3283064365386963e-10f;
-    return f + 1.1641532182693481e-10f;
+    /* the product by 2^-32 is exact: fused or not, the same value */
+    return __builtin_fmaf((float)u, 2.3283064365386963e-10f, 1.1641532182693481e-10f);
 }
 
 /* ----- elementary functions ----- */
@@ -141,21 +140,35 @@ GF_HD float pow_f(float a, float b) {
 }
 
 /* Correctly rounded square root of a positive normal float x >= 2^-96 (the
- * variance of the normal approximation, at least 36/N there, and w >= 8 in
- * the inverse normal's tail).  On the
- * device: the hardware estimate (within one ulp) moved by one ulp where the
- * fused residual x - y*y says so, which is the compiler's own correctly
- * rounded expansion without its scaling of tiny inputs and its zero,
- * infinity and NaN cases; the host's sqrtf is correctly rounded. */
+ * variance of the normal approximation).  On the device: the hardware's
+ * reciprocal root g, s = x g, one Newton step s + (x - s s) g / 2 with the
+ * residual in a fused multiply-add: five operations where the compiler's
+ * expansion without its tiny-input scaling takes nine.  Equal to the IEEE
+ * root for every float from 2^-96 up (all of them compared on the device);
+ * the host's sqrtf is correctly rounded. */
 GF_HD float sqrt_pos(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const float y = __builtin_amdgcn_sqrtf(x);
-    const float ydn = bits2f(f2bits(y) - 1u), yup = bits2f(f2bits(y) + 1u);
-    float r = __builtin_fmaf(-ydn, y, x) <= 0.0f ? ydn : y;
-    r = __builtin_fmaf(-yup, y, x) > 0.0f ? yup : r;
-    return r;
+    const float g = __builtin_amdgcn_rsqf(x);
+    const float s = x * g;
+    return __builtin_fmaf(__builtin_fmaf(-s, s, x), 0.5f * g, s);
 #else
     return __builtin_sqrtf(x);
+#endif
+}
+
+/* num / den, correctly rounded, for num = 0 or 2^-80 <= |num| <= 2^20 and
+ * 2^-20 <= |den| <= 2^20: the compiler's expansion (reciprocal, one Newton
+ * step, two residual steps) without the scaling and the special cases, which
+ * do nothing in that range: 8 operations instead of 11. */
+GF_HD float div_mid(float num, float den) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    float r = __builtin_amdgcn_rcpf(den);
+    r = __builtin_fmaf(__builtin_fmaf(-den, r, 1.0f), r, r);
+    float q = num * r;
+    q = __builtin_fmaf(__builtin_fmaf(-den, q, num), r, q);
+    return __builtin_fmaf(__builtin_fmaf(-den, q, num), r, q);
+#else
+    return num / den;
 #endif
 }
 
@@ -403,21 +416,50 @@ GF_HD int round_away_nonneg(float v) {
     return f2i_sat(v) + (d >= 0.5f ? 1 : 0);
 }
 
-/* the rounded normal approximation of the binomial draw, for the caller's
- * clamp to [0, N].  u01 gives 2^-33 <= u <= 1 (never NaN): of
- * normcdfinv_tab's clamps only the top one can act. */
-GF_HD float u01_top(float u) { return u > 0.99999994039535522f ? 0.99999994039535522f : u; }
-
-GF_HD int binom_normal(float u, float mean, float var, const NcdfSeg *ncdf) {
+/* the normal approximation of the binomial draw before its rounding.  u01
+ * gives 2^-33 <= u <= 1 (never NaN): of normcdfinv_tab's clamps only the top
+ * one can act. */
+GF_HD float binom_normal(float u, float mean, float var, const NcdfSeg *ncdf) {
     GF_STRICT_FP
-    return round_away_nonneg(normcdfinv_core(ncdf, u01_top(u)) * sqrt_pos(var) + mean);
+#if defined(__HIP_DEVICE_COMPILE__)
+    u = __builtin_amdgcn_fmed3f(u, 0.0f, 0.99999994039535522f);
+#else
+    u = u > 0.99999994039535522f ? 0.99999994039535522f : u;
+#endif
+    return normcdfinv_core(ncdf, u) * sqrt_pos(var) + mean;
+}
+
+/* v rounded half away from zero and clamped to [0, top], NaN to 0, for an
+ * integer top in [0, 2^31 - 128]: the clamp first, then floor(v + 1/2), which
+ * v_cvt_rpi_i32_f32 computes without rounding v + 1/2 (equal to round half
+ * away for every float >= 0, all of them compared on the device): two
+ * operations instead of six. */
+GF_HD int round_count(float v, float top) {
+    GF_STRICT_FP
+#if defined(__HIP_DEVICE_COMPILE__)
+    int r;
+    asm("v_cvt_rpi_i32_f32 %0, %1" : "=v"(r) : "v"(__builtin_amdgcn_fmed3f(v, 0.0f, top)));
+    return r;
+#else
+    v = v > 0.0f ? v : 0.0f;
+    return f2i_sat(round_away(v < top ? v : top));
+#endif
+}
+
+/* the Poisson (or binomial, N < 100) tails of the binomial draw: lo, the
+ * mean at most 6, else at least N - 6.  A mean of exactly 0 or N (lost or
+ * fixed) is answered without entering the inversion. */
+GF_HD int binom_tail(float u, float mean, bool lo, float N, const ExpSeg *etab) {
+    GF_STRICT_FP
+    const float m = lo ? mean : N - mean;
+    int k = 0;
+    if (m != 0.0f) k = (N < 100.0f) ? binomcdfinv(u, m, m / N, N) : poiscdfinv_tail(u, m, etab);
+    return lo ? k : f2i_sat(N - (float)k);
 }
 
 /* approximate binomial draw (reference shared.cu:10-18): the two Poisson
  * (or binomial, N < 100) tails share one CDF inversion; the rest is the
- * rounded normal approximation.  A mean of exactly 0 or N (lost or fixed:
- * the Poisson inversion of mean 0 returns 0) is answered without entering
- * the inversion.  The result equals the reference's draw wherever that is
+ * rounded normal approximation.  The result equals the reference's draw wherever that is
  * >= 0; where the normal approximation goes below 0 it is some value <= 0
  * (round_away_nonneg), and the caller clamps the result to [0, N]. */
 GF_HD int binom_draw(uint32_t bits, float mean, float var, float N, const NcdfSeg *ncdf = ncdf_table(),
@@ -425,14 +467,18 @@ GF_HD int binom_draw(uint32_t bits, float mean, float var, float N, const NcdfSe
     GF_STRICT_FP
     const float u = u01(bits);
     const bool lo = mean <= 6.0f;
-    const bool hi = !lo && (mean >= N - 6.0f);
-    if (lo || hi) {
-        const float m = lo ? mean : N - mean;
-        int k = 0;
-        if (m != 0.0f) k = (N < 100.0f) ? binomcdfinv(u, m, m / N, N) : poiscdfinv_tail(u, m, etab);
-        return lo ? k : f2i_sat(N - (float)k);
-    }
-    return binom_normal(u, mean, var, ncdf);
+    if (lo || mean >= N - 6.0f) return binom_tail(u, mean, lo, N, etab);
+    return round_away_nonneg(binom_normal(u, mean, var, ncdf));
+}
+
+/* the same draw clamped to [0, Nc] (the drift's), N = (float)Nc */
+GF_HD int binom_count(uint32_t bits, float mean, float var, float N, int Nc, const NcdfSeg *ncdf, const ExpSeg *etab) {
+    GF_STRICT_FP
+    const float u = u01(bits);
+    const bool lo = mean <= 6.0f;
+    const int k = lo || mean >= N - 6.0f ? binom_tail(u, mean, lo, N, etab)
+                                         : round_count(binom_normal(u, mean, var, ncdf), 2147483520.0f);
+    return k < 0 ? 0 : (k < Nc ? k : Nc);
 }
 
 /* approximate Poisson draw (reference shared.cuh:251-256) */

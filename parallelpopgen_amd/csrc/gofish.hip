@@ -508,9 +508,8 @@ struct PlainRun {
         return GF_OK;
     }
 
-    /* entries of each half of d_pre: T + 1 prefix values, rounded up to a
-     * multiple of 4 so that both halves take 16-byte stores */
-    static size_t pre_stride(int64_t tiles) { return ((size_t)tiles + 1 + 3) & ~(size_t)3; }
+    /* entries of each half of d_pre */
+    static size_t pre_stride(int64_t tiles) { return (size_t)pre_entries(tiles); }
 
     /* grow the buffers to hold `need` slots; the current contents (exact
      * count read from the device) move along */
@@ -542,15 +541,17 @@ struct PlainRun {
 
     int advance_const(const FusedLaunch &F, const SegLaunch<P> &sl, int t_first, int grid) {
         if constexpr (P == 1) {
+            const gf_pop_gen &pg = d->params[t_first];
+            const int mid = mid_selection(pg.sel_slope, pg.sel_intercept, pg.F, pg.h);
             if (pois_row < 0 || !same_model(rows[pois_row], rows[t_first])) {
                 GF_TRY(d_pois.alloc(1));
-                hipLaunchKernelGGL(k_pois_table, dim3(1), dim3(64), 0, st, d_rows.p + t_first, d_pois.p);
+                hipLaunchKernelGGL(k_pois_table, dim3(1), dim3(64), 0, st, d_rows.p + t_first, mid, d_pois.p);
                 GF_HIP(hipGetLastError());
                 pois_row = t_first;
             }
             const int Nc_prev = t_first > 1 ? rows[t_first - 1].Nc[0] : nchrom(d->params[0].N, d->params[0].F);
             hipLaunchKernelGGL(k_advance_const, dim3(grid), dim3(WG), 0, st, F, sl, d_pois.p,
-                               Nc_prev == rows[t_first].Nc[0] ? 0 : 1);
+                               mid, Nc_prev == rows[t_first].Nc[0] ? 0 : 1);
         }
         return GF_OK;
     }

@@ -24,7 +24,7 @@ int main() {
                 for (float slope : {0.0f, 0.001f}) {
                     const float F = 0.1f;
                     const ConstModel C{Nc, (float)Nc, 1.0f / (float)Nc, slope, s, (F + h) - (h * F), (F + (2.0f * h)) - ((2.0f * h) * F),
-                                       s == 0.0f && slope == 0.0f};
+                                       s == 0.0f && slope == 0.0f, mid_selection(slope, s, F, h)};
                     uint4 tab[POIS_ROWS * POIS_ROW_VECS];
                     for (int row = 0; row < POIS_ROWS; row++) {
                         const float xs = const_selected((float)(row + 1) / (float)Nc, C);

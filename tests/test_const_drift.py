@@ -75,3 +75,17 @@ def test_mixed_batch(gpu):
         p = gpu.run(S.sweep_plain_desc(b))["samples"][-1]
         f, _ = r["states"][i]
         assert np.array_equal(f.view(np.uint32), p["freq"][0].view(np.uint32)), i
+
+
+# launches whose tiles keep a handful of slots each: a wave gathers over many
+# input tiles, empty ones among them (one population and two)
+@pytest.mark.gpu
+@pytest.mark.parametrize("P,s,kpl", [(1, -0.9, 64), (1, -0.4, 33), (2, -0.9, 48)])
+def test_gather_over_sparse_tiles(gpu, oracle, P, s, kpl):
+    d = S.constant(N=500, L=2e9 / P, G=140, s=s, h=0.9, P=P, m=0.01, compact_interval=kpl)
+    gpu.set_generations_per_launch(kpl)
+    try:
+        a = gpu.run(d)
+    finally:
+        gpu.set_generations_per_launch(0)
+    assert_same(a, oracle.run(d), (P, s, kpl))
