@@ -124,12 +124,11 @@ __device__ __forceinline__ BSim load_bsim(const BSim *p) {
     return b;
 }
 
-/* ---- draw tables, one wave per simulation (once per batch) ---- */
-static __global__ __launch_bounds__(WG) void k_bt_pois(const BSim *__restrict__ sims, int S, PoisTable *__restrict__ out) {
-    const int s = (int)blockIdx.x * (WG / 64) + ((int)threadIdx.x >> 6);
-    if (s >= S || !sims[s].counted) return;   /* the whole wave */
-    const BSim &b = sims[s];
-    pois_table_build(ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral, b.mid}, out + s);
+/* ---- draw tables, one workgroup per simulation (once per batch) ---- */
+static __global__ __launch_bounds__(POIS_BUILD) void k_bt_pois(const BSim *__restrict__ sims, PoisTable *__restrict__ out) {
+    const BSim &b = sims[blockIdx.x];
+    if (!b.counted) return;
+    pois_table_entry(threadIdx.x, ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral, b.mid}, out + blockIdx.x);
 }
 
 /* ---- 1. rows and new-mutation counts of the next block, one thread per simulation ---- */
@@ -651,7 +650,7 @@ struct BatchRun {
                 GF_TRY(d_tot.alloc((size_t)choff));
                 hipLaunchKernelGGL(k_mse_area, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + ns, ns, aoff, d_area.p);
                 hipLaunchKernelGGL(k_mse_chunk_local, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + 2 * ns, ns, choff, d_area.p, d_tot.p);
-                hipLaunchKernelGGL(k_mse_chunk_prefix, dim3((ns + 63) / 64), dim3(64), 0, st, d_segs.p, ns, d_tot.p);
+                hipLaunchKernelGGL(k_mse_chunk_prefix, dim3((ns + 3) / 4), dim3(256), 0, st, d_segs.p, ns, d_tot.p);
                 hipLaunchKernelGGL(k_mse_chunk_add, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + ns, ns, aoff, d_area.p, d_tot.p);
                 GF_HIP(hipGetLastError());
             }
@@ -717,7 +716,7 @@ struct BatchRun {
         GF_HIP(hipMemcpyAsync(d_sims.p, host.data(), (size_t)S * sizeof(BSim), hipMemcpyHostToDevice, st));
         GF_TRY(pois.alloc(S));
         if (any_counted)
-            hipLaunchKernelGGL(k_bt_pois, dim3((S + 3) / 4), dim3(WG), 0, st, (const BSim *)d_sims.p, S, pois.p);
+            hipLaunchKernelGGL(k_bt_pois, dim3(S), dim3(POIS_BUILD), 0, st, (const BSim *)d_sims.p, pois.p);
         GF_HIP(hipGetLastError());
         GF_HIP(hipStreamSynchronize(st));
         return GF_OK;

@@ -18,7 +18,8 @@
  * generations a launch: 6.9e7 vector instructions by k_advance_fused, 5.2e7
  * with the table, 4.5e7 with the arithmetic of gf_math.hpp (div_mid,
  * sqrt_pos, round_count) and the scalar gather (frag_slot) besides.  The
- * 5,000-generation run: 64.1 -> 51.2 -> 46.3 ms; a run of 8.4e3 mutations
+ * 5,000-generation run: 64.1 -> 51.2 -> 46.3 ms (44.4 with 16 generations a
+ * launch); a run of 8.4e3 mutations
  * 2.14 -> 1.81 -> 1.74 ms; a batch of 64 uneven simulations 428 -> 261 ms.
  */
 #ifndef GF_CONST_DRIFT_HPP_
@@ -63,43 +64,48 @@ GF_HD float const_selected(float x, const ConstModel &C) {
     return selected_freq(x, s, C.c1, C.c2, C.mid != 0);
 }
 
-/* row `row` of the table; true if its mean is in [0, 6] */
-GF_HD bool pois_table_row(int row, const ConstModel &C, uint4 *v) {
+/* mean of the next draw of count j */
+GF_HD float const_mean(int j, const ConstModel &C) {
     GF_STRICT_FP
-    uint32_t T[POIS_TERMS];
-    for (int k = 0; k < POIS_TERMS; k++) T[k] = 0xffffffffu;
-    const float mean = const_selected(quot_count((float)(row + 1), C.N, C.r), C) * C.N;
-    const bool ok = mean >= 0.0f && mean <= 6.0f;
-    if (ok) {
-        const int km = mean <= 1.0f ? 1 : (int)__builtin_ceilf(mean);
-        const int jstop = 8 + 3 * km - (km > 4 ? km - 4 : 0);   /* exit_index of a mean up to 14 */
-        float e = expneg_tab(expneg_table(), mean), cdf = e;
-        for (int k = 0; k < jstop; k++) {
-            if (k > 0) {
-                e = e * (mean * kRecip[k - 1]);
-                cdf = cdf + e;
-            }
-            uint32_t lo = 0, hi = 0xffffffffu;   /* u01(0) = 2^-33 < exp(-6) <= cdf */
-            while (lo < hi) {
-                const uint32_t mid = lo + (hi - lo) / 2 + 1;
-                if (u01(mid) <= cdf) lo = mid; else hi = mid - 1;
-            }
-            T[k] = lo;
-        }
-    }
-    v += row * POIS_ROW_VECS;
-    v[0] = make_uint4(T[4], T[9], T[14], T[19]);
-    for (int c = 0; c < 5; c++)
-        v[1 + c] = make_uint4(T[5 * c], T[5 * c + 1], T[5 * c + 2], T[5 * c + 3]);
-    return ok;
+    return const_selected(quot_count((float)j, C.N, C.r), C) * C.N;
 }
 
-/* the table of one model by a wave's first POIS_ROWS lanes (all lanes call) */
-__device__ __forceinline__ void pois_table_build(const ConstModel &C, PoisTable *t) {
-    const int lane = threadIdx.x & 63;
-    const bool ok = lane < POIS_ROWS && pois_table_row(lane, C, t->v);
-    const uint64_t bad = ~__ballot(ok);          /* bit POIS_ROWS is always set */
-    if (lane == 0) t->jn = const_drift_range(C.Nc) ? 1 + __builtin_ctzll(bad) : 1;
+/* T[k] of the row with mean `mean` in [0, 6] */
+GF_HD uint32_t pois_threshold(float mean, int k) {
+    GF_STRICT_FP
+    const int km = mean <= 1.0f ? 1 : (int)__builtin_ceilf(mean);
+    if (k >= 8 + 3 * km - (km > 4 ? km - 4 : 0)) return 0xffffffffu;   /* exit_index of a mean up to 14 */
+    float e = expneg_tab(expneg_table(), mean), cdf = e;
+    for (int i = 1; i <= k; i++) {
+        e = e * (mean * kRecip[i - 1]);
+        cdf = cdf + e;
+    }
+    uint32_t lo = 0, hi = 0xffffffffu;   /* u01(0) = 2^-33 < exp(-6) <= cdf */
+    while (lo < hi) {
+        const uint32_t mid = lo + (hi - lo) / 2 + 1;
+        if (u01(mid) <= cdf) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+/* word of T[k] in its row's vectors */
+GF_HD constexpr int pois_word(int k) { return k % 5 == 4 ? k / 5 : 4 * (1 + k / 5) + k % 5; }
+
+/* Entry `id` of the table of one model, id in [0, POIS_BUILD): row id / 32,
+ * threshold id % 32, one thread each (a single lane per row took 37 us, as
+ * long as the first launch it was built for; 4 us). */
+constexpr int POIS_BUILD = POIS_ROWS * 32;
+
+GF_HD void pois_table_entry(int id, const ConstModel &C, PoisTable *t) {
+    const int row = id >> 5, k = id & 31;
+    const float mean = const_mean(row + 1, C);
+    if (k < POIS_TERMS && mean >= 0.0f && mean <= 6.0f)
+        reinterpret_cast<uint32_t *>(t->v + row * POIS_ROW_VECS)[pois_word(k)] = pois_threshold(mean, k);
+    if (id == 0) {
+        int jn = 1;
+        while (jn <= POIS_ROWS && const_mean(jn, C) >= 0.0f && const_mean(jn, C) <= 6.0f) jn++;
+        t->jn = const_drift_range(C.Nc) ? jn : 1;
+    }
 }
 
 /* number of thresholds of row `row` below `bits` */
@@ -163,11 +169,11 @@ __device__ __forceinline__ int const_count(float x, bool first_freq, const Const
     return x <= 0.0f ? 0 : (x >= 1.0f ? C.Nc : 1);
 }
 
-/* the table of rows[0]'s model, one wave */
-static __global__ __launch_bounds__(64) void k_pois_table(const GenRow<1> *__restrict__ row, int mid,
+/* the table of rows[0]'s model */
+static __global__ __launch_bounds__(POIS_BUILD) void k_pois_table(const GenRow<1> *__restrict__ row, int mid,
                                                            PoisTable *__restrict__ out) {
     const auto &R = *as_const(row);
-    pois_table_build(ConstModel{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1, mid}, out);
+    pois_table_entry(threadIdx.x, ConstModel{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1, mid}, out);
 }
 
 /* k_advance_fused for one population and a launch whose model rows are all

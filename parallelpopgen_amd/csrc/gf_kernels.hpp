@@ -338,18 +338,31 @@ static __global__ void k_mse_chunk_local(const MseSeg *__restrict__ segs, const 
     }
 }
 
-/* sequential exclusive prefix of chunk totals, one thread per segment */
-static __global__ void k_mse_chunk_prefix(const MseSeg *__restrict__ segs, int nseg, float *__restrict__ tot) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= nseg) return;
+/* sequential exclusive prefix of chunk totals (float additions in chunk
+ * order), one wave per segment: 64 totals at a time in the lanes, the next 64
+ * loaded meanwhile, the running sum passed along by lane reads.  A serial
+ * chain of one addition per 64 classes; one thread per segment waited for a
+ * load at each: 297 us at 2e5 classes, 41 us here. */
+static __global__ __launch_bounds__(256) void k_mse_chunk_prefix(const MseSeg *__restrict__ segs, int nseg, float *__restrict__ tot) {
+    GF_STRICT_FP
+    const int s = blockIdx.x * (blockDim.x / 64) + (threadIdx.x >> 6);
+    if (s >= nseg) return;   /* the whole wave */
     const MseSeg &S = segs[s];
     if (S.neutral) return;
+    const int lane = threadIdx.x & 63;
     const int nc = (S.Nc + MSE_CHUNK - 1) / MSE_CHUNK;
-    float pre = 0.0f;
-    for (int c = 0; c < nc; c++) {
-        const float t = tot[S.chunk_off + c];
-        tot[S.chunk_off + c] = pre;
-        pre = pre + t;
+    float *t = tot + S.chunk_off;
+    float pre = 0.0f, next = lane < nc ? t[lane] : 0.0f;
+    for (int c = 0; c < nc; c += 64) {
+        const float mine = next;
+        next = c + 64 + lane < nc ? t[c + 64 + lane] : 0.0f;
+        float before = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 64; i++) {
+            before = lane == i ? pre : before;
+            pre = pre + bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(mine), i));
+        }
+        if (c + lane < nc) t[c + lane] = before;
     }
 }
 

@@ -81,7 +81,9 @@ int scan_counts(const int *d_in, int64_t n, int64_t *d_out, int64_t *d_total, hi
         GF_HIP(hipMemsetAsync(d_total, 0, sizeof(int64_t), stream));
         return GF_OK;
     }
-    int64_t nb = std::min<int64_t>(1024, std::max<int64_t>(1, (n + 4095) / 4096));
+    /* 1,024 counts per block up to 1,024 blocks: four rounds of k_scan_final
+     * (16 at 4,096 counts: 18 us of the 2e4 classes of a small run's start) */
+    int64_t nb = std::min<int64_t>(1024, std::max<int64_t>(1, (n + 1023) / 1024));
     int64_t per = (n + nb - 1) / nb;
     nb = (n + per - 1) / per;
     GF_TRY(scratch.alloc((size_t)nb));
@@ -205,6 +207,7 @@ struct PlainRun {
     std::vector<hipEvent_t> ev_ring;
     int64_t launches = 0;
     int64_t M_bound = 0;                /* upper bound of the current slot count */
+    int64_t M_seen = 0;                 /* the last slot count the host has read (one launch old) */
     int64_t last_new = 0;               /* new slots of the most recent launch */
     DevBuf<PoisTable> d_pois;           /* draw table of row pois_row's model (k_advance_const) */
     int pois_row = -1;
@@ -370,7 +373,7 @@ struct PlainRun {
             GF_TRY(d_tot.alloc((size_t)choff));
             hipLaunchKernelGGL(k_mse_area, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + ns, ns, aoff, d_area.p);
             hipLaunchKernelGGL(k_mse_chunk_local, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + 2 * ns, ns, choff, d_area.p, d_tot.p);
-            hipLaunchKernelGGL(k_mse_chunk_prefix, dim3((ns + 63) / 64), dim3(64), 0, st, d_segs.p, ns, d_tot.p);
+            hipLaunchKernelGGL(k_mse_chunk_prefix, dim3((ns + 3) / 4), dim3(256), 0, st, d_segs.p, ns, d_tot.p);
             hipLaunchKernelGGL(k_mse_chunk_add, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p + ns, ns, aoff, d_area.p, d_tot.p);
             GF_HIP(hipGetLastError());
         }
@@ -545,7 +548,7 @@ struct PlainRun {
             const int mid = mid_selection(pg.sel_slope, pg.sel_intercept, pg.F, pg.h);
             if (pois_row < 0 || !same_model(rows[pois_row], rows[t_first])) {
                 GF_TRY(d_pois.alloc(1));
-                hipLaunchKernelGGL(k_pois_table, dim3(1), dim3(64), 0, st, d_rows.p + t_first, mid, d_pois.p);
+                hipLaunchKernelGGL(k_pois_table, dim3(1), dim3(POIS_BUILD), 0, st, d_rows.p + t_first, mid, d_pois.p);
                 GF_HIP(hipGetLastError());
                 pois_row = t_first;
             }
@@ -635,7 +638,8 @@ struct PlainRun {
         if (launches > 0) {
             const int prev = (int)((launches - 1) % RING);
             GF_HIP(hipEventSynchronize(ev_ring[prev]));
-            M_bound = (int64_t)h_ring.p[prev] + new_in_block;
+            M_seen = h_ring.p[prev];
+            M_bound = M_seen + new_in_block;
         } else {
             M_bound = bound;
         }
@@ -697,16 +701,19 @@ struct PlainRun {
         for (auto &e : ev_ring) GF_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         GF_HIP(hipStreamSynchronize(st));
         mcur = 0;
-        M_bound = M;
+        M_bound = M_seen = M;
 
         int next_compact = start + interval;
         int t = 0;   /* generations done */
         /* generations per launch, unless the caller set it.  One population
          * compacts at every launch: a longer launch saves launch overhead
-         * but carries the slots lost inside it to its end.  Measured best
-         * (N = 1e4, 1,000 generations): 64 at 8.4e3 and 8.4e4 live
-         * mutations (-41 % and -38 % against 10), 16 at 8.4e5; 10 at 2.0e6
-         * (N = 1e5, theta = 2e5).  Several populations end launches at the
+         * (a scan and two gaps, 13 us) but carries the slots lost inside it
+         * to its end.  By the slots in use, measured best (ms per run of
+         * 1,000 generations, live mutations at the end): 8.4e4: 64 (32 2.11,
+         * 48 1.93, 64 1.84); 2.5e5: 48 (16 2.82, 32 2.46, 48 2.44); 8.4e5:
+         * 20 (10 5.35, 16 4.89, 20 4.84, 32 5.07); 2.0e6: 16 (2,000
+         * generations: 10 19.6, 14 18.9, 16 18.9, 24 19.8); 2.6e7: 12 to 20
+         * alike.  Several populations end launches at the
          * compaction interval anyway: up to 2e6 slots a launch runs to it
          * (two populations, N = 1e4, 1,000 generations, interval 35: 20
          * generations per launch 3.73 / 5.82 / 21.9 ms at 1.4e4 / 1.4e5 /
@@ -717,7 +724,7 @@ struct PlainRun {
         auto launch_length = [&]() {
             int k;
             if (k_user > 0) k = k_user;
-            else if (P == 1) k = M_bound <= 200000 ? 64 : (M_bound <= 1200000 ? 16 : 10);
+            else if (P == 1) k = M_seen <= 150000 ? 64 : (M_seen <= 400000 ? 48 : (M_seen <= 1200000 ? 20 : 16));
             else k = M_bound <= 2000000 ? 64 : 20;
             return std::max(1, std::min(KMAX, k));
         };
