@@ -446,15 +446,35 @@ inline void parallel_copy(char *dst, const char *src, size_t bytes) { CopyPool::
 /* Device -> host copy through a process-wide pinned staging buffer (kept
  * between calls, grown on demand): a copy into pageable memory runs at a
  * fraction of the link's bandwidth.  Two halves: the link fills one while
- * the host copies the other out.  Serialised by a mutex. */
-inline int readback(void *dst, const void *src, size_t bytes, hipStream_t st) {
+ * the host copies the other out.  Serialised by a mutex.  Contiguous device
+ * memory may go to several host buffers. */
+struct ReadPart { void *dst; size_t bytes; };   /* dst NULL: that part is skipped */
+
+inline int readback_parts(const ReadPart *parts, int nparts, const void *src, hipStream_t st) {
     static std::mutex mu;
     static PinBuf<char> stage;
+    size_t bytes = 0;
+    for (int k = 0; k < nparts; k++) bytes += parts[k].bytes;
     if (bytes == 0) return GF_OK;
     std::lock_guard<std::mutex> lock(mu);
     const size_t half = std::min(bytes, (size_t)16 << 20);
     if (stage.n < 2 * half) GF_TRY(stage.alloc(2 * half));
     const size_t h = stage.n / 2;
+    /* bytes [off, off + n) of the source, staged at `from`, to their parts */
+    auto spread = [&](size_t off, size_t n, const char *from) {
+        size_t at = 0;
+        for (int k = 0; k < nparts; k++) {
+            const size_t lo = std::max(off, at), hi = std::min(off + n, at + parts[k].bytes);
+            if (lo < hi && parts[k].dst) parallel_copy((char *)parts[k].dst + (lo - at), from + (lo - off), hi - lo);
+            at += parts[k].bytes;
+        }
+    };
+    if (bytes <= h) {   /* one piece: no events */
+        GF_HIP(hipMemcpyAsync(stage.p, src, bytes, hipMemcpyDeviceToHost, st));
+        GF_HIP(hipStreamSynchronize(st));
+        spread(0, bytes, stage.p);
+        return GF_OK;
+    }
     struct Events {   /* created on the stream's device, destroyed on return */
         hipEvent_t e[2] = {nullptr, nullptr};
         ~Events() { for (auto x : e) if (x) (void)hipEventDestroy(x); }
@@ -472,10 +492,14 @@ inline int readback(void *dst, const void *src, size_t bytes, hipStream_t st) {
     for (size_t c = 0; c < nchunks; c++) {
         if (c + 1 < nchunks) GF_TRY(issue(c + 1));   /* the other half was copied out in the previous round */
         GF_HIP(hipEventSynchronize(filled[c & 1]));
-        const size_t off = c * h;
-        parallel_copy((char *)dst + off, stage.p + (c & 1) * h, std::min(h, bytes - off));
+        spread(c * h, std::min(h, bytes - c * h), stage.p + (c & 1) * h);
     }
     return GF_OK;
+}
+
+inline int readback(void *dst, const void *src, size_t bytes, hipStream_t st) {
+    const ReadPart part{dst, bytes};
+    return readback_parts(&part, 1, src, st);
 }
 
 /* HIP-event based kernel timer (on the library's stream): with stride s,

@@ -9,9 +9,10 @@
  * forward, backward and Adam kernels.  Every matrix product runs on the
  * gfx950 matrix cores (v_mfma_f32_32x32x16_bf16): k_gemm's global->LDS
  * stage handles the three operand layouts of forward (X W^T), input
- * gradient (dZ W) and weight gradient (dZ^T X) at training batch sizes;
- * k_gemm_nt runs the forward products of large batches (prediction); the
- * ensemble members are the grid's z dimension.
+ * gradient (dZ W) and weight gradient (dZ^T X) at training batch sizes,
+ * k_gemm_nt the forward products of large training batches, the ensemble
+ * members being the grid's z dimension; k_mlp runs the whole network for
+ * prediction.
  */
 #include "gf_runtime.hpp"
 
@@ -25,6 +26,8 @@ namespace sg {
 
 typedef __bf16 bf16;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int IN_PAD = 64;    /* input features padded to one K tile */
@@ -33,6 +36,7 @@ constexpr int NHID = 4;
 constexpr int OUT = 100;      /* 99 bins + log-total */
 constexpr int OUT_PAD = 128;
 constexpr int NBINS = 99;
+constexpr int POUT = NBINS + 2;   /* floats of one prediction: bins, log-total, disagreement */
 constexpr int TILE = 64;
 constexpr int KSTEP = 32;
 constexpr int LDSK = KSTEP + 8; /* padded LDS row (bf16 elements) */
@@ -156,7 +160,7 @@ __global__ __launch_bounds__(256) void k_gemm(const GemmArgs g) {
 }
 
 /* ---- large forward products: C = A B^T with both operands K-contiguous ----
- * (the forward pass and prediction at batches of thousands of rows).  A
+ * (training at batches of thousands of rows).  A
  * 128 x 128 tile per workgroup of 4 waves, each wave a 64 x 64 quadrant of
  * 2 x 2 blocks of v_mfma_f32_32x32x16_bf16; K in stages of 64 through two
  * LDS buffers, fed from two register sets: stage s + 2's global loads are
@@ -280,11 +284,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     }
     __syncthreads();
     /* epilogue: accumulator r of lane l is C[8(r/4) + 4(l/32) + r%4][l%32]
-     * of its block.  The tile goes through LDS (free after the loop's last
-     * barrier) so that global stores are whole 16-byte row pieces: a lane's
-     * accumulators run down a column.  Row strides of 144 bf16 / 136 fp32
-     * put the two half-waves (rows 4 apart) on different LDS banks. */
-    if (g.epi == EPI_HIDDEN && g.Cf) {   /* pre-activations kept as well: direct stores */
+     * of its block.  An output tile goes through LDS (free after the loop's
+     * last barrier) so that global stores are whole 16-byte row pieces: a
+     * lane's accumulators run down a column.  A row stride of 136 floats puts
+     * the two half-waves (rows 4 apart) on different LDS banks. */
+    if (g.epi == EPI_HIDDEN) {   /* pre-activations and activations: direct stores */
 #pragma unroll
         for (int j = 0; j < 2; j++) {
             const int n = n0 + wn * 64 + j * 32 + fr;
@@ -302,51 +306,223 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
         }
         return;
     }
-    if (g.epi == EPI_HIDDEN) {
-        constexpr int S = GT + 16;
-        static_assert(GT * S * sizeof(bf16) <= sizeof(sm), "bf16 output tile fits the operand LDS");
-        bf16 *cs = &sm[0][0][0][0];
+    constexpr int S = GT + 8;
+    static_assert(GT * S * sizeof(float) <= sizeof(sm), "fp32 output tile fits the operand LDS");
+    float *cs = reinterpret_cast<float *>(&sm[0][0][0][0]);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int c = wn * 64 + j * 32 + fr;
-            const float bias = g.bias[z * g.sBias + n0 + c];
+    for (int j = 0; j < 2; j++) {
+        const int c = wn * 64 + j * 32 + fr;
+        const float bias = g.bias ? g.bias[z * g.sBias + n0 + c] : 0.0f;
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+        for (int i = 0; i < 2; i++)
 #pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    const int rr = wm * 64 + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                    cs[rr * S + c] = (bf16)gelu(acc[i][j][q] + bias);
-                }
-        }
+            for (int q = 0; q < 16; q++) {
+                const int rr = wm * 64 + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
+                cs[rr * S + c] = acc[i][j][q] + bias;
+            }
+    }
+    __syncthreads();
+    float *dst = g.Cf + z * g.sCf;
+    for (int p = t; p < GT * (GT / 4); p += 256) {
+        const int rr = p / (GT / 4), c = (p % (GT / 4)) * 4;
+        *(f32x4 *)&dst[(int64_t)(m0 + rr) * g.ldc + n0 + c] = *(const f32x4 *)&cs[rr * S + c];
+    }
+}
+
+/* ---- the whole network in one kernel (prediction) ----
+ * One workgroup takes 64 inputs (32 where that is enough for every CU to have
+ * one) through every layer of one ensemble member: the activations stay in
+ * LDS (64 rows of 512 bf16, 66 KB; two workgroups a CU), and the weights
+ * stream from L2 straight into the registers that feed the matrix cores.
+ * Each of the 8 waves owns 64 of a layer's 512 columns for all rows (2 x 2
+ * blocks of v_mfma_f32_32x32x16_bf16), so no weight is read twice by a
+ * workgroup and the K loop has no barrier; the weights are the first operand,
+ * so a lane's accumulators run along the columns of one row and go back to
+ * LDS as 8-byte pieces.  The two workgroups of a CU are independent: one's
+ * GELU runs on the vector unit while the other's products run on the matrix
+ * cores.
+ *
+ * The weights are kept a second time in fragment order (k_pack_weights):
+ * block (nb, ks) of a layer holds the 64 lanes' 16-byte operands of columns
+ * 32 nb .. and k = 16 ks .., so every weight load is one contiguous KB.
+ *
+ * Tiles are dealt XCD-aware: the hardware hands workgroup b to XCD b % 8, so
+ * consecutive tiles of one member go to one XCD, whose L2 then holds that
+ * member's 1.7 MB of weights.
+ *
+ * Each output accumulates its k = 0, 16, 32, ... products in that order, as
+ * k_gemm does: the same bits.
+ *
+ * Bound: 262,144 inputs and 4 members take 1.94 ms, 930 TFLOP/s, of 0.9 ms
+ * the matrix cores need at the 1.95 GHz they run at here.  Timing variants:
+ * without the weights' L2 traffic (13 TB/s) 1.5 ms, with the identity for
+ * GELU 1.75 ms, without both 1.3 ms: what is left are the layers' ends, where
+ * the two workgroups cannot cover each other's latencies.  Tried: 4 waves of
+ * 128 columns 2.03 ms, 128 rows and one workgroup a CU 1.98 ms (half the L2
+ * traffic, nothing beside GELU), wave priorities and a staggered start no
+ * change.  The layer-by-layer products it replaced (128 x 128 tiles through
+ * LDS, activations through HBM) took 3.6 ms.
+ * 16 inputs: 20 us with 32-row tiles and 8 k-steps of weights in flight, 44
+ * with 64 rows and 4; five products one after the other took 62. */
+constexpr int MR = 64;            /* rows a prediction batch is padded to */
+constexpr int MLDS = HID + 8;     /* padded LDS row: conflict-free 16-byte fragment reads */
+constexpr int BIASES = NHID * HID + OUT_PAD;
+
+struct MlpArgs {
+    const float *x;               /* [n][6] */
+    int n;                        /* rows past it read as zero */
+    const bf16 *wp; int64_t sP;   /* weights in fragment order, per member */
+    const float *w; int64_t sW;   /* master parameters (biases) */
+    int64_t woff[NHID + 1], boff[NHID + 1];
+    float *logits; int64_t sL;    /* [E][rows][OUT_PAD] */
+    int MT, T;                    /* row tiles, row tiles x members */
+};
+
+/* parameters [E][total] -> fragment order; one thread per 16-byte operand */
+__global__ void k_pack_weights(const bf16 *__restrict__ wb, bf16 *__restrict__ wp, const Layout lay, int E) {
+    const int64_t per = (int64_t)lay.total / 8;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < per * E; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t z = i / per, q = (i % per) * 8;
+        int l = 0;
+        while (l < NHID && q >= (int64_t)lay.W[l + 1]) l++;
+        const int64_t r = q - (int64_t)lay.W[l];
+        const int K = lay.in[l];
+        if (r >= (int64_t)K * lay.out[l]) continue;   /* biases */
+        const int64_t f = r / 512;                    /* fragment (nb, ks) */
+        const int lane = (int)(r % 512) / 8, KS = K / 16;
+        const int nb = (int)(f / KS), ks = (int)(f % KS);
+        const int64_t src = (int64_t)lay.W[l] + (int64_t)(nb * 32 + (lane & 31)) * K + ks * 16 + 8 * (lane >> 5);
+        *(bf16x8 *)(wp + z * (int64_t)lay.total + q) = *(const bf16x8 *)(wb + z * (int64_t)lay.total + src);
+    }
+}
+
+/* RB: blocks of 32 rows per workgroup; DEPTH: k-steps of weights in flight
+ * per wave */
+template <int RB, int DEPTH, int EU>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void k_mlp(const MlpArgs g) {
+    constexpr int WAVES = 8, JB = 16 / WAVES, ROWS = 32 * RB, KS = HID / 16;
+    __shared__ __attribute__((aligned(16))) bf16 act[ROWS][MLDS];
+    __shared__ __attribute__((aligned(16))) float bias[BIASES];
+    const int b = (int)blockIdx.x;
+    const int xcd = b & 7, rr = b >> 3;
+    const int per = g.T >> 3, rem = g.T & 7;
+    const int L = xcd < rem ? xcd * (per + 1) + rr : rem * (per + 1) + (xcd - rem) * per + rr;
+    const int z = L / g.MT, m0 = (L % g.MT) * ROWS;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 31, hi = lane >> 5;
+    const bf16 *wp = g.wp + z * g.sP;
+    const float *par = g.w + z * g.sW;
+    /* weight operands of this wave's column blocks JB w .. JB w + JB - 1 */
+    bf16x8 fb[DEPTH][JB];
+    auto fetch = [&](const bf16x8 *p, int ks, int steps, int u) {
+#pragma unroll
+        for (int j = 0; j < JB; j++) fb[u][j] = p[((int64_t)j * steps + ks) * 64];
+    };
+    auto weights = [&](int l, int steps) { return (const bf16x8 *)(wp + g.woff[l]) + (int64_t)(JB * w) * steps * 64 + lane; };
+    fetch(weights(0, IN_PAD / 16), 0, IN_PAD / 16, 0);
+    for (int k = t; k < BIASES; k += 64 * WAVES) bias[k] = par[g.boff[k / HID] + k % HID];
+    for (int k = t; k < ROWS * 4; k += 64 * WAVES) {   /* inputs: 6 features in the first k-step, the rest of it zero */
+        const int r = k >> 2, c = (k & 3) * 4;
+        bf16x4 v;
+#pragma unroll
+        for (int q = 0; q < 4; q++) v[q] = (bf16)(c + q < 6 && m0 + r < g.n ? g.x[(int64_t)(m0 + r) * 6 + c + q] : 0.0f);
+        *(bf16x4 *)&act[r][c] = v;
+    }
+    f32x16 acc[RB][JB];
+    bf16x8 fa[2][RB];
+    auto rows = [&](int ks, int v) {
+#pragma unroll
+        for (int i = 0; i < RB; i++) fa[v][i] = *(const bf16x8 *)&act[i * 32 + fr][ks * 16 + 8 * hi];
+    };
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int j = 0; j < JB; j++) acc[i][j] = f32x16{};
+    };
+    auto step = [&](int u, int v) {
+#pragma unroll
+        for (int j = 0; j < JB; j++)
+#pragma unroll
+            for (int i = 0; i < RB; i++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[u][j], fa[v][i], acc[i][j], 0, 0, 0);
+    };
+    /* acc -> bias, GELU, bf16 -> act.  Accumulator r of lane l of block (i, j)
+     * is row 32 i + l % 32, column 32 (JB w + j) + 8 (r/4) + 4 (l/32) + r%4. */
+    auto activate = [&](int l) {
+        bf16x4 pk[RB][JB][4];
+#pragma unroll
+        for (int j = 0; j < JB; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const f32x4 bv = *(const f32x4 *)&bias[l * HID + 32 * (JB * w + j) + 8 * q + 4 * hi];
+#pragma unroll
+                for (int i = 0; i < RB; i++)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) pk[i][j][q][k] = (bf16)gelu(acc[i][j][4 * q + k] + bv[k]);
+            }
+        __syncthreads();   /* every wave has read this layer's inputs */
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int j = 0; j < JB; j++)
+#pragma unroll
+                for (int q = 0; q < 4; q++) *(bf16x4 *)&act[i * 32 + fr][32 * (JB * w + j) + 8 * q + 4 * hi] = pk[i][j][q];
         __syncthreads();
-        bf16 *dst = g.Cb + z * g.sCb;
-        for (int p = t; p < GT * (GT / 8); p += 256) {
-            const int rr = p / (GT / 8), c = (p % (GT / 8)) * 8;
-            *(bf16x8 *)&dst[(int64_t)(m0 + rr) * g.ldc + n0 + c] = *(const bf16x8 *)&cs[rr * S + c];
-        }
-    } else {
-        constexpr int S = GT + 8;
-        static_assert(GT * S * sizeof(float) <= sizeof(sm), "fp32 output tile fits the operand LDS");
-        typedef float f32x4 __attribute__((ext_vector_type(4)));
-        float *cs = reinterpret_cast<float *>(&sm[0][0][0][0]);
+    };
+    __syncthreads();
+    /* layer 1: one k-step holds all six inputs */
+    clear();
+    rows(0, 0);
+    step(0, 0);
 #pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int c = wn * 64 + j * 32 + fr;
-            const float bias = g.bias ? g.bias[z * g.sBias + n0 + c] : 0.0f;
+    for (int u = 0; u < DEPTH; u++) fetch(weights(1, KS), u, KS, u);
+    activate(0);
+    for (int l = 1; l < NHID; l++) {
+        const bf16x8 *p = weights(l, KS);
+        clear();
+        rows(0, 0);
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks + 1 < KS) rows(ks + 1, (ks + 1) & 1);
+            step(ks % DEPTH, ks & 1);
+            if (ks + DEPTH < KS) fetch(p, ks + DEPTH, KS, ks % DEPTH);
+        }
+        /* the next hidden layer's first operands arrive during this one's epilogue */
+        if (l + 1 < NHID) {
 #pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    const int rr = wm * 64 + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                    cs[rr * S + c] = acc[i][j][q] + bias;
-                }
+            for (int u = 0; u < DEPTH; u++) fetch(weights(l + 1, KS), u, KS, u);
         }
-        __syncthreads();
-        float *dst = g.Cf + z * g.sCf;
-        for (int p = t; p < GT * (GT / 4); p += 256) {
-            const int rr = p / (GT / 4), c = (p % (GT / 4)) * 4;
-            *(f32x4 *)&dst[(int64_t)(m0 + rr) * g.ldc + n0 + c] = *(const f32x4 *)&cs[rr * S + c];
+        activate(l);
+    }
+    /* output layer: four column blocks, one each for the first four waves */
+    if (w < 4) {
+        const bf16x8 *po = (const bf16x8 *)(wp + g.woff[NHID]) + (int64_t)w * KS * 64 + lane;
+        f32x16 o[RB];
+#pragma unroll
+        for (int i = 0; i < RB; i++) o[i] = f32x16{};
+        bf16x8 fo[16];
+#pragma unroll
+        for (int k = 0; k < 16; k++) fo[k] = po[k * 64];
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            rows(ks, 0);
+#pragma unroll
+            for (int i = 0; i < RB; i++) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fo[ks % 16], fa[0][i], o[i], 0, 0, 0);
+            if (ks + 16 < KS) fo[ks % 16] = po[(ks + 16) * 64];
         }
+        float *dst = g.logits + z * g.sL + (int64_t)m0 * OUT_PAD;
+#pragma unroll
+        for (int i = 0; i < RB; i++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int c = 32 * w + 8 * q + 4 * hi;
+                const f32x4 bv = *(const f32x4 *)&bias[NHID * HID + c];
+                f32x4 v;
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[k] = o[i][4 * q + k] + bv[k];
+                *(f32x4 *)&dst[(int64_t)(i * 32 + fr) * OUT_PAD + c] = v;
+            }
     }
 }
 
@@ -515,6 +691,8 @@ struct gf_sg_model {
     OwnedStream cst;  /* prediction read-back, beside the next batch's compute on st */
     DevBuf<float> w, g, m, v;       /* [E][total] */
     DevBuf<bf16> wb;
+    DevBuf<bf16> wp;                /* weights in fragment order (prediction) */
+    bool wp_stale = true;           /* the weights have changed since wp was written */
     DevBuf<bf16> x;                 /* [B][64] */
     DevBuf<float> Z;                /* [E][NHID][B][512] */
     DevBuf<bf16> H;                 /* [E][NHID][B][512] */
@@ -522,7 +700,7 @@ struct gf_sg_model {
     DevBuf<bf16> dlog;              /* [E][B][128] */
     DevBuf<bf16> dz0, dz1;          /* [E][B][512] */
     DevBuf<float> y, tot, loss, xin;
-    DevBuf<float> psfs, ptot, pdis; /* two batches' prediction outputs */
+    DevBuf<float> pout;             /* two batches' prediction outputs */
     int64_t step = 0;
     float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
 };
@@ -537,7 +715,6 @@ static int gemm(gf_sg_model &S, GemmArgs a) {
         const int MT = a.M / GT, NT = a.N / GT, T = MT * NT * S.E;
         hipLaunchKernelGGL(k_gemm_nt, dim3(T), dim3(256), 0, S.st, a, MT, NT, T);
     } else {
-        if (a.epi == EPI_HIDDEN && !a.Cf) { set_error("surrogate gemm: small products keep Z"); return GF_ERR_ARG; }
         hipLaunchKernelGGL(k_gemm, dim3(a.N / TILE, a.M / TILE, S.E), dim3(256), 0, S.st, a);
     }
     GF_HIP(hipGetLastError());
@@ -557,17 +734,66 @@ static int ensure_batch(gf_sg_model &S, int B) {
     GF_TRY(S.y.alloc((size_t)B * NBINS));
     GF_TRY(S.tot.alloc(B));
     GF_TRY(S.xin.alloc((size_t)B * 6));
-    GF_TRY(S.psfs.alloc((size_t)2 * B * NBINS));
-    GF_TRY(S.ptot.alloc((size_t)2 * B));
-    GF_TRY(S.pdis.alloc((size_t)2 * B));
     S.Bmax = B;
     return GF_OK;
 }
 
-/* forward pass of the whole ensemble on S.x (B rows); keep_z: also store
- * the hidden layers' pre-activations Z (the backward pass reads them) */
-static int forward(gf_sg_model &S, int B, bool keep_z) {
-    keep_z = keep_z || B < 4096 || B % GT != 0;   /* k_gemm always stores Z */
+/* buffers of prediction batches of up to B rows; host: also two batches'
+ * inputs and outputs */
+static int ensure_predict(gf_sg_model &S, int B, bool host) {
+    GF_TRY(S.wp.alloc((size_t)S.E * S.lay.total));
+    GF_TRY(S.logits.alloc((size_t)S.E * B * OUT_PAD));
+    if (host) {
+        GF_TRY(S.xin.alloc((size_t)B * 6));
+        GF_TRY(S.pout.alloc((size_t)2 * B * POUT));
+    }
+    return GF_OK;
+}
+
+/* logits of the whole ensemble for n rows of x (device, [n][6]), B = n
+ * rounded up to MR rows: S.logits [E][B][128] */
+static int predict_logits(gf_sg_model &S, const float *x, int n, int B) {
+    const Layout &L = S.lay;
+    if (S.wp_stale) {
+        hipLaunchKernelGGL(k_pack_weights, dim3(1024), dim3(256), 0, S.st, S.wb.p, S.wp.p, L, S.E);
+        GF_HIP(hipGetLastError());
+        S.wp_stale = false;
+    }
+    MlpArgs a{};
+    a.x = x;
+    a.n = n;
+    a.wp = S.wp.p; a.sP = (int64_t)L.total;
+    a.w = S.w.p; a.sW = (int64_t)L.total;
+    for (int l = 0; l <= NHID; l++) { a.woff[l] = (int64_t)L.W[l]; a.boff[l] = (int64_t)L.b[l]; }
+    a.logits = S.logits.p; a.sL = (int64_t)B * OUT_PAD;
+    /* 32-row tiles as long as they give each CU at most one workgroup (whole
+     * call, 4 members: 1,024 inputs 40 us against 52, 2,048 44 against 54,
+     * 4,096 62 against 59) */
+    const int tiles32 = (n + 31) / 32;
+    if ((int64_t)tiles32 * S.E <= num_cus()) {
+        a.MT = tiles32;
+        a.T = a.MT * S.E;
+        hipLaunchKernelGGL((k_mlp<1, 8, 2>), dim3(a.T), dim3(512), 0, S.st, a);
+    } else {
+        a.MT = B / MR;
+        a.T = a.MT * S.E;
+        hipLaunchKernelGGL((k_mlp<2, 4, 4>), dim3(a.T), dim3(512), 0, S.st, a);
+    }
+    GF_HIP(hipGetLastError());
+    return GF_OK;
+}
+
+/* ensemble statistics of the cnt rows predict_logits left in S.logits */
+static int predict_stats(gf_sg_model &S, int cnt, float *sfs, float *tot, float *dis) {
+    const int64_t sL = (int64_t)((cnt + MR - 1) / MR * MR) * OUT_PAD;
+    hipLaunchKernelGGL(k_predict_stats, dim3((cnt + 3) / 4), dim3(256), 0, S.st, S.logits.p, sL, S.E, cnt, sfs, tot, dis);
+    GF_HIP(hipGetLastError());
+    return GF_OK;
+}
+
+/* forward pass of the whole ensemble on S.x (B rows) for training: also
+ * stores the hidden layers' pre-activations Z (the backward pass reads them) */
+static int forward(gf_sg_model &S, int B) {
     const Layout &L = S.lay;
     const int64_t sW = (int64_t)L.total;
     const int64_t sAct = (int64_t)NHID * B * HID;
@@ -581,7 +807,7 @@ static int forward(gf_sg_model &S, int B, bool keep_z) {
         a.bias = S.w.p + L.b[l]; a.sBias = sW;
         if (l < NHID) {
             a.epi = EPI_HIDDEN;
-            a.Cf = keep_z ? S.Z.p + (int64_t)l * B * HID : nullptr; a.sCf = sAct; a.ldc = HID;
+            a.Cf = S.Z.p + (int64_t)l * B * HID; a.sCf = sAct; a.ldc = HID;
             a.Cb = S.H.p + (int64_t)l * B * HID; a.sCb = sAct;
         } else {
             a.epi = EPI_OUTPUT;
@@ -598,7 +824,7 @@ static int train_step(gf_sg_model &S, int B, float lr, float w_tot, bool update)
     const int E = S.E;
     const int64_t sW = (int64_t)L.total;
     const int64_t sAct = (int64_t)NHID * B * HID;
-    GF_TRY(forward(S, B, true));
+    GF_TRY(forward(S, B));
     hipLaunchKernelGGL(k_loss, dim3((B + 127) / 128, E), dim3(128), 0, S.st, S.logits.p, (int64_t)B * OUT_PAD,
                        S.y.p, S.tot.p, B, w_tot, S.dlog.p, (int64_t)B * OUT_PAD, S.loss.p);
     GF_HIP(hipGetLastError());
@@ -637,6 +863,7 @@ static int train_step(gf_sg_model &S, int B, float lr, float w_tot, bool update)
         const float c1 = 1.0f - std::pow(S.b1, (float)S.step);
         const float c2 = 1.0f - std::pow(S.b2, (float)S.step);
         const int64_t n = (int64_t)E * L.total;
+        S.wp_stale = true;
         hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, S.st, S.w.p, S.wb.p, S.g.p, S.m.p, S.v.p, n, lr, S.b1,
                            S.b2, S.eps, c1, c2);
         GF_HIP(hipGetLastError());
@@ -719,6 +946,7 @@ int32_t gf_sg_set_params(gf_sg_model *S, const float *in) {
     if (!S || !in) return GF_ERR_ARG;
     const size_t n = (size_t)S->E * S->lay.total;
     GF_HIP(hipMemcpy(S->w.p, in, n * sizeof(float), hipMemcpyHostToDevice));
+    S->wp_stale = true;
     hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, S->st, S->w.p, S->wb.p, (int64_t)n);
     GF_HIP(hipGetLastError());
     GF_HIP(hipStreamSynchronize(S->st));
@@ -792,52 +1020,48 @@ int32_t gf_sg_train(gf_sg_model *S, const float *x, const float *y, const float 
 }
 
 /* ensemble prediction for n inputs: mean normalised SFS (bins 1..99),
- * mean log-total and the ensemble disagreement per input.  Batches of up
+ * mean log-total and the ensemble disagreement per input.  A batch's outputs
+ * ([cnt][99], [cnt], [cnt], contiguous) come back in one copy.  Batches of up
  * to 65,536 inputs alternate between two output buffers: while batch i is
  * computed on the model's stream, batch i - 1 is read back on the copy
- * stream (each waits for the other through events). */
+ * stream (each waits for the other through events); a single batch is read
+ * back on the model's stream itself. */
 int32_t gf_sg_predict(gf_sg_model *S, const float *x, int32_t n, float *sfs, float *tot, float *dis) {
     if (!S || !x || n <= 0 || !sfs) { set_error("gf_sg_predict: invalid arguments"); return GF_ERR_ARG; }
     StreamScope scope(S->st);   /* buffers (re)allocated here belong to the model's stream */
-    GF_HIP(S->cst.create());
-    const int B = std::min(65536, ((n + GT - 1) / GT) * GT);
-    GF_TRY(ensure_batch(*S, B));
+    const int B = std::min(65536, ((n + MR - 1) / MR) * MR);
+    GF_TRY(ensure_predict(*S, B, true));
+    const int nb = (n + B - 1) / B;
     struct Events {   /* [0..1] computed, [2..3] read back, per output buffer */
         hipEvent_t e[4] = {nullptr, nullptr, nullptr, nullptr};
         ~Events() { for (auto v : e) if (v) (void)hipEventDestroy(v); }
     } ev;
-    for (auto &v : ev.e) GF_HIP(hipEventCreateWithFlags(&v, hipEventDisableTiming));
-    std::vector<float> xb[2];   /* a batch's inputs stay untouched until its compute has started */
-    for (auto &v : xb) v.assign((size_t)B * 6, 0.0f);
-    const int nb = (n + B - 1) / B;
+    if (nb > 1) {
+        GF_HIP(S->cst.create());
+        for (auto &v : ev.e) GF_HIP(hipEventCreateWithFlags(&v, hipEventDisableTiming));
+    }
     for (int i = 0; i <= nb; i++) {
         if (i < nb) {
             const int off = i * B, cnt = std::min(B, n - off), u = i & 1;
-            memcpy(xb[u].data(), x + (size_t)off * 6, (size_t)cnt * 6 * sizeof(float));
-            if (cnt < B) memset(xb[u].data() + (size_t)cnt * 6, 0, (size_t)(B - cnt) * 6 * sizeof(float));
+            float *out = S->pout.p + (size_t)u * B * POUT;
             if (i >= 2) GF_HIP(hipStreamWaitEvent(S->st, ev.e[2 + u], 0));   /* buffer u read back */
-            GF_TRY(load_batch(*S, xb[u].data(), nullptr, nullptr, B));
-            GF_TRY(forward(*S, B, false));
-            hipLaunchKernelGGL(k_predict_stats, dim3((B + 3) / 4), dim3(256), 0, S->st, S->logits.p,
-                               (int64_t)B * OUT_PAD, S->E, B, S->psfs.p + (size_t)u * B * NBINS,
-                               S->ptot.p + (size_t)u * B, S->pdis.p + (size_t)u * B);
-            GF_HIP(hipGetLastError());
-            GF_HIP(hipEventRecord(ev.e[u], S->st));
+            GF_HIP(hipMemcpyAsync(S->xin.p, x + (size_t)off * 6, (size_t)cnt * 6 * sizeof(float), hipMemcpyHostToDevice, S->st));
+            GF_TRY(predict_logits(*S, S->xin.p, cnt, (cnt + MR - 1) / MR * MR));
+            GF_TRY(predict_stats(*S, cnt, out, out + (size_t)cnt * NBINS, out + (size_t)cnt * (NBINS + 1)));
+            if (nb > 1) GF_HIP(hipEventRecord(ev.e[u], S->st));
         }
         if (i >= 1) {
             const int j = i - 1, off = j * B, cnt = std::min(B, n - off), u = j & 1;
-            GF_HIP(hipStreamWaitEvent(S->cst, ev.e[u], 0));
-            /* the spectra (99 floats per input) through the pinned staging path */
-            GF_TRY(readback(sfs + (size_t)off * NBINS, S->psfs.p + (size_t)u * B * NBINS,
-                            (size_t)cnt * NBINS * sizeof(float), S->cst));
-            if (tot) GF_HIP(hipMemcpyAsync(tot + off, S->ptot.p + (size_t)u * B, (size_t)cnt * sizeof(float),
-                                           hipMemcpyDeviceToHost, S->cst));
-            if (dis) GF_HIP(hipMemcpyAsync(dis + off, S->pdis.p + (size_t)u * B, (size_t)cnt * sizeof(float),
-                                           hipMemcpyDeviceToHost, S->cst));
-            GF_HIP(hipEventRecord(ev.e[2 + u], S->cst));
+            hipStream_t st = nb > 1 ? (hipStream_t)S->cst : (hipStream_t)S->st;
+            if (nb > 1) GF_HIP(hipStreamWaitEvent(st, ev.e[u], 0));
+            const ReadPart parts[3] = {{sfs + (size_t)off * NBINS, (size_t)cnt * NBINS * sizeof(float)},
+                                       {tot ? tot + off : nullptr, (size_t)cnt * sizeof(float)},
+                                       {dis ? dis + off : nullptr, (size_t)cnt * sizeof(float)}};
+            GF_TRY(readback_parts(parts, 3, S->pout.p + (size_t)u * B * POUT, st));
+            if (nb > 1) GF_HIP(hipEventRecord(ev.e[2 + u], st));
         }
     }
-    GF_HIP(hipStreamSynchronize(S->cst));
+    if (nb > 1) GF_HIP(hipStreamSynchronize(S->cst));
     GF_HIP(hipStreamSynchronize(S->st));
     return GF_OK;
 }
@@ -860,17 +1084,12 @@ int32_t gf_sg_predict_device(gf_sg_model *S, const float *x, int32_t n, float *s
         }
     }
     StreamScope scope(S->st);
-    const int B = std::min(65536, ((n + GT - 1) / GT) * GT);
-    GF_TRY(ensure_batch(*S, B));
+    const int B = std::min(65536, ((n + MR - 1) / MR) * MR);
+    GF_TRY(ensure_predict(*S, B, false));
     for (int off = 0; off < n; off += B) {
         const int cnt = std::min(B, n - off);
-        hipLaunchKernelGGL(k_pack_inputs, dim3((B * IN_PAD + 255) / 256), dim3(256), 0, S->st, x + (size_t)off * 6, B,
-                           cnt, 6, S->x.p);
-        GF_HIP(hipGetLastError());
-        GF_TRY(forward(*S, B, false));
-        hipLaunchKernelGGL(k_predict_stats, dim3((cnt + 3) / 4), dim3(256), 0, S->st, S->logits.p, (int64_t)B * OUT_PAD,
-                           S->E, cnt, sfs + (size_t)off * NBINS, tot ? tot + off : nullptr, dis ? dis + off : nullptr);
-        GF_HIP(hipGetLastError());
+        GF_TRY(predict_logits(*S, x + (size_t)off * 6, cnt, (cnt + MR - 1) / MR * MR));
+        GF_TRY(predict_stats(*S, cnt, sfs + (size_t)off * NBINS, tot ? tot + off : nullptr, dis ? dis + off : nullptr));
     }
     GF_HIP(hipStreamSynchronize(S->st));
     return GF_OK;
@@ -878,14 +1097,13 @@ int32_t gf_sg_predict_device(gf_sg_model *S, const float *x, int32_t n, float *s
 
 /* raw ensemble logits for n inputs (n a multiple of 64): [E][n][128] */
 int32_t gf_sg_forward(gf_sg_model *S, const float *x, int32_t n, float *logits) {
-    if (!S || !x || !logits || n <= 0 || n % TILE) { set_error("gf_sg_forward: invalid arguments"); return GF_ERR_ARG; }
+    if (!S || !x || !logits || n <= 0 || n % MR) { set_error("gf_sg_forward: invalid arguments"); return GF_ERR_ARG; }
     StreamScope scope(S->st);   /* buffers (re)allocated here belong to the model's stream */
-    GF_TRY(ensure_batch(*S, n));
-    GF_TRY(load_batch(*S, x, nullptr, nullptr, n));
-    GF_TRY(forward(*S, n, false));
+    GF_TRY(ensure_predict(*S, n, true));
+    GF_HIP(hipMemcpyAsync(S->xin.p, x, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, S->st));
+    GF_TRY(predict_logits(*S, S->xin.p, n, n));
+    GF_TRY(readback(logits, S->logits.p, (size_t)S->E * n * OUT_PAD * sizeof(float), S->st));
     GF_HIP(hipStreamSynchronize(S->st));
-    for (int e = 0; e < S->E; e++)
-        GF_HIP(hipMemcpy(logits + (size_t)e * n * OUT_PAD, S->logits.p + (size_t)e * n * OUT_PAD, (size_t)n * OUT_PAD * sizeof(float), hipMemcpyDeviceToHost));
     return GF_OK;
 }
 
