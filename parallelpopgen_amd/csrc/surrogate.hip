@@ -7,12 +7,13 @@
  * (99 softmax logits for the n = 100 SFS bins 1..99, one log-total head),
  * BF16 weights and activations, FP32 accumulation, trained by this file's
  * forward, backward and Adam kernels.  Every matrix product runs on the
- * gfx950 matrix cores (v_mfma_f32_32x32x16_bf16): k_gemm's global->LDS
- * stage handles the three operand layouts of forward (X W^T), input
- * gradient (dZ W) and weight gradient (dZ^T X) at training batch sizes,
- * k_gemm_nt the forward products of large training batches, the ensemble
- * members being the grid's z dimension; k_mlp runs the whole network for
- * prediction.
+ * gfx950 matrix cores (v_mfma_f32_32x32x16_bf16) from operands kept in
+ * fragment order, so that a wave's load is one contiguous KB:
+ *   k_mlp            prediction: the whole network in one kernel
+ *   k_train_rows     training: forward, loss and the backward chain of 16
+ *                    rows in one kernel
+ *   k_train_weights  training: every layer's weight and bias gradients and
+ *                    their Adam update in one kernel
  */
 #include "gf_runtime.hpp"
 
@@ -37,9 +38,6 @@ constexpr int OUT = 100;      /* 99 bins + log-total */
 constexpr int OUT_PAD = 128;
 constexpr int NBINS = 99;
 constexpr int POUT = NBINS + 2;   /* floats of one prediction: bins, log-total, disagreement */
-constexpr int TILE = 64;
-constexpr int KSTEP = 32;
-constexpr int LDSK = KSTEP + 8; /* padded LDS row (bf16 elements) */
 
 /* parameter layout of one model, in floats */
 struct Layout {
@@ -81,254 +79,6 @@ __device__ __forceinline__ float gelu_grad(float x) {
     return sg + 2.0f * x * sg * (1.0f - sg) * du;
 }
 
-enum Epi { EPI_HIDDEN = 0, EPI_OUTPUT = 1, EPI_DX = 2, EPI_DW = 3 };
-
-struct GemmArgs {
-    const bf16 *A; int64_t lda; int a_km; int64_t sA;   /* A(m,k) = a_km ? A[k*lda+m] : A[m*lda+k] */
-    const bf16 *B; int64_t ldb; int b_nk; int64_t sB;   /* B(k,n) = b_nk ? B[n*ldb+k] : B[k*ldb+n] */
-    int M, N, K;
-    /* epilogue */
-    const float *bias; int64_t sBias;
-    float *Cf; int64_t ldc; int64_t sCf;                 /* fp32 output (Z, logits, dW) */
-    bf16 *Cb; int64_t sCb;                               /* bf16 output (H or dZ) */
-    const float *Zprev; int64_t sZ;                      /* pre-activation for GELU' */
-    int epi;
-};
-
-/* C = A B (+ epilogue), 64x64 tile per workgroup of 4 waves; each wave owns
- * a 32x32 sub-tile accumulated by 32x32x16 BF16 MFMAs from LDS. */
-__global__ __launch_bounds__(256) void k_gemm(const GemmArgs g) {
-    __shared__ bf16 As[TILE][LDSK];   /* [m][k] */
-    __shared__ bf16 Bs[TILE][LDSK];   /* [n][k] */
-    const int z = blockIdx.z;
-    const bf16 *A = g.A + z * g.sA;
-    const bf16 *B = g.B + z * g.sB;
-    const int m0 = blockIdx.y * TILE, n0 = blockIdx.x * TILE;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    f32x16 acc = {};
-    for (int k0 = 0; k0 < g.K; k0 += KSTEP) {
-        /* ---- global -> LDS: 64 x 32 elements of each operand ---- */
-        if (!g.a_km) {
-            const int m = t >> 2, kc = (t & 3) * 8;
-            const bf16x8 v = *(const bf16x8 *)(A + (int64_t)(m0 + m) * g.lda + k0 + kc);
-            *(bf16x8 *)&As[m][kc] = v;
-        } else {
-            const int k = t >> 3, mc = (t & 7) * 8;
-            const bf16x8 v = *(const bf16x8 *)(A + (int64_t)(k0 + k) * g.lda + m0 + mc);
-#pragma unroll
-            for (int q = 0; q < 8; q++) As[mc + q][k] = v[q];
-        }
-        if (g.b_nk) {
-            const int n = t >> 2, kc = (t & 3) * 8;
-            const bf16x8 v = *(const bf16x8 *)(B + (int64_t)(n0 + n) * g.ldb + k0 + kc);
-            *(bf16x8 *)&Bs[n][kc] = v;
-        } else {
-            const int k = t >> 3, nc = (t & 7) * 8;
-            const bf16x8 v = *(const bf16x8 *)(B + (int64_t)(k0 + k) * g.ldb + n0 + nc);
-#pragma unroll
-            for (int q = 0; q < 8; q++) Bs[nc + q][k] = v[q];
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < KSTEP; kk += 16) {
-            const bf16x8 a = *(const bf16x8 *)&As[wm * 32 + (lane & 31)][kk + 8 * (lane >> 5)];
-            const bf16x8 b = *(const bf16x8 *)&Bs[wn * 32 + (lane & 31)][kk + 8 * (lane >> 5)];
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-        }
-        __syncthreads();
-    }
-    /* ---- epilogue: accumulator r of lane l is C[8(r/4) + 4(l/32) + r%4][l%32] ---- */
-    const int n = n0 + wn * 32 + (lane & 31);
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-        const int m = m0 + wm * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-        const int64_t o = (int64_t)m * g.ldc + n;
-        const float v = acc[r];
-        if (g.epi == EPI_HIDDEN) {
-            const float zz = v + g.bias[z * g.sBias + n];
-            g.Cf[z * g.sCf + o] = zz;
-            g.Cb[z * g.sCb + o] = (bf16)gelu(zz);
-        } else if (g.epi == EPI_OUTPUT) {
-            g.Cf[z * g.sCf + o] = v + g.bias[z * g.sBias + n];
-        } else if (g.epi == EPI_DX) {
-            g.Cb[z * g.sCb + o] = (bf16)(v * gelu_grad(g.Zprev[z * g.sZ + o]));
-        } else {
-            g.Cf[z * g.sCf + o] = v;
-        }
-    }
-}
-
-/* ---- large forward products: C = A B^T with both operands K-contiguous ----
- * (training at batches of thousands of rows).  A
- * 128 x 128 tile per workgroup of 4 waves, each wave a 64 x 64 quadrant of
- * 2 x 2 blocks of v_mfma_f32_32x32x16_bf16; K in stages of 64 through two
- * LDS buffers, fed from two register sets: stage s + 2's global loads are
- * issued before stage s's MFMAs, and stage s + 1 (loaded during stage
- * s - 1) is stored to the other buffer after them, one barrier per stage.
- * The register sets and accumulators take 231 VGPRs, held to two waves per
- * SIMD.  Each output element accumulates its k = 0, 16, 32, ... products
- * in the same order as k_gemm, so both kernels give the same bits.
- *
- * Tiles are dealt XCD-aware: the hardware hands workgroup b to XCD b % 8,
- * so tile L is given to the workgroup that puts the tiles of one stretch of
- * L (the N tiles of an M tile, fastest) on one XCD, where they share the A
- * rows in that XCD's L2. */
-constexpr int GT = 128;
-constexpr int GK = 64;
-constexpr int GLDS = GK + 8;   /* padded LDS row: conflict-free 16-byte fragment reads */
-constexpr int GR = GK / 8;     /* threads per tile row in the global -> LDS copy */
-constexpr int GRS = 256 / GR;  /* rows one pass of the workgroup copies */
-constexpr int GP = GT / GRS;   /* passes per operand and stage */
-
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_gemm_nt(const GemmArgs g, int MT, int NT, int T) {
-    /* operand stages; after the K loop the same LDS stages the output tile */
-    __shared__ __attribute__((aligned(16))) bf16 sm[2][2][GT][GLDS];
-    auto &As = sm[0];
-    auto &Bs = sm[1];
-    const int b = (int)blockIdx.x;
-    const int xcd = b & 7, r = b >> 3;
-    const int per = T >> 3, rem = T & 7;
-    const int L = xcd < rem ? xcd * (per + 1) + r : rem * (per + 1) + (xcd - rem) * per + r;
-    const int nt = L % NT, mt = (L / NT) % MT, z = L / (NT * MT);
-    const bf16 *A = g.A + z * g.sA;
-    const bf16 *B = g.B + z * g.sB;
-    const int m0 = mt * GT, n0 = nt * GT;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wm = w >> 1, wn = w & 1;
-    /* global -> LDS: each thread moves rows lr + GRS i (i < GP), 8 bf16 at column lk */
-    const int lr = t / GR, lk = (t % GR) * 8;
-    const bf16 *pa = A + (int64_t)(m0 + lr) * g.lda + lk;
-    const bf16 *pb = B + (int64_t)(n0 + lr) * g.ldb + lk;
-    const int64_t da = GRS * g.lda, db = GRS * g.ldb;
-    /* stage s + 1's operands wait in registers while stage s is in LDS:
-     * two register sets, loads issued two stages ahead */
-    bf16x8 ra[2][GP], rb[2][GP];
-    const int ns = g.K / GK;
-    auto load = [&](bf16x8 (&xa)[GP], bf16x8 (&xb)[GP], int k1) {
-#pragma unroll
-        for (int i = 0; i < GP; i++) {
-            xa[i] = *(const bf16x8 *)(pa + i * da + k1);
-            xb[i] = *(const bf16x8 *)(pb + i * db + k1);
-        }
-    };
-    auto store = [&](const bf16x8 (&xa)[GP], const bf16x8 (&xb)[GP], int buf) {
-#pragma unroll
-        for (int i = 0; i < GP; i++) {
-            *(bf16x8 *)&As[buf][lr + GRS * i][lk] = xa[i];
-            *(bf16x8 *)&Bs[buf][lr + GRS * i][lk] = xb[i];
-        }
-    };
-    f32x16 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; i++)
-#pragma unroll
-        for (int j = 0; j < 2; j++) acc[i][j] = f32x16{};
-    const int fr = lane & 31, fk = 8 * (lane >> 5);
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int kk = 0; kk < GK; kk += 16) {
-            bf16x8 fa[2], fb[2];
-#pragma unroll
-            for (int i = 0; i < 2; i++) fa[i] = *(const bf16x8 *)&As[buf][wm * 64 + i * 32 + fr][kk + fk];
-#pragma unroll
-            for (int j = 0; j < 2; j++) fb[j] = *(const bf16x8 *)&Bs[buf][wn * 64 + j * 32 + fr][kk + fk];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int j = 0; j < 2; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[i], fb[j], acc[i][j], 0, 0, 0);
-        }
-    };
-    /* every load of the steady-state loop is unconditional, so that the
-     * compiler's wait before a store counts only the older register set
-     * (a load under a branch makes it wait for both) */
-    load(ra[0], rb[0], 0);
-    load(ra[1], rb[1], ns > 1 ? GK : 0);   /* one stage: a harmless reload */
-    store(ra[0], rb[0], 0);
-    __syncthreads();
-    /* at the top of each pass: stage s in LDS buffer 0, stage s + 1 in
-     * flight into register set 1, set 0 free (its stage was stored in the
-     * previous pass).  A buffer is written only after the barrier that
-     * ended the last stage reading it. */
-    int s = 0;
-    for (; s + 3 < ns; s += 2) {
-        load(ra[0], rb[0], (s + 2) * GK);
-        __builtin_amdgcn_sched_barrier(0);   /* keep the loads ahead of the MFMAs */
-        compute(0);
-        store(ra[1], rb[1], 1);
-        __syncthreads();
-        load(ra[1], rb[1], (s + 3) * GK);
-        __builtin_amdgcn_sched_barrier(0);   /* keep the loads ahead of the MFMAs */
-        compute(1);
-        store(ra[0], rb[0], 0);
-        __syncthreads();
-    }
-    const int left = ns - s;   /* 1, 2 or 3 stages */
-    if (left == 3) {
-        load(ra[0], rb[0], (s + 2) * GK);
-        __builtin_amdgcn_sched_barrier(0);   /* keep the loads ahead of the MFMAs */
-        compute(0);
-        store(ra[1], rb[1], 1);
-        __syncthreads();
-        compute(1);
-        store(ra[0], rb[0], 0);
-        __syncthreads();
-        compute(0);
-    } else if (left == 2) {
-        compute(0);
-        store(ra[1], rb[1], 1);
-        __syncthreads();
-        compute(1);
-    } else {
-        compute(0);
-    }
-    __syncthreads();
-    /* epilogue: accumulator r of lane l is C[8(r/4) + 4(l/32) + r%4][l%32]
-     * of its block.  An output tile goes through LDS (free after the loop's
-     * last barrier) so that global stores are whole 16-byte row pieces: a
-     * lane's accumulators run down a column.  A row stride of 136 floats puts
-     * the two half-waves (rows 4 apart) on different LDS banks. */
-    if (g.epi == EPI_HIDDEN) {   /* pre-activations and activations: direct stores */
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            const int n = n0 + wn * 64 + j * 32 + fr;
-            const float bias = g.bias[z * g.sBias + n];
-#pragma unroll
-            for (int i = 0; i < 2; i++)
-#pragma unroll
-                for (int q = 0; q < 16; q++) {
-                    const int m = m0 + wm * 64 + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                    const int64_t o = (int64_t)m * g.ldc + n;
-                    const float v = acc[i][j][q] + bias;
-                    g.Cf[z * g.sCf + o] = v;
-                    g.Cb[z * g.sCb + o] = (bf16)gelu(v);
-                }
-        }
-        return;
-    }
-    constexpr int S = GT + 8;
-    static_assert(GT * S * sizeof(float) <= sizeof(sm), "fp32 output tile fits the operand LDS");
-    float *cs = reinterpret_cast<float *>(&sm[0][0][0][0]);
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int c = wn * 64 + j * 32 + fr;
-        const float bias = g.bias ? g.bias[z * g.sBias + n0 + c] : 0.0f;
-#pragma unroll
-        for (int i = 0; i < 2; i++)
-#pragma unroll
-            for (int q = 0; q < 16; q++) {
-                const int rr = wm * 64 + i * 32 + 8 * (q >> 2) + 4 * (lane >> 5) + (q & 3);
-                cs[rr * S + c] = acc[i][j][q] + bias;
-            }
-    }
-    __syncthreads();
-    float *dst = g.Cf + z * g.sCf;
-    for (int p = t; p < GT * (GT / 4); p += 256) {
-        const int rr = p / (GT / 4), c = (p % (GT / 4)) * 4;
-        *(f32x4 *)&dst[(int64_t)(m0 + rr) * g.ldc + n0 + c] = *(const f32x4 *)&cs[rr * S + c];
-    }
-}
-
 /* ---- the whole network in one kernel (prediction) ----
  * One workgroup takes 64 inputs (32 where that is enough for every CU to have
  * one) through every layer of one ensemble member: the activations stay in
@@ -342,16 +92,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
  * GELU runs on the vector unit while the other's products run on the matrix
  * cores.
  *
- * The weights are kept a second time in fragment order (k_pack_weights):
- * block (nb, ks) of a layer holds the 64 lanes' 16-byte operands of columns
- * 32 nb .. and k = 16 ks .., so every weight load is one contiguous KB.
+ * The weights are read in fragment order (frag_w below).
  *
- * Tiles are dealt XCD-aware: the hardware hands workgroup b to XCD b % 8, so
- * consecutive tiles of one member go to one XCD, whose L2 then holds that
- * member's 1.7 MB of weights.
+ * Tiles are dealt XCD-aware (xcd_order): consecutive tiles of one member go
+ * to one XCD, whose L2 then holds that member's 1.7 MB of weights.
  *
  * Each output accumulates its k = 0, 16, 32, ... products in that order, as
- * k_gemm does: the same bits.
+ * k_train_rows does: the same bits.
  *
  * Bound: 262,144 inputs and 4 members take 1.94 ms, 930 TFLOP/s, of 0.9 ms
  * the matrix cores need at the 1.95 GHz they run at here.  Timing variants:
@@ -378,22 +125,36 @@ struct MlpArgs {
     int MT, T;                    /* row tiles, row tiles x members */
 };
 
-/* parameters [E][total] -> fragment order; one thread per 16-byte operand */
-__global__ void k_pack_weights(const bf16 *__restrict__ wb, bf16 *__restrict__ wp, const Layout lay, int E) {
-    const int64_t per = (int64_t)lay.total / 8;
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < per * E; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t z = i / per, q = (i % per) * 8;
+/* Fragment order of a matrix operand: 512 elements for 32 rows (or columns)
+ * `r` and 16 contraction indices `c`, lane (r & 31) + 32 ((c >> 3) & 1)
+ * holding the 8 elements c & 7 = 0..7 contiguously: what one lane feeds
+ * v_mfma_f32_32x32x16_bf16 for either operand.  cs: contraction steps (of
+ * 16) of the whole matrix. */
+__host__ __device__ __forceinline__ int64_t frag(int r, int c, int cs) {
+    return ((int64_t)(r >> 5) * cs + (c >> 4)) * 512 + ((r & 31) + 32 * ((c >> 3) & 1)) * 8 + (c & 7);
+}
+
+/* BF16 copies of the weights W_l [out][in], per member at W_l's offset: wp
+ * contracts the inputs (forward), wt the outputs (backward) */
+__global__ void k_pack_weights(const float *__restrict__ w, bf16 *__restrict__ wp, bf16 *__restrict__ wt, const Layout lay, int E) {
+    const int64_t n = (int64_t)lay.total * E;
+    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
+        const int64_t z = i / (int64_t)lay.total, q = i % (int64_t)lay.total;
         int l = 0;
         while (l < NHID && q >= (int64_t)lay.W[l + 1]) l++;
-        const int64_t r = q - (int64_t)lay.W[l];
-        const int K = lay.in[l];
-        if (r >= (int64_t)K * lay.out[l]) continue;   /* biases */
-        const int64_t f = r / 512;                    /* fragment (nb, ks) */
-        const int lane = (int)(r % 512) / 8, KS = K / 16;
-        const int nb = (int)(f / KS), ks = (int)(f % KS);
-        const int64_t src = (int64_t)lay.W[l] + (int64_t)(nb * 32 + (lane & 31)) * K + ks * 16 + 8 * (lane >> 5);
-        *(bf16x8 *)(wp + z * (int64_t)lay.total + q) = *(const bf16x8 *)(wb + z * (int64_t)lay.total + src);
+        const int r = (int)(q - (int64_t)lay.W[l]), in = lay.in[l], out = lay.out[l];
+        if (r >= in * out) continue;   /* biases */
+        const int64_t base = z * (int64_t)lay.total + (int64_t)lay.W[l];
+        wp[base + frag(r / in, r % in, in / 16)] = (bf16)w[i];
+        wt[base + frag(r % in, r / in, out / 16)] = (bf16)w[i];
     }
+}
+
+/* Index of workgroup b of T such that consecutive indices run on one XCD:
+ * the hardware hands workgroup b to XCD b % 8 */
+__device__ __forceinline__ int xcd_order(int b, int T) {
+    const int xcd = b & 7, r = b >> 3, per = T >> 3, rem = T & 7;
+    return xcd < rem ? xcd * (per + 1) + r : rem * (per + 1) + (xcd - rem) * per + r;
 }
 
 /* RB: blocks of 32 rows per workgroup; DEPTH: k-steps of weights in flight
@@ -403,10 +164,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void 
     constexpr int WAVES = 8, JB = 16 / WAVES, ROWS = 32 * RB, KS = HID / 16;
     __shared__ __attribute__((aligned(16))) bf16 act[ROWS][MLDS];
     __shared__ __attribute__((aligned(16))) float bias[BIASES];
-    const int b = (int)blockIdx.x;
-    const int xcd = b & 7, rr = b >> 3;
-    const int per = g.T >> 3, rem = g.T & 7;
-    const int L = xcd < rem ? xcd * (per + 1) + rr : rem * (per + 1) + (xcd - rem) * per + rr;
+    const int L = xcd_order((int)blockIdx.x, g.T);
     const int z = L / g.MT, m0 = (L % g.MT) * ROWS;
     const int t = threadIdx.x, lane = t & 63;
     const int w = __builtin_amdgcn_readfirstlane(t >> 6);
@@ -421,7 +179,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void 
     };
     auto weights = [&](int l, int steps) { return (const bf16x8 *)(wp + g.woff[l]) + (int64_t)(JB * w) * steps * 64 + lane; };
     fetch(weights(0, IN_PAD / 16), 0, IN_PAD / 16, 0);
-    for (int k = t; k < BIASES; k += 64 * WAVES) bias[k] = par[g.boff[k / HID] + k % HID];
+    {
+        float bv[NHID + 1];
+#pragma unroll
+        for (int i = 0; i <= NHID; i++) bv[i] = i < NHID || t < OUT_PAD ? par[g.boff[i] + t] : 0.0f;
+#pragma unroll
+        for (int i = 0; i <= NHID; i++)
+            if (i < NHID || t < OUT_PAD) bias[i * HID + t] = bv[i];
+    }
     for (int k = t; k < ROWS * 4; k += 64 * WAVES) {   /* inputs: 6 features in the first k-step, the rest of it zero */
         const int r = k >> 2, c = (k & 3) * 4;
         bf16x4 v;
@@ -526,107 +291,434 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void 
     }
 }
 
-/* softmax cross-entropy on the 99 bins + weighted squared error on the
- * log-total head; writes dLogits (bf16, /batch) and the summed loss */
-__global__ void k_loss(const float *__restrict__ logits, int64_t sL, const float *__restrict__ y,
-                       const float *__restrict__ tot, int B, float w_tot, bf16 *__restrict__ dlog, int64_t sD,
-                       float *__restrict__ loss) {
-    const int z = blockIdx.y;
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= B) return;
-    const float *L = logits + z * sL + (int64_t)b * OUT_PAD;
-    bf16 *D = dlog + z * sD + (int64_t)b * OUT_PAD;
-    const float *Y = y + (int64_t)b * NBINS;
-    float mx = L[0];
-    for (int k = 1; k < NBINS; k++) mx = fmaxf(mx, L[k]);
-    float s = 0.f;
-    for (int k = 0; k < NBINS; k++) s += __expf(L[k] - mx);
-    const float ls = logf(s) + mx;
-    float ce = 0.f;
-    const float invB = 1.0f / (float)B;
-    for (int k = 0; k < NBINS; k++) {
-        const float p = __expf(L[k] - ls);
-        ce -= Y[k] * (L[k] - ls);
-        D[k] = (bf16)((p - Y[k]) * invB);
-    }
-    const float e = L[NBINS] - tot[b];
-    D[NBINS] = (bf16)(2.0f * w_tot * e * invB);
-    for (int k = OUT; k < OUT_PAD; k++) D[k] = (bf16)0.0f;
-    atomicAdd(&loss[z], (ce + w_tot * e * e) * invB);
-}
+/* ---- training: forward, loss and backward of 16 rows in one kernel ----
+ * One workgroup takes 16 rows of the batch through one member's layers, the
+ * loss and back, the activations (then the gradients) in LDS, the weights
+ * streamed from L2 in fragment order: wp on the way up, wt on the way down.
+ * It leaves what the weight gradients contract over the batch, in fragment
+ * order with the batch as contraction: the layer inputs (xt, ht) and the
+ * gradients of the pre-activations and logits (dt, lt).  The
+ * pre-activations a lane produced come back to that lane (Z, 1 KB per wave
+ * and store).  Here the rows are the first MFMA operand, so a lane holds four
+ * consecutive rows of one column: 8 contiguous bytes of a batch fragment.
+ *
+ * Bound: the latency of the weight stream (2 x 1.7 MB per workgroup, most of
+ * it just written by k_train_weights on other XCDs: 40 to 50 B a clock) and the GELU derivative's vector
+ * work, with one workgroup on half of the CUs (512 rows, 4 members).  16 rows
+ * instead of 32 halve the vector work of a CU for the same stream, and 16
+ * k-steps in flight instead of 8: 62 -> 49 us.  Rounding points and the order
+ * of every sum (products by k, the softmax sum by bin) are those of the
+ * layer-by-layer kernels it replaces: the same gradients bit for bit; the
+ * loss, which those summed with one atomic per row, differs in its last bits.
+ * One step (512 rows, 4 members) was 14 products of 6 to 20 us, loss 15,
+ * column sums 5 x 4.6, Adam 17, gather and packing 9, together 300 us; now
+ * this kernel and k_train_weights, 80 us. */
+constexpr int TR = 16;            /* rows per workgroup: half an MFMA block (its other rows repeat them and are not used) */
+constexpr int TDEPTH = 16;        /* k-steps of weights in flight per wave */
+constexpr int LGS = OUT_PAD + 4;  /* LDS row of the logits */
 
-/* column sums of a bf16 [B][N] matrix -> fp32 [N] (bias gradients), N a
- * multiple of 64.  A workgroup sums 64 columns: 32 row lanes, each of 32
- * threads reading two adjacent columns (one 4-byte load) of every 32nd
- * row, then the 32 partial sums of a column are added in a fixed order, so
- * the result does not depend on timing. */
-constexpr int COLSUM_LANES = 32;
-static_assert(HID % 64 == 0 && OUT_PAD % 64 == 0, "k_colsum sums 64 columns per workgroup");
-__global__ __launch_bounds__(1024) void k_colsum(const bf16 *__restrict__ dz, int64_t sD, int B, int N,
-                                                 float *__restrict__ out, int64_t sO) {
-    __shared__ float part[COLSUM_LANES][64 + 1];
-    const int z = blockIdx.y;
-    const int cp = (int)threadIdx.x & 31;
-    const int rl = (int)threadIdx.x >> 5;
-    const int n0 = (int)blockIdx.x * 64;
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(dz + z * sD + n0) + cp;
-    const int64_t row = N / 2;   /* in 4-byte words */
-    float s0 = 0.f, s1 = 0.f;
-#pragma unroll 4
-    for (int b = rl; b < B; b += COLSUM_LANES) {
-        const uint32_t v = src[(int64_t)b * row];
-        s0 += __builtin_bit_cast(float, v << 16);            /* column n0 + 2 cp */
-        s1 += __builtin_bit_cast(float, v & 0xffff0000u);    /* column n0 + 2 cp + 1 */
-    }
-    part[rl][2 * cp] = s0;
-    part[rl][2 * cp + 1] = s1;
+struct TrainArgs {
+    const float *X, *Y, *T;       /* [rows][6], [rows][99], [rows] */
+    const int32_t *ord;           /* batch row b is row ord[b]; NULL: row b */
+    int B;
+    float w_tot;
+    const bf16 *wp, *wt;
+    const float *w;
+    int64_t sW;                   /* member stride of wp, wt and w */
+    int64_t woff[NHID + 1], boff[NHID + 1];
+    float *Z;                     /* [E][NHID][B / TR][8 waves][4][64 lanes][4] */
+    bf16 *xt, *ht, *dt, *lt;      /* batch fragments: [2], [E][NHID][16], [E][NHID][16], [E][4] x [B / 16][512] */
+    float *loss;                  /* [E] */
+};
+
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k_train_rows(const TrainArgs g) {
+    constexpr int KS = HID / 16;
+    __shared__ __attribute__((aligned(16))) bf16 act[TR][MLDS];
+    __shared__ __attribute__((aligned(16))) float bias[BIASES];
+    __shared__ float lg[TR][LGS], ex[TR][LGS];
+    __shared__ float wloss[8];
+    const int tiles = g.B / TR, L = xcd_order((int)blockIdx.x, (int)gridDim.x);   /* a member's tiles on one or two XCDs */
+    const int tile = L % tiles, z = L / tiles;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 31, hi = lane >> 5;
+    const int cs = g.B / 16;   /* contraction steps of the batch: one per tile */
+    const bf16 *wp = g.wp + z * g.sW, *wt = g.wt + z * g.sW;
+    const float *par = g.w + z * g.sW;
+    auto row_of = [&](int r) { const int b = tile * TR + r; return (int64_t)(g.ord ? g.ord[b] : b); };
+    bf16x8 fb[TDEPTH][2];
+    auto fetch = [&](const bf16x8 *p, int ks, int steps, int u) {
+        fb[u][0] = p[(int64_t)ks * 64];
+        fb[u][1] = p[((int64_t)steps + ks) * 64];
+    };
+    auto up = [&](int l, int steps) { return (const bf16x8 *)(wp + g.woff[l]) + (int64_t)(2 * w) * steps * 64 + lane; };
+    auto down = [&](int l, int steps) { return (const bf16x8 *)(wt + g.woff[l]) + (int64_t)(2 * w) * steps * 64 + lane; };
+    fetch(up(0, IN_PAD / 16), 0, IN_PAD / 16, 0);
+    /* targets of the loss: 32 threads per row, 4 bins each */
+    const int lr = t >> 5, lc = t & 31;
+    const int64_t src = row_of(lr);
+    float y[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) y[i] = lc + 32 * i < NBINS ? g.Y[src * NBINS + lc + 32 * i] : g.T[src];
+    const float x = lc < 6 ? g.X[src * 6 + lc] : 0.0f;
+    float bv[NHID + 1];
+#pragma unroll
+    for (int i = 0; i <= NHID; i++) bv[i] = i < NHID || t < OUT_PAD ? par[g.boff[i] + t] : 0.0f;
+    if (lc < 16) act[lr][lc] = (bf16)x;   /* 6 features, zero up to 16 (one k-step; the others only add zeros) */
+#pragma unroll
+    for (int i = 0; i <= NHID; i++)
+        if (i < NHID || t < OUT_PAD) bias[i * HID + t] = bv[i];
     __syncthreads();
-    if (threadIdx.x < 64) {
-        float s = 0.f;
-        for (int k = 0; k < COLSUM_LANES; k++) s += part[k][threadIdx.x];
-        out[z * sO + n0 + (int)threadIdx.x] = s;
+    if (z == 0 && w < 2) {   /* the inputs' batch fragments: 2 column blocks */
+        bf16x8 v;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = w == 0 && fr < 16 ? act[8 * hi + e][fr] : (bf16)0.0f;
+        *(bf16x8 *)(g.xt + ((int64_t)w * cs + tile) * 512 + lane * 8) = v;
+    }
+    f32x16 acc[2];
+    bf16x8 fa[2];
+    auto rows = [&](int ks, int v) { fa[v] = *(const bf16x8 *)&act[fr % TR][ks * 16 + 8 * hi]; };
+    auto step = [&](int u, int v) {
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[v], fb[u][j], acc[j], 0, 0, 0);
+    };
+    /* acc = act x operand over 32 k-steps, the first TDEPTH already in fb */
+    auto product = [&](const bf16x8 *p) {
+        acc[0] = f32x16{};
+        acc[1] = f32x16{};
+        rows(0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks + 1 < KS) rows(ks + 1, (ks + 1) & 1);
+            step(ks % TDEPTH, ks & 1);
+            if (ks + TDEPTH < KS) fetch(p, ks + TDEPTH, KS, ks % TDEPTH);
+        }
+    };
+    auto prefetch = [&](const bf16x8 *p, int steps) {
+#pragma unroll
+        for (int u = 0; u < TDEPTH; u++) fetch(p, u, steps, u);
+    };
+    /* accumulator r < 8 of lane l of block j is row 8 (r/4) + 4 (l/32) + r%4,
+     * column 64 w + 32 j + l%32 */
+    auto zpos = [&](int l) { return (f32x4 *)g.Z + ((((int64_t)z * NHID + l) * tiles + tile) * 8 + w) * 256 + lane; };
+    /* four rows of column block cb of a batch fragment array */
+    auto put = [&](bf16 *base, int cb, int q, bf16x4 v) {
+        *(bf16x4 *)(base + ((int64_t)cb * cs + tile) * 512 + (fr + 32 * q) * 8 + 4 * hi) = v;
+    };
+    auto to_act = [&](const bf16x4 (&v)[2][2]) {
+        __syncthreads();   /* every wave has read this layer's rows */
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int q = 0; q < 2; q++)
+#pragma unroll
+                for (int k = 0; k < 4; k++) act[8 * q + 4 * hi + k][64 * w + 32 * j + fr] = v[j][q][k];
+        __syncthreads();
+    };
+    auto activate = [&](int l) {
+        bf16x4 v[2][2];
+        f32x4 *zp = zpos(l);
+        bf16 *ht = g.ht + ((int64_t)z * NHID + l) * g.B * HID;
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            const float b = bias[l * HID + 64 * w + 32 * j + fr];
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+                f32x4 zz;
+#pragma unroll
+                for (int k = 0; k < 4; k++) { zz[k] = acc[j][4 * q + k] + b; v[j][q][k] = (bf16)gelu(zz[k]); }
+                zp[(j * 2 + q) * 64] = zz;
+                put(ht, 2 * w + j, q, v[j][q]);
+            }
+        }
+        to_act(v);
+    };
+    acc[0] = f32x16{};
+    acc[1] = f32x16{};
+    rows(0, 0);
+    step(0, 0);
+    prefetch(up(1, KS), KS);
+    activate(0);
+    for (int l = 1; l < NHID; l++) {
+        product(up(l, KS));
+        if (l + 1 < NHID) {
+            prefetch(up(l + 1, KS), KS);
+        } else if (w < 4) {   /* the output layer's column block w, whole */
+            const bf16x8 *po = (const bf16x8 *)(wp + g.woff[NHID]) + (int64_t)w * KS * 64 + lane;
+#pragma unroll
+            for (int ks = 0; ks < KS; ks++) fb[ks / 2][ks % 2] = po[ks * 64];
+        }
+        activate(l);
+    }
+    static_assert(KS == 2 * TDEPTH, "an output column block fills the operand registers");
+    if (w < 4) {   /* logits: column block w */
+        f32x16 o = f32x16{};
+        rows(0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++) {
+            if (ks + 1 < KS) rows(ks + 1, (ks + 1) & 1);
+            o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[ks & 1], fb[ks / 2][ks % 2], o, 0, 0, 0);
+        }
+        const float b = bias[NHID * HID + 32 * w + fr];
+#pragma unroll
+        for (int r = 0; r < 8; r++) lg[8 * (r >> 2) + 4 * hi + (r & 3)][32 * w + fr] = o[r] + b;
+    }
+    /* the first backward product's operands arrive during the loss */
+    constexpr int OS = OUT_PAD / 16;
+    static_assert(OS <= TDEPTH, "the output layer's contraction is prefetched whole");
+#pragma unroll
+    for (int u = 0; u < OS; u++) fetch(down(NHID, OS), u, OS, u);
+    __syncthreads();
+    {   /* softmax cross-entropy + w_tot (log-total - target)^2: 32 threads per row */
+        float lv[4], mx = lg[lr][0];
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            lv[i] = lg[lr][lc + 32 * i];
+            if (lc + 32 * i < NBINS) mx = fmaxf(mx, lv[i]);
+        }
+#pragma unroll
+        for (int off = 16; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+            if (lc + 32 * i < NBINS) ex[lr][lc + 32 * i] = __expf(lv[i] - mx);
+        __syncthreads();
+        float ls = 0.0f;
+        if (lc == 0) {   /* the sum in bin order */
+            float sum = 0.0f;
+#pragma unroll
+            for (int k = 0; k < NBINS; k++) sum += ex[lr][k];
+            ls = logf(sum) + mx;
+        }
+        ls = __shfl(ls, lane & 32);
+        const float invB = 1.0f / (float)g.B;
+        float ce = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const int k = lc + 32 * i;
+            float d = 0.0f;
+            if (k < NBINS) {
+                const float p = __expf(lv[i] - ls);
+                ce -= y[i] * (lv[i] - ls);
+                d = (p - y[i]) * invB;
+            } else if (k == NBINS) {   /* y holds the log-total target there */
+                const float e = lv[i] - y[i];
+                ce += g.w_tot * e * e;
+                d = 2.0f * g.w_tot * e * invB;
+            }
+            act[lr][k] = (bf16)d;   /* the logits' inputs have been read by all waves */
+        }
+        ce *= invB;
+#pragma unroll
+        for (int off = 32; off > 0; off >>= 1) ce += __shfl_xor(ce, off);
+        if (lane == 0) wloss[w] = ce;
+    }
+    __syncthreads();
+    if (t == 0) {
+        float sum = 0.0f;
+        for (int k = 0; k < 8; k++) sum += wloss[k];
+        atomicAdd(&g.loss[z], sum);
+    }
+    if (w < 4) {   /* the logit gradients' batch fragments: column block w */
+        bf16x8 v;
+#pragma unroll
+        for (int e = 0; e < 8; e++) v[e] = act[8 * hi + e][w * 32 + fr];
+        *(bf16x8 *)(g.lt + (((int64_t)z * 4 + w) * cs + tile) * 512 + lane * 8) = v;
+    }
+    /* gradient of layer l's pre-activation from acc = dY W_(l+1) */
+    auto back = [&](int l, const f32x4 (&zz)[4]) {
+        bf16x4 v[2][2];
+        bf16 *dt = g.dt + ((int64_t)z * NHID + l) * g.B * HID;
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+            for (int q = 0; q < 2; q++) {
+#pragma unroll
+                for (int k = 0; k < 4; k++) v[j][q][k] = (bf16)(acc[j][4 * q + k] * gelu_grad(zz[j * 2 + q][k]));
+                put(dt, 2 * w + j, q, v[j][q]);
+            }
+        if (l > 0) to_act(v);
+    };
+    f32x4 zz[4];
+    auto load_z = [&](int l) {
+        const f32x4 *zp = zpos(l);
+#pragma unroll
+        for (int k = 0; k < 4; k++) zz[k] = zp[k * 64];
+    };
+    load_z(NHID - 1);
+    acc[0] = f32x16{};
+    acc[1] = f32x16{};
+#pragma unroll
+    for (int ks = 0; ks < OS; ks++) {
+        rows(ks, 0);
+        step(ks, 0);
+    }
+    prefetch(down(NHID - 1, KS), KS);
+    back(NHID - 1, zz);
+    for (int l = NHID - 1; l > 0; l--) {
+        load_z(l - 1);
+        product(down(l, KS));
+        if (l > 1) prefetch(down(l - 1, KS), KS);
+        back(l - 1, zz);
     }
 }
 
-/* Adam on fp32 master weights; refreshes the bf16 copy */
-__global__ void k_adam(float *__restrict__ w, bf16 *__restrict__ wb, const float *__restrict__ gr,
-                       float *__restrict__ m, float *__restrict__ v, int64_t n, float lr, float b1, float b2,
-                       float eps, float c1, float c2) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const float g = gr[i];
-        const float mi = b1 * m[i] + (1.0f - b1) * g;
-        const float vi = b2 * v[i] + (1.0f - b2) * g * g;
-        m[i] = mi;
-        v[i] = vi;
-        const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        w[i] = wi;
-        wb[i] = (bf16)wi;
+/* ---- training: weight and bias gradients of every layer and Adam ----
+ * dW_l = dY_l^T X_l contracts the batch: both operands are k_train_rows'
+ * batch fragments, loaded straight into the registers of the matrix cores.
+ * A workgroup of 4 waves covers 128 x 128 weights of one layer and member
+ * (each wave 64 x 64), and the accumulators go through Adam where they are
+ * (UPDATE), which also refreshes the two BF16 copies, or into the gradient
+ * array.  The waves over a layer's first input columns also sum the gradient's
+ * rows (the bias gradient) from the same fragments: 32 sums over every 32nd
+ * row, then those in order.
+ * Bound: Adam's 32 B per parameter (110 MB at 4 members: 18 us at 6 TB/s) after
+ * 8 us of products: 31 us; 51 before a block's loads were issued together. */
+struct WeightArgs {
+    const bf16 *xt, *ht, *dt, *lt;
+    int B;
+    float *w, *m, *v, *gr;
+    bf16 *wp, *wt;
+    int64_t sW;
+    int64_t woff[NHID + 1], boff[NHID + 1];
+    float lr, b1, b2, eps, c1, c2;
+};
+
+constexpr int WBLOCKS = 3 * 16 + 4 + 4;   /* 128 x 128 blocks of a member: layers 1..3, 4, 0 */
+
+template <bool UPDATE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_train_weights(const WeightArgs g) {
+    __shared__ __attribute__((aligned(16))) bf16 sh[4][64][64 + 8];
+    const int L = xcd_order((int)blockIdx.x, (int)gridDim.x);
+    const int z = L / WBLOCKS, blk = L % WBLOCKS;
+    const int t = threadIdx.x, lane = t & 63;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int fr = lane & 31, hi = lane >> 5;
+    int l, bo, bi;
+    if (blk < 48) { l = 1 + blk / 16; bo = blk % 16 / 4; bi = blk % 4; }
+    else if (blk < 52) { l = NHID; bo = 0; bi = blk - 48; }
+    else { l = 0; bo = blk - 52; bi = 0; }
+    const int o0 = bo * 128 + (w >> 1) * 64, i0 = bi * 128 + (w & 1) * 64;
+    const int in = l == 0 ? IN_PAD : HID, out = l == NHID ? OUT_PAD : HID;
+    if (i0 >= in) return;
+    const int cs = g.B / 16;
+    const bf16 *dy = l == NHID ? g.lt + (int64_t)z * 4 * cs * 512 : g.dt + ((int64_t)z * NHID + l) * g.B * HID;
+    const bf16 *xx = l == 0 ? g.xt : g.ht + ((int64_t)z * NHID + l - 1) * g.B * HID;
+    const bf16x8 *pa = (const bf16x8 *)dy + (int64_t)(o0 / 32) * cs * 64 + lane;
+    const bf16x8 *pb = (const bf16x8 *)xx + (int64_t)(i0 / 32) * cs * 64 + lane;
+    constexpr int D = 4;
+    bf16x8 fa[D][2], fb[D][2];
+    auto fetch = [&](int ks, int u) {
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            fa[u][k] = pa[((int64_t)k * cs + ks) * 64];
+            fb[u][k] = pb[((int64_t)k * cs + ks) * 64];
+        }
+    };
+    f32x16 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) acc[a][b] = f32x16{};
+    /* sums[a][s][e]: rows 16 s + 8 hi + e modulo 32 of column o0 + 32 a + fr */
+    const bool bias_sums = i0 == 0;
+    float sums[2][2][8] = {};
+    auto step = [&](int u) {
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u][a], fb[u][b], acc[a][b], 0, 0, 0);
+        if (bias_sums) {
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) sums[a][u & 1][e] += (float)fa[u][a][e];
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < D; u++) fetch(u, u);   /* B is a multiple of 64: at least D steps */
+    for (int ks = 0; ks + D < cs; ks += D) {
+#pragma unroll
+        for (int u = 0; u < D; u++) {
+            step(u);
+            fetch(ks + D + u, u);
+        }
     }
-}
-
-__global__ void k_to_bf16(const float *__restrict__ in, bf16 *__restrict__ out, int64_t n) {
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = (bf16)in[i];
-}
-
-/* rows ord[0..B) of the staged training set -> the batch buffers */
-__global__ void k_gather(const float *__restrict__ X, const float *__restrict__ Y, const float *__restrict__ T,
-                         const int32_t *__restrict__ ord, int B, float *__restrict__ x, float *__restrict__ y,
-                         float *__restrict__ t) {
-    const int b = blockIdx.x;
-    const int64_t src = ord[b];
-    for (int k = threadIdx.x; k < NBINS; k += blockDim.x) y[(int64_t)b * NBINS + k] = Y[src * NBINS + k];
-    if (threadIdx.x < 6) x[(int64_t)b * 6 + threadIdx.x] = X[src * 6 + threadIdx.x];
-    if (threadIdx.x == 0) t[b] = T[src];
-}
-
-/* inputs [nvalid][6] fp32 -> [B][64] bf16, zero padded (columns past nin,
- * rows past nvalid) */
-__global__ void k_pack_inputs(const float *__restrict__ x, int B, int nvalid, int nin, bf16 *__restrict__ out) {
-    const int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (i >= (int64_t)B * IN_PAD) return;
-    const int b = (int)(i / IN_PAD), k = (int)(i % IN_PAD);
-    out[i] = (bf16)(k < nin && b < nvalid ? x[(int64_t)b * nin + k] : 0.0f);
+#pragma unroll
+    for (int u = 0; u < D; u++) step(u);
+    const int64_t base = z * g.sW;
+    auto adam = [&](float &w, float &m, float &v, float gr) {
+        m = g.b1 * m + (1.0f - g.b1) * gr;
+        v = g.b2 * v + (1.0f - g.b2) * gr * gr;
+        w = w - g.lr * (m / g.c1) / (sqrtf(v / g.c2) + g.eps);
+    };
+    if (bias_sums) {
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            float s = 0.0f;   /* rows 0..7 in the lower half, 8..15 in the upper, 16..23, 24..31 */
+#pragma unroll
+            for (int part = 0; part < 4; part++) {
+                float x = s;
+#pragma unroll
+                for (int e = 0; e < 8; e++) x += sums[a][part >> 1][e];
+                s = __shfl(x, fr + 32 * (part & 1));
+            }
+            const int64_t i = base + g.boff[l] + o0 + 32 * a + fr;
+            if (hi == 0) {
+                if (UPDATE) adam(g.w[i], g.m[i], g.v[i], s);
+                else g.gr[i] = s;
+            }
+        }
+    }
+    /* accumulator r of lane l of block (a, b): weight row o0 + 32 a + 8 (r/4)
+     * + 4 (l/32) + r%4, column i0 + 32 b + l%32.  A block's 48 loads are issued
+     * together, ahead of its 48 stores. */
+#pragma unroll
+    for (int a = 0; a < 2; a++)
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            const int i = i0 + 32 * b + fr;
+            const int64_t at = base + g.woff[l] + (int64_t)(o0 + 32 * a + 4 * hi) * in + i;
+            if (UPDATE) {
+                float wv[16], mv[16], vv[16];
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t p = at + (int64_t)(8 * (r >> 2) + (r & 3)) * in;
+                    wv[r] = g.w[p];
+                    mv[r] = g.m[p];
+                    vv[r] = g.v[p];
+                }
+#pragma unroll
+                for (int r = 0; r < 16; r++) adam(wv[r], mv[r], vv[r], acc[a][b][r]);
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const int64_t p = at + (int64_t)(8 * (r >> 2) + (r & 3)) * in;
+                    g.w[p] = wv[r];
+                    g.m[p] = mv[r];
+                    g.v[p] = vv[r];
+                }
+#pragma unroll
+                for (int q = 0; q < 4; q++) {
+                    const int ob = 32 * a + 8 * q + 4 * hi;
+                    bf16x4 v;
+#pragma unroll
+                    for (int k = 0; k < 4; k++) {
+                        v[k] = (bf16)wv[4 * q + k];
+                        sh[w][ob + k][32 * b + fr] = v[k];
+                    }
+                    *(bf16x4 *)(g.wt + base + g.woff[l] + frag(i, o0 + ob, out / 16)) = v;
+                }
+            } else {
+#pragma unroll
+                for (int r = 0; r < 16; r++) g.gr[at + (int64_t)(8 * (r >> 2) + (r & 3)) * in] = acc[a][b][r];
+            }
+        }
+    if (UPDATE) {   /* wp's pieces of 8 inputs, through this wave's LDS tile */
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int ol = (lane & 31) + 32 * (k & 1), il = 16 * (k >> 1) + 8 * hi;
+            *(bf16x8 *)(g.wp + base + g.woff[l] + frag(o0 + ol, i0 + il, in / 16)) = *(const bf16x8 *)&sh[w][ol][il];
+        }
+    }
 }
 
 /* ensemble statistics of the predictions: per-model softmax, mean SFS,
@@ -690,16 +782,14 @@ struct gf_sg_model {
     OwnedStream st;   /* before the buffers: they are released while it is alive */
     OwnedStream cst;  /* prediction read-back, beside the next batch's compute on st */
     DevBuf<float> w, g, m, v;       /* [E][total] */
-    DevBuf<bf16> wb;
-    DevBuf<bf16> wp;                /* weights in fragment order (prediction) */
-    bool wp_stale = true;           /* the weights have changed since wp was written */
-    DevBuf<bf16> x;                 /* [B][64] */
-    DevBuf<float> Z;                /* [E][NHID][B][512] */
-    DevBuf<bf16> H;                 /* [E][NHID][B][512] */
+    DevBuf<bf16> wp, wt;            /* BF16 weights in fragment order */
+    /* training, Bmax rows */
+    DevBuf<float> Z;
+    DevBuf<bf16> xt, ht, dt, lt;
+    DevBuf<float> loss;
+    /* prediction */
     DevBuf<float> logits;           /* [E][B][128] */
-    DevBuf<bf16> dlog;              /* [E][B][128] */
-    DevBuf<bf16> dz0, dz1;          /* [E][B][512] */
-    DevBuf<float> y, tot, loss, xin;
+    DevBuf<float> xin;
     DevBuf<float> pout;             /* two batches' prediction outputs */
     int64_t step = 0;
     float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
@@ -708,40 +798,28 @@ struct gf_sg_model {
 namespace gf {
 namespace sg {
 
-static int gemm(gf_sg_model &S, GemmArgs a) {
-    if (a.M % TILE || a.N % TILE || a.K % KSTEP) { set_error("surrogate gemm: shape not a multiple of the tile"); return GF_ERR_ARG; }
-    const bool nt = !a.a_km && a.b_nk && (a.epi == EPI_HIDDEN || a.epi == EPI_OUTPUT);
-    if (nt && a.M >= 4096 && a.M % GT == 0 && a.N % GT == 0 && a.K % GK == 0) {
-        const int MT = a.M / GT, NT = a.N / GT, T = MT * NT * S.E;
-        hipLaunchKernelGGL(k_gemm_nt, dim3(T), dim3(256), 0, S.st, a, MT, NT, T);
-    } else {
-        hipLaunchKernelGGL(k_gemm, dim3(a.N / TILE, a.M / TILE, S.E), dim3(256), 0, S.st, a);
-    }
-    GF_HIP(hipGetLastError());
+static int ensure_batch(gf_sg_model &S, int B) {
+    if (B <= S.Bmax) return GF_OK;
+    const size_t E = (size_t)S.E, act = E * NHID * (size_t)B * HID;
+    GF_TRY(S.Z.alloc(act));
+    GF_TRY(S.ht.alloc(act));
+    GF_TRY(S.dt.alloc(act));
+    GF_TRY(S.xt.alloc((size_t)B * IN_PAD));
+    GF_TRY(S.lt.alloc(E * B * OUT_PAD));
+    S.Bmax = B;
     return GF_OK;
 }
 
-static int ensure_batch(gf_sg_model &S, int B) {
-    if (B <= S.Bmax) return GF_OK;
-    const int E = S.E;
-    GF_TRY(S.x.alloc((size_t)B * IN_PAD));
-    GF_TRY(S.Z.alloc((size_t)E * NHID * B * HID));
-    GF_TRY(S.H.alloc((size_t)E * NHID * B * HID));
-    GF_TRY(S.logits.alloc((size_t)E * B * OUT_PAD));
-    GF_TRY(S.dlog.alloc((size_t)E * B * OUT_PAD));
-    GF_TRY(S.dz0.alloc((size_t)E * B * HID));
-    GF_TRY(S.dz1.alloc((size_t)E * B * HID));
-    GF_TRY(S.y.alloc((size_t)B * NBINS));
-    GF_TRY(S.tot.alloc(B));
-    GF_TRY(S.xin.alloc((size_t)B * 6));
-    S.Bmax = B;
+/* both BF16 copies from the master weights */
+static int pack_weights(gf_sg_model &S) {
+    hipLaunchKernelGGL(k_pack_weights, dim3(2048), dim3(256), 0, S.st, S.w.p, S.wp.p, S.wt.p, S.lay, S.E);
+    GF_HIP(hipGetLastError());
     return GF_OK;
 }
 
 /* buffers of prediction batches of up to B rows; host: also two batches'
  * inputs and outputs */
 static int ensure_predict(gf_sg_model &S, int B, bool host) {
-    GF_TRY(S.wp.alloc((size_t)S.E * S.lay.total));
     GF_TRY(S.logits.alloc((size_t)S.E * B * OUT_PAD));
     if (host) {
         GF_TRY(S.xin.alloc((size_t)B * 6));
@@ -754,11 +832,6 @@ static int ensure_predict(gf_sg_model &S, int B, bool host) {
  * rounded up to MR rows: S.logits [E][B][128] */
 static int predict_logits(gf_sg_model &S, const float *x, int n, int B) {
     const Layout &L = S.lay;
-    if (S.wp_stale) {
-        hipLaunchKernelGGL(k_pack_weights, dim3(1024), dim3(256), 0, S.st, S.wb.p, S.wp.p, L, S.E);
-        GF_HIP(hipGetLastError());
-        S.wp_stale = false;
-    }
     MlpArgs a{};
     a.x = x;
     a.n = n;
@@ -791,91 +864,53 @@ static int predict_stats(gf_sg_model &S, int cnt, float *sfs, float *tot, float 
     return GF_OK;
 }
 
-/* forward pass of the whole ensemble on S.x (B rows) for training: also
- * stores the hidden layers' pre-activations Z (the backward pass reads them) */
-static int forward(gf_sg_model &S, int B) {
-    const Layout &L = S.lay;
-    const int64_t sW = (int64_t)L.total;
-    const int64_t sAct = (int64_t)NHID * B * HID;
-    for (int l = 0; l <= NHID; l++) {
-        GemmArgs a{};
-        if (l == 0) { a.A = S.x.p; a.lda = IN_PAD; a.sA = 0; }
-        else { a.A = S.H.p + (int64_t)(l - 1) * B * HID; a.lda = HID; a.sA = sAct; }
-        a.a_km = 0;
-        a.B = S.wb.p + L.W[l]; a.ldb = L.in[l]; a.b_nk = 1; a.sB = sW;
-        a.M = B; a.N = L.out[l]; a.K = L.in[l];
-        a.bias = S.w.p + L.b[l]; a.sBias = sW;
-        if (l < NHID) {
-            a.epi = EPI_HIDDEN;
-            a.Cf = S.Z.p + (int64_t)l * B * HID; a.sCf = sAct; a.ldc = HID;
-            a.Cb = S.H.p + (int64_t)l * B * HID; a.sCb = sAct;
-        } else {
-            a.epi = EPI_OUTPUT;
-            a.Cf = S.logits.p; a.sCf = (int64_t)B * OUT_PAD; a.ldc = OUT_PAD;
-        }
-        GF_TRY(gemm(S, a));
-    }
+/* n rows of host inputs and targets on the device (the caller synchronises
+ * the stream before it returns) */
+static int stage_rows(gf_sg_model &S, const float *x, const float *y, const float *t, int n, DevBuf<float> &dx,
+                      DevBuf<float> &dy, DevBuf<float> &dt) {
+    GF_TRY(dx.alloc((size_t)n * 6));
+    GF_TRY(dy.alloc((size_t)n * NBINS));
+    GF_TRY(dt.alloc(n));
+    GF_HIP(hipMemcpyAsync(dx.p, x, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, S.st));
+    GF_HIP(hipMemcpyAsync(dy.p, y, (size_t)n * NBINS * sizeof(float), hipMemcpyHostToDevice, S.st));
+    GF_HIP(hipMemcpyAsync(dt.p, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice, S.st));
     return GF_OK;
 }
 
-/* loss + backward + Adam for one batch already in S.x / S.y / S.tot */
-static int train_step(gf_sg_model &S, int B, float lr, float w_tot, bool update) {
+/* forward, backward and (update) Adam for a batch of B rows of X, Y, T
+ * (device): rows ord[0..B), or 0..B where ord is NULL */
+static int train_step(gf_sg_model &S, const float *X, const float *Y, const float *T, const int32_t *ord, int B, float lr,
+                      float w_tot, bool update) {
     const Layout &L = S.lay;
-    const int E = S.E;
-    const int64_t sW = (int64_t)L.total;
-    const int64_t sAct = (int64_t)NHID * B * HID;
-    GF_TRY(forward(S, B));
-    hipLaunchKernelGGL(k_loss, dim3((B + 127) / 128, E), dim3(128), 0, S.st, S.logits.p, (int64_t)B * OUT_PAD,
-                       S.y.p, S.tot.p, B, w_tot, S.dlog.p, (int64_t)B * OUT_PAD, S.loss.p);
-    GF_HIP(hipGetLastError());
-    /* dY of layer l lives in `dcur` ([E][B][out_l] bf16) */
-    const bf16 *dcur = S.dlog.p;
-    int64_t sD = (int64_t)B * OUT_PAD;
-    for (int l = NHID; l >= 0; l--) {
-        const int O = L.out[l], I = L.in[l];
-        /* dW_l = dY^T X_l : M = O, N = I, K = B */
-        GemmArgs a{};
-        a.A = dcur; a.lda = O; a.a_km = 1; a.sA = sD;
-        if (l == 0) { a.B = S.x.p; a.ldb = IN_PAD; a.sB = 0; }
-        else { a.B = S.H.p + (int64_t)(l - 1) * B * HID; a.ldb = HID; a.sB = sAct; }
-        a.b_nk = 0;
-        a.M = O; a.N = I; a.K = B;
-        a.epi = EPI_DW; a.Cf = S.g.p + L.W[l]; a.ldc = I; a.sCf = sW;
-        GF_TRY(gemm(S, a));
-        hipLaunchKernelGGL(k_colsum, dim3(O / 64, E), dim3(32 * COLSUM_LANES), 0, S.st, dcur, sD, B, O,
-                           S.g.p + L.b[l], sW);
-        GF_HIP(hipGetLastError());
-        if (l == 0) break;
-        /* dZ_(l-1) = (dY W_l) * gelu'(Z_(l-1)) : M = B, N = I, K = O */
-        bf16 *dnext = (dcur == S.dz0.p) ? S.dz1.p : S.dz0.p;
-        GemmArgs b{};
-        b.A = dcur; b.lda = O; b.a_km = 0; b.sA = sD;
-        b.B = S.wb.p + L.W[l]; b.ldb = I; b.b_nk = 0; b.sB = sW;
-        b.M = B; b.N = I; b.K = O;
-        b.epi = EPI_DX; b.Cb = dnext; b.sCb = (int64_t)B * HID; b.ldc = HID;
-        b.Zprev = S.Z.p + (int64_t)(l - 1) * B * HID; b.sZ = sAct;
-        GF_TRY(gemm(S, b));
-        dcur = dnext;
-        sD = (int64_t)B * HID;
+    TrainArgs a{};
+    a.X = X; a.Y = Y; a.T = T; a.ord = ord;
+    a.B = B;
+    a.w_tot = w_tot;
+    a.wp = S.wp.p; a.wt = S.wt.p; a.w = S.w.p;
+    a.Z = S.Z.p;
+    a.xt = S.xt.p; a.ht = S.ht.p; a.dt = S.dt.p; a.lt = S.lt.p;
+    a.loss = S.loss.p;
+    WeightArgs b{};
+    b.xt = S.xt.p; b.ht = S.ht.p; b.dt = S.dt.p; b.lt = S.lt.p;
+    b.B = B;
+    b.w = S.w.p; b.m = S.m.p; b.v = S.v.p; b.gr = S.g.p;
+    b.wp = S.wp.p; b.wt = S.wt.p;
+    a.sW = b.sW = (int64_t)L.total;
+    for (int l = 0; l <= NHID; l++) {
+        a.woff[l] = b.woff[l] = (int64_t)L.W[l];
+        a.boff[l] = b.boff[l] = (int64_t)L.b[l];
     }
+    hipLaunchKernelGGL(k_train_rows, dim3(B / TR * S.E), dim3(512), 0, S.st, a);
+    GF_HIP(hipGetLastError());
     if (update) {
         S.step++;
-        const float c1 = 1.0f - std::pow(S.b1, (float)S.step);
-        const float c2 = 1.0f - std::pow(S.b2, (float)S.step);
-        const int64_t n = (int64_t)E * L.total;
-        S.wp_stale = true;
-        hipLaunchKernelGGL(k_adam, dim3(1024), dim3(256), 0, S.st, S.w.p, S.wb.p, S.g.p, S.m.p, S.v.p, n, lr, S.b1,
-                           S.b2, S.eps, c1, c2);
-        GF_HIP(hipGetLastError());
+        b.lr = lr; b.b1 = S.b1; b.b2 = S.b2; b.eps = S.eps;
+        b.c1 = 1.0f - std::pow(S.b1, (float)S.step);
+        b.c2 = 1.0f - std::pow(S.b2, (float)S.step);
+        hipLaunchKernelGGL(k_train_weights<true>, dim3(WBLOCKS * S.E), dim3(256), 0, S.st, b);
+    } else {
+        hipLaunchKernelGGL(k_train_weights<false>, dim3(WBLOCKS * S.E), dim3(256), 0, S.st, b);
     }
-    return GF_OK;
-}
-
-static int load_batch(gf_sg_model &S, const float *x, const float *y, const float *t, int B) {
-    GF_HIP(hipMemcpyAsync(S.xin.p, x, (size_t)B * 6 * sizeof(float), hipMemcpyHostToDevice, S.st));
-    if (y) GF_HIP(hipMemcpyAsync(S.y.p, y, (size_t)B * NBINS * sizeof(float), hipMemcpyHostToDevice, S.st));
-    if (t) GF_HIP(hipMemcpyAsync(S.tot.p, t, (size_t)B * sizeof(float), hipMemcpyHostToDevice, S.st));
-    hipLaunchKernelGGL(k_pack_inputs, dim3((B * IN_PAD + 255) / 256), dim3(256), 0, S.st, S.xin.p, B, B, 6, S.x.p);
     GF_HIP(hipGetLastError());
     return GF_OK;
 }
@@ -898,7 +933,8 @@ int32_t gf_sg_create(int32_t ensemble, uint64_t seed, int32_t device, gf_sg_mode
     GF_TRY(S->g.alloc(n));
     GF_TRY(S->m.alloc(n));
     GF_TRY(S->v.alloc(n));
-    GF_TRY(S->wb.alloc(n));
+    GF_TRY(S->wp.alloc(n));
+    GF_TRY(S->wt.alloc(n));
     GF_TRY(S->loss.alloc(S->E));
     /* He-style initialisation from a seeded host generator: W ~ U(-a, a),
      * a = sqrt(6 / fan_in); biases 0; padded input columns and output rows 0 */
@@ -924,8 +960,7 @@ int32_t gf_sg_create(int32_t ensemble, uint64_t seed, int32_t device, gf_sg_mode
     GF_HIP(hipMemcpy(S->w.p, h.data(), n * sizeof(float), hipMemcpyHostToDevice));
     GF_HIP(hipMemset(S->m.p, 0, n * sizeof(float)));
     GF_HIP(hipMemset(S->v.p, 0, n * sizeof(float)));
-    hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, S->st, S->w.p, S->wb.p, (int64_t)n);
-    GF_HIP(hipGetLastError());
+    GF_TRY(pack_weights(*S));
     GF_HIP(hipStreamSynchronize(S->st));
     *out = S.release();
     return GF_OK;
@@ -937,18 +972,14 @@ int32_t gf_sg_num_params(const gf_sg_model *S) { return S ? (int32_t)S->lay.tota
 
 int32_t gf_sg_get_params(gf_sg_model *S, float *out) {
     if (!S || !out) return GF_ERR_ARG;
-    GF_HIP(hipStreamSynchronize(S->st));
-    GF_HIP(hipMemcpy(out, S->w.p, (size_t)S->E * S->lay.total * sizeof(float), hipMemcpyDeviceToHost));
-    return GF_OK;
+    return readback(out, S->w.p, (size_t)S->E * S->lay.total * sizeof(float), S->st);
 }
 
 int32_t gf_sg_set_params(gf_sg_model *S, const float *in) {
     if (!S || !in) return GF_ERR_ARG;
     const size_t n = (size_t)S->E * S->lay.total;
     GF_HIP(hipMemcpy(S->w.p, in, n * sizeof(float), hipMemcpyHostToDevice));
-    S->wp_stale = true;
-    hipLaunchKernelGGL(k_to_bf16, dim3(1024), dim3(256), 0, S->st, S->w.p, S->wb.p, (int64_t)n);
-    GF_HIP(hipGetLastError());
+    GF_TRY(pack_weights(*S));
     GF_HIP(hipStreamSynchronize(S->st));
     return GF_OK;
 }
@@ -957,15 +988,16 @@ int32_t gf_sg_set_params(gf_sg_model *S, const float *in) {
  * gradients [E][total] and per-model loss, for gradient checks */
 int32_t gf_sg_gradients(gf_sg_model *S, const float *x, const float *y, const float *t, int32_t B, float w_tot,
                         float *grad_out, float *loss_out) {
-    if (!S || !x || !y || !t || B <= 0 || B % TILE) { set_error("gf_sg_gradients: invalid arguments"); return GF_ERR_ARG; }
+    if (!S || !x || !y || !t || B <= 0 || B % 64) { set_error("gf_sg_gradients: invalid arguments"); return GF_ERR_ARG; }
     StreamScope scope(S->st);   /* buffers (re)allocated here belong to the model's stream */
     GF_TRY(ensure_batch(*S, B));
+    DevBuf<float> dx, dy, dt;
+    GF_TRY(stage_rows(*S, x, y, t, B, dx, dy, dt));
     GF_HIP(hipMemsetAsync(S->loss.p, 0, S->E * sizeof(float), S->st));
-    GF_TRY(load_batch(*S, x, y, t, B));
-    GF_TRY(train_step(*S, B, 0.0f, w_tot, false));
+    GF_TRY(train_step(*S, dx.p, dy.p, dt.p, nullptr, B, 0.0f, w_tot, false));
+    if (grad_out) GF_TRY(readback(grad_out, S->g.p, (size_t)S->E * S->lay.total * sizeof(float), S->st));
+    if (loss_out) GF_TRY(readback(loss_out, S->loss.p, S->E * sizeof(float), S->st));
     GF_HIP(hipStreamSynchronize(S->st));
-    if (grad_out) GF_HIP(hipMemcpy(grad_out, S->g.p, (size_t)S->E * S->lay.total * sizeof(float), hipMemcpyDeviceToHost));
-    if (loss_out) GF_HIP(hipMemcpy(loss_out, S->loss.p, S->E * sizeof(float), hipMemcpyDeviceToHost));
     return GF_OK;
 }
 
@@ -974,18 +1006,13 @@ int32_t gf_sg_gradients(gf_sg_model *S, const float *x, const float *y, const fl
  * the mean loss per epoch (averaged over models) */
 int32_t gf_sg_train(gf_sg_model *S, const float *x, const float *y, const float *t, int32_t n, int32_t epochs,
                     int32_t B, float lr, float w_tot, const int32_t *order, float *epoch_loss) {
-    if (!S || !x || !y || !t || n < B || B <= 0 || B % TILE || epochs <= 0) { set_error("gf_sg_train: invalid arguments"); return GF_ERR_ARG; }
+    if (!S || !x || !y || !t || n < B || B <= 0 || B % 64 || epochs <= 0) { set_error("gf_sg_train: invalid arguments"); return GF_ERR_ARG; }
     StreamScope scope(S->st);   /* buffers (re)allocated here belong to the model's stream */
     GF_TRY(ensure_batch(*S, B));
     /* stage the whole training set on the device once */
     DevBuf<float> dx, dy, dt;
     DevBuf<int32_t> dord;
-    GF_TRY(dx.alloc((size_t)n * 6));
-    GF_TRY(dy.alloc((size_t)n * NBINS));
-    GF_TRY(dt.alloc(n));
-    GF_HIP(hipMemcpyAsync(dx.p, x, (size_t)n * 6 * sizeof(float), hipMemcpyHostToDevice, S->st));
-    GF_HIP(hipMemcpyAsync(dy.p, y, (size_t)n * NBINS * sizeof(float), hipMemcpyHostToDevice, S->st));
-    GF_HIP(hipMemcpyAsync(dt.p, t, (size_t)n * sizeof(float), hipMemcpyHostToDevice, S->st));
+    GF_TRY(stage_rows(*S, x, y, t, n, dx, dy, dt));
     const int nb = n / B;
     std::vector<float> lossv(S->E);
     if (order) {
@@ -995,17 +1022,11 @@ int32_t gf_sg_train(gf_sg_model *S, const float *x, const float *y, const float 
     for (int e = 0; e < epochs; e++) {
         GF_HIP(hipMemsetAsync(S->loss.p, 0, S->E * sizeof(float), S->st));
         for (int b = 0; b < nb; b++) {
-            if (order) {
-                hipLaunchKernelGGL(k_gather, dim3(B), dim3(128), 0, S->st, dx.p, dy.p, dt.p,
-                                   dord.p + (size_t)e * n + (size_t)b * B, B, S->xin.p, S->y.p, S->tot.p);
-                GF_HIP(hipGetLastError());
-            } else {
-                GF_HIP(hipMemcpyAsync(S->xin.p, dx.p + (size_t)b * B * 6, (size_t)B * 6 * sizeof(float), hipMemcpyDeviceToDevice, S->st));
-                GF_HIP(hipMemcpyAsync(S->y.p, dy.p + (size_t)b * B * NBINS, (size_t)B * NBINS * sizeof(float), hipMemcpyDeviceToDevice, S->st));
-                GF_HIP(hipMemcpyAsync(S->tot.p, dt.p + (size_t)b * B, (size_t)B * sizeof(float), hipMemcpyDeviceToDevice, S->st));
-            }
-            hipLaunchKernelGGL(k_pack_inputs, dim3((B * IN_PAD + 255) / 256), dim3(256), 0, S->st, S->xin.p, B, B, 6, S->x.p);
-            GF_TRY(train_step(*S, B, lr, w_tot, true));
+            if (order)
+                GF_TRY(train_step(*S, dx.p, dy.p, dt.p, dord.p + (size_t)e * n + (size_t)b * B, B, lr, w_tot, true));
+            else
+                GF_TRY(train_step(*S, dx.p + (size_t)b * B * 6, dy.p + (size_t)b * B * NBINS, dt.p + (size_t)b * B, nullptr, B,
+                                  lr, w_tot, true));
         }
         GF_HIP(hipMemcpyAsync(lossv.data(), S->loss.p, S->E * sizeof(float), hipMemcpyDeviceToHost, S->st));
         GF_HIP(hipStreamSynchronize(S->st));
