@@ -74,7 +74,13 @@ int joint_sfs_of_device_rows(const float *d_fa, const float *d_fb, int M, int na
     GF_HIP(hipMemcpyAsync(d_l.p, la.data(), la.size() * sizeof(float), hipMemcpyHostToDevice, st));
     GF_HIP(hipMemcpyAsync(d_l.p + la.size(), lb.data(), lb.size() * sizeof(float), hipMemcpyHostToDevice, st));
     GF_HIP(hipMemsetAsync(d_acc.p, 0, (size_t)B * sizeof(unsigned long long), st));
-    if (M > 0) {
+    if (M > 0 && na <= JW_MAX_N && nb <= JW_MAX_N) {
+        /* at most two workgroups a CU: each adds its bins to the global ones once */
+        const int grid = std::max(1, std::min((int)(((int64_t)M + JW_BATCH * (JW_WG / 64) - 1) / (JW_BATCH * (JW_WG / 64))), 2 * num_cus()));
+        hipLaunchKernelGGL(k_joint_sfs_wave, dim3(grid), dim3(JW_WG), (size_t)B * sizeof(unsigned long long), st, d_fa, d_fb, M,
+                           na, nb, ha, hb, d_l.p, d_l.p + la.size(), d_acc.p);
+        GF_HIP(hipGetLastError());
+    } else if (M > 0) {
         const int batch = std::max(1, std::min(32, JS_LDS_FLOATS / (na + nb + 2)));
         const dim3 grid((unsigned)((M + JS_MUT_PER_WG - 1) / JS_MUT_PER_WG), (unsigned)((B + WG * JS_PER_THREAD - 1) / (WG * JS_PER_THREAD)));
         const size_t lds = (size_t)batch * (na + nb + 2) * sizeof(float);
