@@ -14,21 +14,23 @@
  * the prefix pre_s and the source-tile table src0_s) live in a device
  * array of BSim records.
  *
- * One block (up to 32 generations) is four kernels over every simulation,
+ * One block (up to 32 generations) is two kernels over every simulation,
  * with no host round trip:
- *   k_bt_rows     per simulation: the block's generation rows and new-
- *                 mutation counts; a simulation whose survivors and new
- *                 mutations would not fit its tiles stalls (its state stays)
  *   k_bt_advance  the drift kernel with tile-local compaction
  *                 (migration_selection_drift + add_new_mutations +
  *                 compaction, as k_advance_fused): reads the current
  *                 buffer, writes each tile's survivors packed into the other
  *   k_bt_scan     per simulation: prefix of its tiles' survivor counts (the
- *                 next block's gather table), new slot count, generation
- *   k_bt_status   active / stalled counts and the live mutation-generations
- *                 into pinned host memory
- * The block is captured once in a hipGraph and replayed; the host looks at
- * the status every few replays.  Stalled simulations get larger regions
+ *                 next block's gather table), new slot count, generation;
+ *                 then the next block's generation rows and new-mutation
+ *                 counts (k_bt_rows for a layout's first block); a simulation
+ *                 whose survivors and new mutations would not fit its tiles
+ *                 stalls (its state stays)
+ * GRAPH_BLOCKS blocks are captured in a hipGraph and replayed; every few replays
+ * k_bt_status writes the active / stalled counts and the live mutation-
+ * generations into pinned host memory, where the host reads them.  (A block
+ * of a 64-simulation sweep: rows, advance, scan and status as four kernels
+ * spent 20 us beside the drift, and as much in the gaps between them.)  Stalled simulations get larger regions
  * (the host re-lays out the live ones, densely, into new buffers, which also
  * drops finished simulations once they hold most of the tiles).  Finished
  * simulations are finalised (SFS of n chromosomes, optionally the state)
@@ -71,6 +73,7 @@ struct gf_batch_result {
 namespace gf {
 
 constexpr int BK_MAX = 32;                   /* longest block the autotuner tries */
+constexpr int GRAPH_BLOCKS = 4;              /* blocks per captured graph (15 to 30 us lie between two replays) */
 static float g_region_scale = 1.0f;          /* gf_set_batch_region_scale */
 enum { BS_ACTIVE = 0, BS_DONE = 1, BS_STALLED = 2 };
 
@@ -131,19 +134,27 @@ static __global__ __launch_bounds__(POIS_BUILD) void k_bt_pois(const BSim *__res
     pois_table_entry(threadIdx.x, ConstModel{b.Nc, b.fN, b.newfreq, 0.0f, b.s, b.c1, b.c2, b.neutral, b.mid}, out + blockIdx.x);
 }
 
-/* ---- 1. rows and new-mutation counts of the next block, one thread per simulation ---- */
-static __global__ void k_bt_rows(BSim *__restrict__ sims, BBufs B) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= B.S) return;
+/* Rows and new-mutation counts of simulation s's next block, by one wave:
+ * lane t draws the count of the block's generation t (the counts are
+ * independent; a thread per simulation drew up to 32 in a row, 6 to 10 us a
+ * block), a wave prefix turns them into the rows' cumulative counts. */
+__device__ __forceinline__ void next_rows(BSim *__restrict__ sims, int s, const BBufs &B) {
+    const int lane = threadIdx.x & 63;
     BSim &b = sims[s];
-    b.Kb = 0;
-    b.tiles = 0;
-    if (b.status != BS_ACTIVE || b.g >= b.G) return;
-    const int K = min(*B.K, b.G - b.g);
-    GenRow<1> *rows = B.rows + (size_t)s * BK_MAX;
-    int cum = 0;
-    for (int t = 0; t < K; t++) {
-        const int g = b.g + 1 + t;
+    const bool run = b.status == BS_ACTIVE && b.g < b.G;
+    const int K = run ? min(*B.K, b.G - b.g) : 0;   /* at most BK_MAX = 32 */
+    const int n = lane < K ? new_mutation_count(b.Nc, b.mu, b.L, b.k0, b.k1, b.g + 1 + lane, 0) : 0;
+    int cum = n;
+#pragma unroll
+    for (int off = 1; off < BK_MAX; off <<= 1) {
+        const int y = __shfl_up(cum, off);
+        if (lane >= off) cum += y;
+    }
+    const int total = __shfl(cum, BK_MAX - 1);
+    const int64_t need = (int64_t)b.M + total;
+    const int tiles = (int)((need + WG - 1) / WG);
+    const bool fits = tiles <= b.nt;
+    if (lane < K && fits) {
         GenRow<1> r;
         r.Nc[0] = b.Nc;
         r.fN[0] = b.fN;
@@ -154,23 +165,27 @@ static __global__ void k_bt_rows(BSim *__restrict__ sims, BBufs B) {
         r.c2[0] = b.c2;
         r.mig[0][0] = 1.0f;
         r.newfreq[0] = b.newfreq;
-        r.newcum[0] = cum;
-        cum += new_mutation_count(b.Nc, b.mu, b.L, b.k0, b.k1, g, 0);
+        r.newcum[0] = cum - n;
         r.newcum[1] = cum;
         r.present_mask = b.N > 0 ? 1 : 0;
         r.neutral_mask = b.neutral ? 1 : 0;
-        rows[t] = r;
+        B.rows[(size_t)s * BK_MAX + lane] = r;
     }
-    const int64_t need = (int64_t)b.M + cum;
-    const int tiles = (int)((need + WG - 1) / WG);
-    if (tiles > b.nt) {   /* does not fit its region: wait for the host */
-        b.status = BS_STALLED;
-        b.need = tiles;
-        return;
+    if (lane == 0) {
+        if (run && !fits) {   /* does not fit its region: wait for the host */
+            b.status = BS_STALLED;
+            b.need = tiles;
+        }
+        b.Kb = fits ? K : 0;
+        b.nnew = total;
+        b.tiles = run && fits ? tiles : 0;
     }
-    b.Kb = K;
-    b.nnew = cum;
-    b.tiles = tiles;
+}
+
+/* ---- 1. rows of the first block of a layout (k_bt_scan prepares the following ones), or with another block length ---- */
+static __global__ __launch_bounds__(WG) void k_bt_rows(BSim *__restrict__ sims, const BBufs B) {
+    const int s = (int)blockIdx.x * (WG / 64) + ((int)threadIdx.x >> 6);
+    if (s < B.S) next_rows(sims, s, B);   /* the whole wave */
 }
 
 /* ---- 2. drift + new mutations + tile-local compaction of every simulation's block ----
@@ -297,7 +312,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     if (lane == 0 && live) atomicAdd(&B.live[(blockIdx.x * (WG / 64) + w) & 63], (unsigned long long)live);
 }
 
-/* ---- 3. per simulation: prefix of the block's survivor counts ---- */
+/* ---- 3. per simulation: prefix of the block's survivor counts, then the next block's rows ---- */
 static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims, const BBufs B) {
     const int s = blockIdx.x;
     __shared__ int sh_w[4];
@@ -354,7 +369,10 @@ static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims,
         r.cur = out;
         r.g += Kb;
         if (r.g >= r.G) r.status = BS_DONE;
+        __threadfence_block();
     }
+    __syncthreads();
+    if (w == 0) next_rows(sims, s, B);
 }
 
 /* ---- 4. status for the host: [active, stalled], live mutation-generations ---- */
@@ -633,7 +651,7 @@ struct BatchRun {
         }
         std::vector<int64_t> Minit(S, 0);
         const int ns = (int)segs.size();
-        std::vector<int64_t> scan;
+        std::vector<int64_t> bounds;
         DevBuf<MseSeg> d_segs;
         DevBuf<int64_t> d_offs, d_scan, d_scratch, d_total;
         const unsigned grid = (unsigned)std::max(1, num_cus() * 8);
@@ -656,18 +674,24 @@ struct BatchRun {
             }
             DevBuf<int> d_counts;
             GF_TRY(d_counts.alloc((size_t)coff));
-            GF_TRY(d_scan.alloc((size_t)coff + 1));
+            GF_TRY(d_scan.alloc((size_t)coff));
             GF_TRY(d_total.alloc(1));
             hipLaunchKernelGGL(k_mse_counts, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p, ns, coff,
                                any_sel ? d_area.p : nullptr, d_counts.p);
             GF_HIP(hipGetLastError());
             GF_TRY(scan_counts(d_counts.p, coff, d_scan.p, d_total.p, st, d_scratch));
-            GF_HIP(hipMemcpyAsync(d_scan.p + coff, d_total.p, sizeof(int64_t), hipMemcpyDeviceToDevice, st));
-            scan.resize((size_t)coff + 1);
-            GF_HIP(hipMemcpyAsync(scan.data(), d_scan.p, scan.size() * sizeof(int64_t), hipMemcpyDeviceToHost, st));
+            /* the segments' first offsets and the total (the whole scan is one
+             * entry per frequency class: 131 MB for 8,192 simulations of
+             * 1,000 diploids, 35 ms of copying) */
+            DevBuf<int64_t> d_bounds;
+            GF_TRY(d_bounds.alloc((size_t)ns + 1));
+            hipLaunchKernelGGL(k_seg_bounds, dim3((ns + 256) / 256), dim3(256), 0, st, d_scan.p, d_offs.p, ns, d_total.p, d_bounds.p);
+            GF_HIP(hipGetLastError());
+            bounds.resize((size_t)ns + 1);
+            GF_HIP(hipMemcpyAsync(bounds.data(), d_bounds.p, bounds.size() * sizeof(int64_t), hipMemcpyDeviceToHost, st));
             GF_HIP(hipStreamSynchronize(st));
             for (int k = 0; k < ns; k++) {
-                const int64_t tot = scan[segs[k].class_off + segs[k].Nc - 1] - scan[segs[k].class_off];
+                const int64_t tot = bounds[k + 1] - bounds[k];
                 if (tot > 2000000000LL) { set_error("gf_batch_run: initial mutation count exceeds 2e9"); return GF_ERR_UNSUPPORTED; }
                 Minit[seg_sim[k]] = tot;
             }
@@ -703,11 +727,11 @@ struct BatchRun {
                 const int s = seg_sim[k];
                 segs[k].slot_base = (int64_t)host[s].t0 * WG;
                 segs[k].sim_base = segs[k].slot_base;
-                out_offs[k] = scan[segs[k].class_off];
+                out_offs[k] = bounds[k];
             }
             GF_HIP(hipMemcpyAsync(d_segs.p, segs.data(), ns * sizeof(MseSeg), hipMemcpyHostToDevice, st));
             GF_HIP(hipMemcpyAsync(d_offs.p, out_offs.data(), ns * sizeof(int64_t), hipMemcpyHostToDevice, st));
-            const int64_t total = scan[coff];
+            const int64_t total = bounds[ns];
             if (total > 0)
                 hipLaunchKernelGGL(k_mse_fill<1>, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p, ns, total, d_scan.p,
                                    freq[0].p, (int64_t)freq[0].n, ids[0].p);
@@ -764,24 +788,31 @@ struct BatchRun {
         return B;
     }
 
-    /* one block = rows, advance, scan, status: captured once per layout */
+    /* a block = advance, scan + the next block's rows; captured once per
+     * layout, which starts with the first block's rows */
     int capture() {
         if (exec) { (void)hipGraphExecDestroy(exec); exec = nullptr; }
         if (graph) { (void)hipGraphDestroy(graph); graph = nullptr; }
         const BBufs B = bufs();
         const int grid = std::max(1, std::min<int>((int)ntiles, num_cus() * 8));
         GF_HIP(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-        hipLaunchKernelGGL(k_bt_rows, dim3((S + 127) / 128), dim3(128), 0, st, d_sims.p, B);
-        if (any_counted) hipLaunchKernelGGL(k_bt_advance<true>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
-        if (any_general) hipLaunchKernelGGL(k_bt_advance<false>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
-        hipLaunchKernelGGL(k_bt_scan, dim3(S), dim3(256), 0, st, d_sims.p, B);
-        hipLaunchKernelGGL(k_bt_status, dim3(1), dim3(1024), 0, st, (const BSim *)d_sims.p, B, h_status.p);
+        for (int r = 0; r < GRAPH_BLOCKS; r++) {
+            if (any_counted) hipLaunchKernelGGL(k_bt_advance<true>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
+            if (any_general) hipLaunchKernelGGL(k_bt_advance<false>, dim3(grid), dim3(WG), 0, st, (const BSim *)d_sims.p, B);
+            hipLaunchKernelGGL(k_bt_scan, dim3(S), dim3(256), 0, st, d_sims.p, B);
+        }
         const hipError_t e = hipStreamEndCapture(st, &graph);
         if (e != hipSuccess) {
             set_error(std::string("gf_batch_run: graph capture failed: ") + hipGetErrorString(e));
             return GF_ERR_DEVICE;
         }
         GF_HIP(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
+        return first_rows();
+    }
+
+    int first_rows() {
+        hipLaunchKernelGGL(k_bt_rows, dim3((S + WG / 64 - 1) / (WG / 64)), dim3(WG), 0, st, d_sims.p, bufs());
+        GF_HIP(hipGetLastError());
         return GF_OK;
     }
 
@@ -977,7 +1008,7 @@ struct BatchRun {
         GF_HIP(hipStreamSynchronize(st));
         GF_TRY(capture());
         unsigned long long live_prev = 0;
-        int per_check = 4;
+        int per_check = GRAPH_BLOCKS;   /* a multiple of it */
         /* every replay advances each active simulation by at least one
          * generation unless it stalls, and a stall is resolved at the next
          * check: a bound no progressing batch reaches */
@@ -988,8 +1019,10 @@ struct BatchRun {
                 return GF_ERR_DEVICE;
             }
             GF_HIP(hipEventRecord(w0, st));
-            for (int r = 0; r < per_check; r++) GF_HIP(hipGraphLaunch(exec, st));
+            for (int r = 0; r < per_check; r += GRAPH_BLOCKS) GF_HIP(hipGraphLaunch(exec, st));
             blocks += per_check;
+            hipLaunchKernelGGL(k_bt_status, dim3(1), dim3(1024), 0, st, (const BSim *)d_sims.p, bufs(), h_status.p);
+            GF_HIP(hipGetLastError());
             GF_HIP(hipEventRecord(w1, st));
             GF_HIP(hipEventSynchronize(w1));
             const int active = h_status.p[0], stalled = h_status.p[1];
@@ -1002,15 +1035,16 @@ struct BatchRun {
             } else if (per_check < 32) {
                 per_check *= 2;
             }
+            live_prev = lv;
+            if (active == 0 && stalled == 0) break;
             if (forced <= 0) {
                 const int nextK = BlockTuner::get().next(key, cap, measuring);
                 if (nextK != K) {
                     K = nextK;
                     GF_HIP(hipMemcpyAsync(d_K.p, &K, sizeof(int), hipMemcpyHostToDevice, st));
+                    GF_TRY(first_rows());
                 }
             }
-            live_prev = lv;
-            if (active == 0 && stalled == 0) break;
             if (stalled > 0) {
                 GF_TRY(relayout(K));
                 continue;

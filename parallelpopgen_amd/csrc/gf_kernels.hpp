@@ -441,6 +441,14 @@ static __global__ void k_mse_fill(const MseSeg *__restrict__ segs, const int64_t
     }
 }
 
+/* first slot of every segment, and the total behind the last one */
+static __global__ void k_seg_bounds(const int64_t *__restrict__ class_scan, const int64_t *__restrict__ class_offs, int nseg,
+                                    const int64_t *__restrict__ total, int64_t *__restrict__ bounds) {
+    const int s = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+    if (s < nseg) bounds[s] = class_scan[class_offs[s]];
+    else if (s == nseg) bounds[s] = *total;
+}
+
 /* generic exclusive scan of int32 counts into int64 offsets (three-phase,
  * deterministic): per-block sums, single-block scan of the sums, per-block
  * rescan */
