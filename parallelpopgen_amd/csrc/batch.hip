@@ -441,7 +441,7 @@ static __global__ __launch_bounds__(WG) void k_bt_move(const BMove *__restrict__
 struct BFin {
     int64_t base;          /* first slot of the region */
     const int *pre;        /* fragmented layout (NULL: dense) */
-    const unsigned int *cnt;
+    const int *src0;
     int T, M, cur, tile_first;
     int64_t out_base;      /* first slot of the dense copy */
 };
@@ -452,8 +452,26 @@ static __global__ __launch_bounds__(WG) void k_bt_final(const BFin *__restrict__
                                                         int n, int half_n, const float *__restrict__ lc,
                                                         unsigned long long *__restrict__ acc,
                                                         float *__restrict__ copy_freq, gf_mutid *__restrict__ copy_ids) {
-    __shared__ unsigned long long sh[LDS ? SFS_LDS_BINS : 1];
-    for (int gt = blockIdx.x; gt < ntiles; gt += gridDim.x) {
+    /* consecutive tiles, so that a simulation's sums are cleared and added
+     * once per workgroup and not once per tile */
+    extern __shared__ unsigned long long sh_fin[];   /* LDS: sums, then the table */
+    float *sh_lc = reinterpret_cast<float *>(sh_fin + n + 2);
+    if (LDS)
+        for (int k = threadIdx.x; k < half_n; k += WG) sh_lc[k] = lc[k];
+    __syncthreads();
+    const int per = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x;
+    const int g0 = (int)blockIdx.x * per, g1 = g0 + per < ntiles ? g0 + per : ntiles;
+    const int w = wave_index();
+    int sim = -1;
+    auto flush = [&]() {   /* the sums of simulation `sim` */
+        __syncthreads();
+        if (LDS && sim >= 0) {
+            unsigned long long *out = acc + (size_t)sim * (n + 2);
+            for (int k = threadIdx.x; k < n + 2; k += WG)
+                if (sh_fin[k]) atomicAdd(&out[k], sh_fin[k]);
+        }
+    };
+    for (int gt = g0; gt < g1; gt++) {
         int lo = 0, hi = nfin - 1;
         while (lo < hi) {
             const int mid = (lo + hi + 1) >> 1;
@@ -462,36 +480,31 @@ static __global__ __launch_bounds__(WG) void k_bt_final(const BFin *__restrict__
         const BFin f = fin[lo];
         const int j = gt - f.tile_first;
         unsigned long long *out = acc + (size_t)lo * (n + 2);
-        __syncthreads();
-        if (LDS) {
-            for (int k = threadIdx.x; k < n + 2; k += WG) sh[k] = 0;
-            __syncthreads();
-        }
-        /* slot of this lane and its compacted index */
-        bool has;
-        int ci;
-        if (f.pre) {
-            has = j < f.T && (unsigned int)threadIdx.x < f.cnt[j];
-            ci = has ? f.pre[j] + (int)threadIdx.x : 0;
-        } else {
-            ci = j * WG + (int)threadIdx.x;
-            has = ci < f.M;
-        }
-        if (has) {
-            const int64_t slot = f.base + (int64_t)j * WG + threadIdx.x;
-            const float x = freq[f.cur][slot];
-            sfs_add_mutation<LDS>(x, n, half_n, lc, sh, out);
-            if (copy_freq) {
-                copy_freq[f.out_base + ci] = x;
-                copy_ids[f.out_base + ci] = ids[f.cur][slot];
+        if (lo != sim) {
+            flush();
+            sim = lo;
+            if (LDS) {
+                for (int k = threadIdx.x; k < n + 2; k += WG) sh_fin[k] = 0;   /* each its own words of the flush */
+                __syncthreads();
             }
         }
-        if (LDS) {
-            __syncthreads();
-            for (int k = threadIdx.x; k < n + 2; k += WG)
-                if (sh[k]) atomicAdd(&out[k], sh[k]);
+        /* a lane per compacted index: half of the lanes would idle over the
+         * fragmented tiles of a state full of new mutations */
+        const int li = j * WG + (int)threadIdx.x, first = j * WG + w * 64;
+        int64_t slot = li;
+        if (f.pre && first < f.M) slot = frag_slot(li, first, j, f.src0, f.pre, f.T);
+        if (li < f.M) {
+            slot += f.base;
+            const float x = freq[f.cur][slot];
+            if (LDS) sfs_add_mutation<LDS>(x, n, half_n, sh_lc, sh_fin, out);
+            else sfs_add_mutation<LDS>(x, n, half_n, lc, sh_fin, out);
+            if (copy_freq) {
+                copy_freq[f.out_base + li] = x;
+                copy_ids[f.out_base + li] = ids[f.cur][slot];
+            }
         }
     }
+    flush();
 }
 
 /* ---------------- block-length autotuner ----------------
@@ -827,13 +840,13 @@ struct BatchRun {
             BFin &f = fin[k];
             f.base = (int64_t)b.t0 * WG;
             f.pre = b.T >= 0 ? pre[b.cur].p + b.p0 : nullptr;
-            f.cnt = cnt.p + b.t0;
+            f.src0 = b.T >= 0 ? src0[b.cur].p + b.t0 : nullptr;
             f.T = b.T;
             f.M = b.M;
             f.cur = b.cur;
             f.tile_first = (int)tiles;
             f.out_base = total;
-            tiles += b.T >= 0 ? b.T : (b.M + WG - 1) / WG;
+            tiles += (b.M + WG - 1) / WG;
             total += b.M;
         }
         std::vector<float> lc;
@@ -859,7 +872,7 @@ struct BatchRun {
             float *cfp = keep && total > 0 ? cf.p : nullptr;
             gf_mutid *cip = keep && total > 0 ? ci.p : nullptr;
             if (n + 2 <= SFS_LDS_BINS)
-                hipLaunchKernelGGL((k_bt_final<true>), dim3(grid), dim3(WG), 0, st, d_fin.p, nd, (int)tiles, d_fptr.p,
+                hipLaunchKernelGGL((k_bt_final<true>), dim3(grid), dim3(WG), sfs_lds_bytes(n, half_n), st, d_fin.p, nd, (int)tiles, d_fptr.p,
                                    d_iptr.p, n, half_n, d_lc.p, d_acc.p, cfp, cip);
             else
                 hipLaunchKernelGGL((k_bt_final<false>), dim3(grid), dim3(WG), 0, st, d_fin.p, nd, (int)tiles, d_fptr.p,

@@ -4,7 +4,7 @@
  * k_pop_hist: integer histogram of round(Nc * x) with bin Nc folded into 0
  *   (reference population_hist, spectrum.cu:74-83), LDS-privatised in passes
  *   over bin ranges of up to 40,960 bins.
- * k_sfs: expected SFS of an n-chromosome sample, sum over segregating
+ * k_sfs_row: expected SFS of an n-chromosome sample, sum over segregating
  *   mutations of exp(log C(n,k) + k log p + (n-k) log q) for k = 0..n
  *   (reference binom, spectrum.cu:111-139).  Each term is truncated to 2^-32
  *   fixed point and summed in 64-bit integers (LDS, then global), so the
@@ -99,30 +99,6 @@ __device__ __forceinline__ void sfs_add_mutation(float pf, int n, int half_n, co
     }
 }
 
-/* acc layout per segment: [0..n] fixed-point level sums, [n+1] count of
- * mutations that are not segregating (p <= 0 or p >= 1) */
-template <bool LDS>
-__global__ __launch_bounds__(WG) void k_sfs(const float *__restrict__ freq, const int64_t *__restrict__ seg_base,
-                                            const int *__restrict__ seg_M, const int *__restrict__ tile_seg,
-                                            const int *__restrict__ tile_first, int n, int half_n,
-                                            const float *__restrict__ lc, unsigned long long *__restrict__ acc) {
-    __shared__ unsigned long long sh[LDS ? SFS_LDS_BINS : 1];
-    const int tile = blockIdx.x;
-    const int s = tile_seg[tile];
-    const int li = (tile - tile_first[s]) * WG + (int)threadIdx.x;
-    unsigned long long *out = acc + (size_t)s * (n + 2);
-    if (LDS) {
-        for (int k = threadIdx.x; k < n + 2; k += WG) sh[k] = 0;
-        __syncthreads();
-    }
-    if (li < seg_M[s]) sfs_add_mutation<LDS>(freq[seg_base[s] + li], n, half_n, lc, sh, out);
-    if (LDS) {
-        __syncthreads();
-        for (int k = threadIdx.x; k < n + 2; k += WG)
-            if (sh[k]) atomicAdd(&out[k], sh[k]);
-    }
-}
-
 /* The sample SFS of one device row with every step on the device (no host
  * copy, no allocation): k_sfs_prep writes the log-binomial table lc[0 ..
  * half_n) with the host table's sequential float sum (log_binom_table) and
@@ -130,22 +106,36 @@ __global__ __launch_bounds__(WG) void k_sfs(const float *__restrict__ freq, cons
  * the M mutations; k_sfs_finish converts to the float spectrum as
  * finish_sfs does. */
 __global__ void k_sfs_prep(int n, int half_n, float *__restrict__ lc, unsigned long long *__restrict__ acc);
+/* level sums of the M mutations of one row: acc[0 .. n], and acc[n + 1] the
+ * mutations that are not segregating.  A grid-stride loop of SFS_ROW_WGS
+ * workgroups a CU at most, each with its own sums in LDS (dynamic, n + 2
+ * words) added to the global ones once: a workgroup per 256 mutations spent
+ * most of a small row's time on clearing and adding its sums. */
+constexpr int SFS_ROW_WGS = 4;
 template <bool LDS>
 __global__ __launch_bounds__(WG) void k_sfs_row(const float *__restrict__ freq, int M, int n, int half_n,
                                                 const float *__restrict__ lc, unsigned long long *__restrict__ acc) {
-    __shared__ unsigned long long sh[LDS ? SFS_LDS_BINS : 1];
+    extern __shared__ unsigned long long sh_sfs[];   /* LDS: sums, then the table: a lane reads it level by level */
+    float *sh_lc = reinterpret_cast<float *>(sh_sfs + n + 2);
     if (LDS) {
-        for (int k = threadIdx.x; k < n + 2; k += WG) sh[k] = 0;
+        for (int k = threadIdx.x; k < n + 2; k += WG) sh_sfs[k] = 0;
+        for (int k = threadIdx.x; k < half_n; k += WG) sh_lc[k] = lc[k];
         __syncthreads();
     }
-    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < M; i += (int64_t)gridDim.x * WG)
-        sfs_add_mutation<LDS>(freq[i], n, half_n, lc, sh, acc);
+    for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < M; i += (int64_t)gridDim.x * WG) {
+        if (LDS) sfs_add_mutation<LDS>(freq[i], n, half_n, sh_lc, sh_sfs, acc);
+        else sfs_add_mutation<LDS>(freq[i], n, half_n, lc, sh_sfs, acc);
+    }
     if (LDS) {
         __syncthreads();
         for (int k = threadIdx.x; k < n + 2; k += WG)
-            if (sh[k]) atomicAdd(&acc[k], sh[k]);
+            if (sh_sfs[k]) atomicAdd(&acc[k], sh_sfs[k]);
     }
 }
+/* bytes of LDS the sums of one sample size and its table take */
+inline size_t sfs_lds_bytes(int n, int half_n) { return (size_t)(n + 2) * sizeof(unsigned long long) + (size_t)half_n * sizeof(float); }
+/* k_sfs_row over a row on `st` */
+hipError_t launch_sfs_row(const float *d_freq, int M, int n, int half_n, const float *d_lc, unsigned long long *d_acc, hipStream_t st);
 __global__ void k_sfs_finish(const unsigned long long *__restrict__ acc, int n, int M, float num_sites,
                              float *__restrict__ out);
 
@@ -157,19 +147,14 @@ void finish_sfs(const unsigned long long *acc, unsigned long long nonseg, int n,
 struct SfsScratch {
     DevBuf<float> lc;
     DevBuf<unsigned long long> acc;
-    DevBuf<int> meta;
-    DevBuf<int64_t> base;
 };
 int sfs_of_device_row(const float *d_row, int M, int n, float num_sites, float *out, hipStream_t st,
                       SfsScratch *scratch = nullptr);
-int sfs_device(const float *d_freq, const int64_t *d_seg_base, const int *d_seg_M, const int *d_tile_seg,
-               const int *d_tile_first, int num_tiles, int nseg, int n, unsigned long long *d_acc,
-               hipStream_t st, DevBuf<float> &d_lc);
 
 /* ---------------- joint sample SFS of two populations ----------------
  * (no reference counterpart: the reference's spectrum is per population,
  * spectrum.h:23).  out[ka (nb+1) + kb] = sum over mutations of
- * Pa(ka) Pb(kb), with the per-population sample probabilities of k_sfs
+ * Pa(ka) Pb(kb), with the per-population sample probabilities of k_sfs_row
  * (mass at k = 0 or n for a frequency of 0 or 1); each product is
  * truncated to 2^-32 fixed point and summed exactly, so the result does
  * not depend on order.  Output-stationary: a workgroup owns

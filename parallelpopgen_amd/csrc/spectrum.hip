@@ -35,25 +35,14 @@ void finish_sfs(const unsigned long long *acc, unsigned long long nonseg, int n,
     for (int k = 1; k < n; k++) out[k] = (float)((double)acc[k] * sc);
 }
 
-int sfs_device(const float *d_freq, const int64_t *d_seg_base, const int *d_seg_M, const int *d_tile_seg,
-               const int *d_tile_first, int num_tiles, int nseg, int n, unsigned long long *d_acc,
-               hipStream_t st, DevBuf<float> &d_lc) {
-    std::vector<float> lc;
-    int half_n;
-    log_binom_table(n, lc, half_n);
-    GF_TRY(d_lc.alloc(lc.size()));
-    GF_HIP(hipMemcpyAsync(d_lc.p, lc.data(), lc.size() * sizeof(float), hipMemcpyHostToDevice, st));
-    GF_HIP(hipMemsetAsync(d_acc, 0, (size_t)nseg * (n + 2) * sizeof(unsigned long long), st));
-    if (num_tiles <= 0) return GF_OK;
-    const bool lds = (n + 2) <= SFS_LDS_BINS;
-    if (lds)
-        hipLaunchKernelGGL((k_sfs<true>), dim3(num_tiles), dim3(WG), 0, st, d_freq, d_seg_base, d_seg_M,
-                           d_tile_seg, d_tile_first, n, half_n, d_lc.p, d_acc);
+hipError_t launch_sfs_row(const float *d_freq, int M, int n, int half_n, const float *d_lc, unsigned long long *d_acc, hipStream_t st) {
+    const int grid = std::max(1, std::min((M + WG - 1) / WG, num_cus() * SFS_ROW_WGS));
+    if (n + 2 <= SFS_LDS_BINS)
+        hipLaunchKernelGGL((k_sfs_row<true>), dim3(grid), dim3(WG), sfs_lds_bytes(n, half_n), st, d_freq, M,
+                           n, half_n, d_lc, d_acc);
     else
-        hipLaunchKernelGGL((k_sfs<false>), dim3(num_tiles), dim3(WG), 0, st, d_freq, d_seg_base, d_seg_M,
-                           d_tile_seg, d_tile_first, n, half_n, d_lc.p, d_acc);
-    GF_HIP(hipGetLastError());
-    return GF_OK;
+        hipLaunchKernelGGL((k_sfs_row<false>), dim3(grid), dim3(WG), 0, st, d_freq, M, n, half_n, d_lc, d_acc);
+    return hipGetLastError();
 }
 
 int joint_sfs_of_device_rows(const float *d_fa, const float *d_fb, int M, int na, int nb, float num_sites, float *out,
@@ -131,19 +120,14 @@ int sfs_of_device_row(const float *d_row, int M, int n, float num_sites, float *
     SfsScratch &sc = scratch ? *scratch : local;
     DevBuf<float> &d_lc = sc.lc;
     DevBuf<unsigned long long> &d_acc = sc.acc;
-    DevBuf<int> &d_meta = sc.meta;
-    DevBuf<int64_t> &d_base = sc.base;
-    const int tiles = (M + WG - 1) / WG;
+    std::vector<float> lc;
+    int half_n;
+    log_binom_table(n, lc, half_n);
+    GF_TRY(d_lc.alloc(lc.size()));
     GF_TRY(d_acc.alloc((size_t)n + 2));
-    GF_TRY(d_meta.alloc((size_t)tiles + 2));
-    GF_TRY(d_base.alloc(1));
-    std::vector<int> meta((size_t)tiles + 2, 0);
-    meta[tiles] = M;      /* seg_M */
-    meta[tiles + 1] = 0;  /* tile_first */
-    const int64_t base0 = 0;
-    GF_HIP(hipMemcpyAsync(d_meta.p, meta.data(), meta.size() * sizeof(int), hipMemcpyHostToDevice, st));
-    GF_HIP(hipMemcpyAsync(d_base.p, &base0, sizeof(int64_t), hipMemcpyHostToDevice, st));
-    GF_TRY(sfs_device(d_row, d_base.p, d_meta.p + tiles, d_meta.p, d_meta.p + tiles + 1, tiles, 1, n, d_acc.p, st, d_lc));
+    GF_HIP(hipMemcpyAsync(d_lc.p, lc.data(), lc.size() * sizeof(float), hipMemcpyHostToDevice, st));
+    GF_HIP(hipMemsetAsync(d_acc.p, 0, ((size_t)n + 2) * sizeof(unsigned long long), st));
+    if (M > 0) GF_HIP(launch_sfs_row(d_row, M, n, half_n, d_lc.p, d_acc.p, st));
     std::vector<unsigned long long> acc((size_t)n + 2);
     GF_HIP(hipMemcpyAsync(acc.data(), d_acc.p, acc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
     GF_HIP(hipStreamSynchronize(st));
@@ -304,13 +288,7 @@ int32_t gf_site_frequency_spectrum_noalloc(const float *d_freq, int32_t M, int32
     const int half_n = (n % 2 == 0) ? n / 2 + 1 : (n + 1) / 2;
     hipStream_t st = (hipStream_t)stream;
     hipLaunchKernelGGL(k_sfs_prep, dim3(1), dim3(WG), 0, st, n, half_n, lc, acc);
-    if (M > 0) {
-        const int grid = std::max(1, std::min((M + WG - 1) / WG, num_cus() * 8));
-        if (n + 2 <= SFS_LDS_BINS)
-            hipLaunchKernelGGL((k_sfs_row<true>), dim3(grid), dim3(WG), 0, st, d_freq, M, n, half_n, lc, acc);
-        else
-            hipLaunchKernelGGL((k_sfs_row<false>), dim3(grid), dim3(WG), 0, st, d_freq, M, n, half_n, lc, acc);
-    }
+    if (M > 0) GF_HIP(launch_sfs_row(d_freq, M, n, half_n, lc, acc, st));
     hipLaunchKernelGGL(k_sfs_finish, dim3(1), dim3(WG), 0, st, acc, n, M, num_sites, d_out);
     GF_HIP(hipGetLastError());
     return GF_OK;
