@@ -331,8 +331,9 @@ int32_t gf_device_math(int32_t op, const void *in0, const void *in1, const void 
 
 /* Frees the device memory the library keeps for reuse on `device` (-1:
  * the current device).  Released device buffers are kept in a per-device
- * cache of at most 32 GiB instead of being returned with hipFree, which
- * waits for the whole device (no counterpart in the reference, which
+ * cache (at most a third of the device's memory) instead of being returned
+ * with hipFree, which waits for the whole device, and a few idle streams and
+ * pinned host blocks beside it; these go as well (no counterpart in the reference, which
  * allocates and frees on every compaction, go_fish_impl.cuh:377-428). */
 int32_t gf_release_device_cache(int32_t device);
 /* The cache's state on `device` (-1: the current device): out[0] bytes

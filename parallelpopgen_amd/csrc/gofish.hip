@@ -172,7 +172,7 @@ struct PlainRun {
     int G, start, final_g, interval;
     uint32_t k0, k1;
     std::vector<GenRow<P>> rows;          /* rows[t], t = 0..G */
-    std::vector<std::vector<uint8_t>> ext_at;
+    std::vector<uint8_t> ext_at;          /* [t][p], as rows */
     DevBuf<GenRow<P>> d_rows;
     DevBuf<unsigned long long> d_live;
     DevBuf<unsigned int> d_tickets;     /* one ticket counter per launch */
@@ -212,11 +212,14 @@ struct PlainRun {
     DevBuf<PoisTable> d_pois;           /* draw table of row pois_row's model (k_advance_const) */
     int pois_row = -1;
 
+    /* a run that ends early may have copies into the pinned words pending */
+    ~PlainRun() { if (st.st) (void)hipStreamSynchronize(st); }
+
     int plan() {
         const int Pn = d->num_populations;
         (void)Pn;
         rows.assign(G + 1, GenRow<P>{});
-        ext_at.assign(G + 1, std::vector<uint8_t>(P, 0));
+        ext_at.assign((size_t)(G + 1) * P, 0);
         std::vector<uint8_t> ext(P, 0);
         if (d->init_mode == GF_INIT_PREV && d->init_num_mutations > 0 && d->init_extinct)
             for (int p = 0; p < P; p++) ext[p] = d->init_extinct[p] ? 1 : 0;
@@ -266,7 +269,7 @@ struct PlainRun {
             }
             r.newcum[P] = (int)cum;
             for (int p = 0; p < P; p++) prevN[p] = pg[p].N;
-            ext_at[t] = ext;
+            std::copy(ext.begin(), ext.end(), ext_at.begin() + (ptrdiff_t)t * P);
         }
         return GF_OK;
     }
@@ -386,19 +389,20 @@ struct PlainRun {
                            any_sel ? d_area.p : nullptr, d_counts.p);
         GF_HIP(hipGetLastError());
         GF_TRY(scan_counts(d_counts.p, coff, d_scan.p, d_total.p, st, d_scratch));
-        /* per-segment first offsets and the total */
-        std::vector<int64_t> seg_first(ns);
-        for (int s = 0; s < ns; s++)
-            GF_HIP(hipMemcpyAsync(&seg_first[s], d_scan.p + segs[s].class_off, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-        int64_t total = 0;
-        GF_HIP(hipMemcpyAsync(&total, d_total.p, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-        GF_HIP(hipStreamSynchronize(st));
+        /* the segments' first offsets and the total */
+        DevBuf<int64_t> d_bounds;
+        GF_TRY(d_bounds.alloc((size_t)ns + 1));
+        hipLaunchKernelGGL(k_seg_bounds, dim3(1), dim3(256), 0, st, d_scan.p, d_offs.p, ns, d_total.p, d_bounds.p);
+        GF_HIP(hipGetLastError());
+        std::vector<int64_t> bounds((size_t)ns + 1);
+        GF_TRY(read_small(bounds.data(), d_bounds.p, bounds.size() * sizeof(int64_t), st));
+        const int64_t total = bounds[ns];
         if (total > 2000000000LL) { set_error("initial mutation count exceeds 2e9"); return GF_ERR_UNSUPPORTED; }
-        for (int s = 0; s < ns; s++) segs[s].slot_base = seg_first[s];
+        for (int s = 0; s < ns; s++) segs[s].slot_base = bounds[s];
         M = 0;
         GF_TRY(ensure_capacity(total + 1));
         GF_HIP(hipMemcpyAsync(d_segs.p, segs.data(), ns * sizeof(MseSeg), hipMemcpyHostToDevice, st));
-        GF_HIP(hipMemcpyAsync(d_offs.p, seg_first.data(), ns * sizeof(int64_t), hipMemcpyHostToDevice, st));
+        GF_HIP(hipMemcpyAsync(d_offs.p, bounds.data(), ns * sizeof(int64_t), hipMemcpyHostToDevice, st));
         if (total > 0) {
             /* zero every row first: k_mse_fill writes all P rows of each slot */
             hipLaunchKernelGGL(k_mse_fill<P>, dim3(grid), dim3(256), 0, st, d_segs.p, d_offs.p, ns, total,
@@ -494,7 +498,7 @@ struct PlainRun {
         const gf_pop_gen *pg = d->params + (size_t)t * P;
         for (int p = 0; p < P; p++) {
             s.Nchrom_e.push_back(nchrom(pg[p].N, pg[p].F));
-            s.extinct.push_back(ext_at[t][p]);
+            s.extinct.push_back(ext_at[(size_t)t * P + p]);
         }
         R->samples.push_back(std::move(s));
         return GF_OK;
@@ -768,7 +772,7 @@ struct PlainRun {
             GF_TRY(exact_M(cur));
             M = cur;
             int err = 0;
-            GF_HIP(hipMemcpy(&err, d_err.p, sizeof(int), hipMemcpyDeviceToHost));
+            GF_TRY(read_small(&err, d_err.p, sizeof(int), st));
             if (err) { set_error("advance kernel: the launch had fewer tiles than slots (internal bound)"); return GF_ERR_DEVICE; }
         }
         GF_TRY(take_sample(G, true));
@@ -780,8 +784,7 @@ struct PlainRun {
         hipLaunchKernelGGL(k_sum_live, dim3((G + 1 + 255) / 256), dim3(256), 0, st, d_live.p, d_sum.p, G + 1);
         GF_HIP(hipGetLastError());
         std::vector<unsigned long long> lv((size_t)G + 1);
-        GF_HIP(hipMemcpyAsync(lv.data(), d_sum.p, lv.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-        GF_HIP(hipStreamSynchronize(st));
+        GF_TRY(read_small(lv.data(), d_sum.p, lv.size() * sizeof(unsigned long long), st));
         R->live.assign(G + 1, 0);
         R->live[0] = live0;
         for (int tt = 1; tt <= G; tt++) R->live[tt] = (int64_t)lv[(size_t)tt];
@@ -837,6 +840,7 @@ int32_t gf_release_device_cache(int32_t device) {
     int dev = 0;
     GF_HIP(hipGetDevice(&dev));
     gf::DevCache::get().flush(dev);
+    gf::HostPool::get().flush(dev);
     if (dev != cur) GF_HIP(hipSetDevice(cur));
     return GF_OK;
 }

@@ -78,8 +78,7 @@ int joint_sfs_of_device_rows(const float *d_fa, const float *d_fb, int M, int na
         GF_HIP(hipGetLastError());
     }
     std::vector<unsigned long long> acc((size_t)B);
-    GF_HIP(hipMemcpyAsync(acc.data(), d_acc.p, acc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    GF_HIP(hipStreamSynchronize(st));
+    GF_TRY(read_small(acc.data(), d_acc.p, acc.size() * sizeof(unsigned long long), st));
     const double sc = 1.0 / 4294967296.0;
     for (int k = 0; k < B; k++) out[k] = (float)((double)acc[k] * sc + (k == 0 ? (double)num_sites - (double)M : 0.0));
     return GF_OK;
@@ -129,10 +128,15 @@ int sfs_of_device_row(const float *d_row, int M, int n, float num_sites, float *
     GF_HIP(hipMemsetAsync(d_acc.p, 0, ((size_t)n + 2) * sizeof(unsigned long long), st));
     if (M > 0) GF_HIP(launch_sfs_row(d_row, M, n, half_n, d_lc.p, d_acc.p, st));
     std::vector<unsigned long long> acc((size_t)n + 2);
-    GF_HIP(hipMemcpyAsync(acc.data(), d_acc.p, acc.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
-    GF_HIP(hipStreamSynchronize(st));
+    GF_TRY(read_small(acc.data(), d_acc.p, acc.size() * sizeof(unsigned long long), st));
     finish_sfs(acc.data(), acc[n + 1], n, M, num_sites, out);
     return GF_OK;
+}
+
+/* the counts as floats in place, bin 0 with the sites that hold no mutation */
+static __global__ __launch_bounds__(WG) void k_hist_out(unsigned int *__restrict__ hist, int Nc, unsigned int mono) {
+    const unsigned int k = blockIdx.x * WG + threadIdx.x;
+    if (k < (unsigned int)Nc) hist[k] = __float_as_uint((float)(hist[k] + (k == 0 ? mono : 0u)));
 }
 
 /* k_pop_hist over every bin range of [0, Nc): bin ranges as large as the
@@ -223,23 +227,22 @@ int32_t gf_population_histogram(const float *freq, int32_t M, int32_t Nc, float 
         rc = d_f.alloc(std::max(M, 1));
         if (!rc) rc = d_h.alloc(Nc);
         if (!rc) {
-            std::vector<unsigned int> h(Nc);
             hipError_t e = hipSuccess;
             if (M > 0) e = hipMemcpyAsync(d_f.p, freq, (size_t)M * sizeof(float), hipMemcpyHostToDevice, st);
             if (e == hipSuccess) e = hipMemsetAsync(d_h.p, 0, (size_t)Nc * sizeof(unsigned int), st);
-            if (e == hipSuccess && M > 0) {
-                e = launch_pop_hist(d_f.p, M, Nc, d_h.p, st);
+            if (e == hipSuccess && M > 0) e = launch_pop_hist(d_f.p, M, Nc, d_h.p, st);
+            if (e == hipSuccess) {
+                /* bin 0 also holds the monomorphic sites (spectrum.cu:82) */
+                const int ns = f2i_sat(__builtin_truncf(num_sites));
+                hipLaunchKernelGGL(k_hist_out, dim3(((unsigned)Nc + WG - 1) / WG), dim3(WG), 0, st, d_h.p, Nc, (unsigned int)(ns - M));
+                e = hipGetLastError();
             }
-            if (e == hipSuccess) e = hipMemcpyAsync(h.data(), d_h.p, (size_t)Nc * sizeof(unsigned int), hipMemcpyDeviceToHost, st);
-            if (e == hipSuccess) e = hipStreamSynchronize(st);
+            if (e == hipSuccess) e = hipStreamSynchronize(st);   /* before the staging buffer is taken */
             if (e != hipSuccess) {
                 set_error(std::string("population_frequency_histogram: ") + hipGetErrorString(e));
                 rc = GF_ERR_DEVICE;
             } else {
-                /* bin 0 also holds the monomorphic sites (spectrum.cu:82) */
-                const int ns = f2i_sat(__builtin_truncf(num_sites));
-                h[0] += (unsigned int)(ns - M);
-                for (int i = 0; i < Nc; i++) out[i] = (float)h[i];
+                rc = readback(out, d_h.p, (size_t)Nc * sizeof(float), st);
             }
         }
     }
