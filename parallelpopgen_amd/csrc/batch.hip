@@ -202,13 +202,34 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     __shared__ uint4 sh_pois[CONST ? POIS_ROWS * POIS_ROW_VECS : 1];
     load_draw_tables(sh_ncdf, sh_eneg);   /* published by the tile loop's first barrier */
     uint64_t live = 0;          /* this thread's slots' live mutation-generations */
-    for (int gt = blockIdx.x;; gt += gridDim.x) {
+    /* This workgroup's tiles are blockIdx.x + k gridDim.x.  Half and more of
+     * a layout's tiles hold nothing in a block (regions have headroom for
+     * the longest block, finished simulations keep theirs until the next
+     * layout), 2e6 of them for 8,192 growing simulations: every wave looks 64
+     * of its workgroup's tiles up at once and goes to the ones in use (one
+     * after the other, with a barrier and two dependent loads each, they
+     * took half of a late block's time). */
+    uint64_t todo = 0;
+    for (int64_t at = blockIdx.x, seen = at;;) {
+        if (todo == 0) {   /* uniform, and alike in all four waves */
+            at = seen;
+            if (at >= B.ntiles) break;
+            const int64_t t = at + (int64_t)lane * gridDim.x;
+            bool use = false;
+            if (t < B.ntiles) {
+                const BSim *b = sims + B.tile_sim[t];
+                use = (int)t - b->t0 < b->tiles && (b->counted != 0) == CONST;
+            }
+            todo = __ballot(use);
+            seen = at + (int64_t)64 * gridDim.x;
+            continue;
+        }
+        const int gt = (int)at + __builtin_ctzll(todo) * (int)gridDim.x;
+        todo &= todo - 1;
         __syncthreads();
-        if (gt >= B.ntiles) break;
         const int s = *as_const(B.tile_sim + gt);
         const BSim S = load_bsim(sims + s);
         const int j = gt - S.t0;
-        if (j >= S.tiles || (bool)S.counted != CONST) continue;
         if constexpr (CONST) {
             if (threadIdx.x < POIS_ROWS * POIS_ROW_VECS) sh_pois[threadIdx.x] = B.pois[s].v[threadIdx.x];
         }
