@@ -393,10 +393,12 @@ private:
         spare_.push_back(e);
     }
 
-    /* whether a block can be used without a wait; a stream that another
-     * thread waits on counts as busy */
+    /* whether a block can be used without a wait for another stream (the
+     * calling thread's own work counts as done, so that a call takes the same
+     * blocks however far the device has come); a stream that another thread
+     * waits on counts as busy */
     static bool ready_(const Block &b) {
-        if (!b.ev) return true;
+        if (!b.ev || b.tag == current_stream_tag()) return true;
         std::unique_lock<std::mutex> lock(b.tag->mu, std::try_to_lock);
         if (!lock.owns_lock()) return false;
         return !b.tag->alive || hipEventQuery(b.ev) == hipSuccess;
