@@ -113,6 +113,7 @@ struct BBufs {
     unsigned long long *live;     /* 64 partial sums of live mutation-generations */
     int *K;                       /* block length (device word: the tuner changes it between replays) */
     int ntiles, S;
+    int spans;                    /* tiles of only new mutations from which a simulation's go in spans (drift_span) */
 };
 
 /* a BSim read through scalar loads (uniform per tile) */
@@ -142,7 +143,8 @@ __device__ __forceinline__ void next_rows(BSim *__restrict__ sims, int s, const 
     const int lane = threadIdx.x & 63;
     BSim &b = sims[s];
     const bool run = b.status == BS_ACTIVE && b.g < b.G;
-    const int K = run ? min(*B.K, b.G - b.g) : 0;   /* at most BK_MAX = 32 */
+    int K = run ? min(*B.K, b.G - b.g) : 0;   /* at most BK_MAX = 32 */
+    if (K >= 8 && K < b.G - b.g) K -= (b.g + K + 1) & 3;   /* blocks end with a Philox block (a sweep 209 -> 205 ms) */
     const int n = lane < K ? new_mutation_count(b.Nc, b.mu, b.L, b.k0, b.k1, b.g + 1 + lane, 0) : 0;
     int cum = n;
 #pragma unroll
@@ -200,6 +202,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
     __shared__ ExpSeg sh_eneg[GF_EXPNEG_SEGMENTS];
     __shared__ uint4 sh_pois[CONST ? POIS_ROWS * POIS_ROW_VECS : 1];
+    __shared__ SpanQueues sh_span[CONST ? WG / 64 : 1];
     load_draw_tables(sh_ncdf, sh_eneg);   /* published by the tile loop's first barrier */
     uint64_t live = 0;          /* this thread's slots' live mutation-generations */
     /* This workgroup's tiles are blockIdx.x + k gridDim.x.  Half and more of
@@ -218,7 +221,13 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
             bool use = false;
             if (t < B.ntiles) {
                 const BSim *b = sims + B.tile_sim[t];
-                use = (int)t - b->t0 < b->tiles && (b->counted != 0) == CONST;
+                const int j = (int)t - b->t0;
+                use = j < b->tiles && (b->counted != 0) == CONST;
+                /* of the tiles that hold only new slots, the first of a group */
+                if (CONST) {
+                    const int old_tiles = (b->M + WG - 1) / WG;
+                    if (b->tiles - old_tiles >= B.spans) use = use && (j < old_tiles || (j - old_tiles) % (WG / 64) == 0);
+                }
             }
             todo = __ballot(use);
             seen = at + (int64_t)64 * gridDim.x;
@@ -250,42 +259,64 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const bool valid = li < Mend;
         const GenRow<1> *rows = B.rows + (size_t)s * BK_MAX;
         const int first = j * WG + w * 64;   /* the wave's first index */
+        if constexpr (CONST) {
+            __syncthreads();   /* sh_pois */
+            const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral, S.mid};
+            const int old_tiles = (M0 + WG - 1) / WG;
+            if (j >= old_tiles && S.tiles - old_tiles >= B.spans) {
+                const int tile = j + w;   /* a tile a wave */
+                if (tile < S.tiles) {
+                    const int64_t slot = base + (int64_t)tile * WG;
+                    const int kept = drift_span(
+                        tile * WG - M0, min((tile + 1) * WG, Mend) - M0, rows, 0, S.Kb, S.g, S.k0, S.k1, C, jn, sh_pois, sh_ncdf,
+                        sh_eneg, sh_span[w], [&](int b, int last) { live += (uint64_t)(last - b + 1); },
+                        [&](int tid, int ogen, int jc, int pos) {
+                            __builtin_nontemporal_store(quot_count((float)jc, C.N, C.r), &freq_out[slot + pos]);
+                            typedef int i4v __attribute__((ext_vector_type(4)));
+                            __builtin_nontemporal_store(i4v{ogen, 0, tid, 0}, reinterpret_cast<i4v *>(&ids_out[slot + pos]));
+                        });
+                    if (lane == 0) B.cnt[gt + w] = (unsigned int)kept;
+                }
+                continue;
+            }
+        }
         int64_t src = li;
         if (!dense && first < M0) src = frag_slot(li, first, j, src0_in, pre_in, S.T);
-        if (CONST) __syncthreads();   /* sh_pois */
         float x = 0.0f;
-        int jc = 0, born = -1;
-        uint32_t tid = 0;
+        int born = -1;
         gf_mutid id;
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
-        const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral, S.mid};
-        /* the start is counted in generation 0's chromosomes */
-        const bool first_freq = S.g == 0 && S.resized;
-        if (valid) {
-            if (li < M0) {
-                x = freq_in[base + src];
-                id = ids_in[base + src];
-                tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
-                jc = const_count(x, first_freq, C);
-            } else {
-                const int rel = li - M0;
-                int tb, pb;
-                find_birth<1>(rows, S.Kb, rel, tb, pb);
+        if (li < M0) {
+            x = freq_in[base + src];
+            id = ids_in[base + src];
+        }
+        if (first + 63 >= M0 && first < Mend) {
+            const int first_rel = max(first - M0, 0);
+            int t_at = first_birth(rows, S.Kb, first_rel), before;
+            const int tb = wave_birth(rows, S.Kb, li - M0, first_rel, t_at, before);
+            if (li >= M0 && valid) {
                 born = tb;
-                tid = (uint32_t)(rel - rows[tb].newcum[0] + 1);
                 id.origin_generation = S.g + 1 + tb;
-                id.origin_threadID = (int32_t)tid;
-                jc = 1;
+                id.origin_threadID = li - M0 - before + 1;
                 x = S.newfreq;
             }
         }
+        const uint32_t tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
         bool keep;
         if constexpr (CONST) {
-            int klast;
-            const_drift(jc, klast, x, first_freq, born, S.Kb, S.g, S.k0, S.k1, tid, id.origin_generation, 0, C, jn,
-                        sh_pois, sh_ncdf, sh_eneg);
-            if (klast >= 0) live += (uint64_t)(klast - (born < 0 ? 0 : born) + 1);
-            keep = klast == S.Kb - 1;
+            const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral, S.mid};
+            /* the start is counted in generation 0's chromosomes */
+            const bool first_freq = S.g == 0 && S.resized;
+            int jc = !valid ? 0 : (born >= 0 ? 1 : const_count(x, first_freq, C));
+            int lived = 0, pb = philox_base(born + 1, S.g);
+            int b = __builtin_amdgcn_readfirstlane(pb);   /* the earliest: births ascend over the lanes */
+            drift_four<true>(jc, lived, pb, born + 1, S.Kb, first_freq, x, S.g, S.k0, S.k1, tid, id.origin_generation, 0, C, jn,
+                             sh_pois, sh_ncdf, sh_eneg);
+            for (b += 4, pb += 4; b < S.Kb; b += 4, pb += 4)
+                drift_four<false>(jc, lived, pb, 0, S.Kb, false, 0.0f, S.g, S.k0, S.k1, tid, id.origin_generation, 0, C, jn, sh_pois,
+                                  sh_ncdf, sh_eneg);
+            live += (uint64_t)(lived + (born >= 0 ? 1 : 0));
+            keep = valid && born + lived == S.Kb - 1;
             x = quot_count((float)jc, C.N, C.r);
         } else {
             const auto *crows = as_const(rows);
@@ -821,6 +852,11 @@ struct BatchRun {
         B.live = live.p;
         B.K = d_K.p;
         B.ntiles = (int)ntiles;
+        /* A span's stages follow one another: spans pay while the layout
+         * keeps the device full (a sweep of 64 simulations, the layouts
+         * that take them from: none 214 ms, 256 tiles per CU 209, 64 219,
+         * any 225), and for a simulation with a workgroup's worth of them. */
+        B.spans = ntiles >= (int64_t)num_cus() * 256 ? 2 * (WG / 64) : INT32_MAX;
         B.S = S;
         return B;
     }

@@ -14,13 +14,20 @@
  * the number of thresholds below the word: two 16-byte LDS reads and eight
  * comparisons instead of exp(-m) and two to three trips of four terms.
  *
+ * A slot's generations go four at a time, one Philox block (drift_four): the
+ * word of each is fixed and nothing but the count and the end is checked in
+ * between.  The mutations born in the launch go in spans (drift_span).
+ *
  * Bound: vector-ALU issue.  2.0e6 mutations of N = 1e5, gamma = -10, ten
  * generations a launch: 6.9e7 vector instructions by k_advance_fused, 5.2e7
  * with the table, 4.5e7 with the arithmetic of gf_math.hpp (div_mid,
  * sqrt_pos, round_count) and the scalar gather (frag_slot) besides.  The
- * 5,000-generation run: 64.1 -> 51.2 -> 46.3 ms (44.4 with 16 generations a
- * launch); a run of 8.4e3 mutations
- * 2.14 -> 1.81 -> 1.74 ms; a batch of 64 uneven simulations 428 -> 261 ms.
+ * 5,000-generation run: 64.1 -> 51.2 -> 46.3 ms, 42.5 with 16 generations a
+ * launch and shorter Philox blocks, 38.6 with spans, 33.1 with 40
+ * generations a launch; a run of
+ * 8.4e3 mutations 1.30 -> 1.21 ms by
+ * drift_four; a batch of 64 uneven simulations 228 -> 214 by drift_four, 205
+ * with spans; training draws (8,192 growing simulations) 29.8 -> 28.9 -> 24.3.
  */
 #ifndef GF_CONST_DRIFT_HPP_
 #define GF_CONST_DRIFT_HPP_
@@ -117,27 +124,32 @@ GF_HD int pois_lookup(const uint4 *tab, int row, uint32_t bits) {
     return 5 * c + (int)(bits > b.x) + (int)(bits > b.y) + (int)(bits > b.z) + (int)(bits > b.w);
 }
 
-/* Advances one slot per lane through generations g0 + 1 .. g0 + K.  j: its
- * count (0 or Nc: absorbed); born: index of its birth generation in the
- * block, -1 for a slot that was there before (ascending over the lanes);
- * klast: the last generation in which it segregates, -1 if none (a slot's
- * birth generation counts).  first_freq: the first generation draws from the
- * frequency x instead of j / Nc (the state was counted in another number of
- * chromosomes). */
-__device__ __forceinline__ void const_drift(int &j, int &klast, float x, bool first_freq, int born, int K, int g0,
-                                            uint32_t k0, uint32_t k1, uint32_t tid, int ogen, int opop,
-                                            const ConstModel &C, int jn, const uint4 *tab, const NcdfSeg *ncdf,
-                                            const ExpSeg *etab) {
+/* Philox block that generation index t of a block of generations after g0
+ * belongs to: the index of its first generation (negative where the block
+ * began before g0 + 1) */
+__device__ __forceinline__ int philox_base(int t, int g0) { return t - ((g0 + 1 + t) & 3); }
+
+/* One Philox block, four generations, of one slot per lane: generation
+ * indices base .. base + 3 (base: philox_base of any of them; lanes need not
+ * agree on it), those before `start` (FIRST) and from K on left out.  j: the
+ * slot's count (0 or Nc: absorbed, nothing happens); lived: grows by one per
+ * generation the slot still segregates in.  first_freq (FIRST): generation
+ * index 0 draws from the frequency x instead of j / Nc (the state was counted
+ * in another number of chromosomes). */
+template <bool FIRST>
+__device__ __forceinline__ void drift_four(int &j, int &lived, int base, int start, int K, bool first_freq, float x, int g0,
+                                           uint32_t k0, uint32_t k1, uint32_t tid, int ogen, int opop, const ConstModel &C,
+                                           int jn, const uint4 *tab, const NcdfSeg *ncdf, const ExpSeg *etab) {
     GF_STRICT_FP
-    u32x4 rc = {0, 0, 0, 0};
     const unsigned inner = (unsigned)(C.Nc - 1);
-    klast = born;
-    for (int t = __builtin_amdgcn_readfirstlane(born) + 1; t < K; t++) {
-        const int g = g0 + 1 + t;
-        if ((unsigned)(j - 1) < inner && born < t) {
-            if ((g & 3) == 0 || t == born + 1) rc = drift_block(k0, k1, tid, ogen, opop, 0, g);
-            const uint32_t bits = lane_of(rc, g & 3);
-            const bool from_x = first_freq && t == 0;
+    const int left = K - base;
+    if (!((unsigned)(j - 1) < inner && left > 0)) return;
+    const u32x4 rc = drift_block(k0, k1, tid, ogen, opop, 0, g0 + 1 + base);
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        if ((unsigned)(j - 1) < inner && i < left && (!FIRST || base + i >= start)) {
+            const uint32_t bits = lane_of(rc, i);
+            const bool from_x = FIRST && first_freq && base + i == 0;
             if (!from_x && j < jn) {
                 j = pois_lookup(tab, j - 1, bits);
             } else {
@@ -155,10 +167,147 @@ __device__ __forceinline__ void const_drift(int &j, int &klast, float x, bool fi
                     j = round_count(binom_normal(u, mean, var, ncdf), C.N);
                 }
             }
-            if ((unsigned)(j - 1) < inner) klast = t;
+            lived += (unsigned)(j - 1) < inner ? 1 : 0;
         }
     }
 }
+
+/* Birth generation of the block's new mutation rel (counted from the run's
+ * start, as newcum) for every lane of a wave, whose lanes hold consecutive
+ * ones from first_rel up, and the cumulative count before it.  t_at: a
+ * generation not after the first lane's, moved up to it (scalar loads; a
+ * binary search per lane took six dependent vector loads). */
+__device__ __forceinline__ int wave_birth(const GenRow<1> *rows, int K, int rel, int first_rel, int &t_at, int &before) {
+    const auto *c = as_const(rows);
+    while (t_at + 1 < K && c[t_at + 1].newcum[0] <= first_rel) t_at++;
+    int t = t_at;
+    before = c[t].newcum[0];
+    for (int k = t_at + 1; k < K; k++) {
+        const int v = c[k].newcum[0];
+        if (v > first_rel + 63) break;
+        const bool passed = v <= rel;
+        t = passed ? k : t;
+        before = passed ? v : before;
+    }
+    return t;
+}
+
+/* the generation of first_rel by a binary search, for wave_birth's t_at */
+__device__ __forceinline__ int first_birth(const GenRow<1> *rows, int K, int first_rel) {
+    const auto *c = as_const(rows);
+    int lo = 0, hi = K - 1;          /* last t with newcum[0] <= first_rel */
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (c[mid].newcum[0] <= first_rel) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+__device__ __forceinline__ int rank_in(uint64_t mask) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+/* ---------------- the mutations born in a block ----------------
+ * More than half of a block's new mutations are lost within two
+ * generations, three quarters within four; in a slot per lane they left 40 %
+ * of all lanes of a run of 2.0e6 mutations idle, and 65 % of a batch of
+ * growing simulations.  A wave therefore takes a span of several hundred of
+ * them through three stages with a queue in LDS between two, each stage with
+ * full waves: the rest of the Philox block they are born in; the next
+ * Philox block; the rest of the launch's generations.  The queues keep the
+ * mutations' order, which the state's layout and the results rest on.  No
+ * barrier: a span is one wave's.  A lane's generation is its own (the model
+ * is the same in all), so a stage mixes mutations of different ages. */
+constexpr int SPAN_QUEUE = 128;  /* a stage starts with 64 waiting, or with the last */
+
+/* queue entry: the count (<= 2^21) and the birth generation (< 64) in one
+ * word, the thread ID in the other */
+struct SpanQueues { uint2 q[2][SPAN_QUEUE]; };
+
+/* New mutations n0 .. n1 - 1 (counted in the block; n0's slot starts a tile)
+ * of a block of K generations after g0.  count(born, last) is called for
+ * every lane whose mutation is gone, last = its last generation index, and
+ * for the survivors with last = K - 1; write(tid, ogen, count, pos) for each
+ * survivor, pos counting up from 0.  Returns the number of survivors. */
+template <typename Count, typename Write>
+__device__ __forceinline__ int drift_span(int n0, int n1, const GenRow<1> *rows, int cum_base, int K, int g0, uint32_t k0,
+                                          uint32_t k1, const ConstModel &C, int jn, const uint4 *tab, const NcdfSeg *ncdf,
+                                          const ExpSeg *etab, SpanQueues &sq, const Count &count, const Write &write) {
+    const int lane = threadIdx.x & 63;
+    const unsigned inner = (unsigned)(C.Nc - 1);
+    int waiting[2] = {0, 0}, head[2] = {0, 0};
+    int at = n0, out = 0;
+    int t_at = first_birth(rows, K, n0 + cum_base);
+    auto push = [&](int q, bool stays, int j, int born, int tid) {
+        const uint64_t b = __ballot(stays);
+        if (stays)
+            sq.q[q][(head[q] + waiting[q] + rank_in(b)) & (SPAN_QUEUE - 1)] =
+                uint2{(uint32_t)j | ((uint32_t)born << 22), (uint32_t)tid};
+        waiting[q] += (int)__popcll(b);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");   /* the queue is this wave's alone */
+    };
+    for (;;) {
+        const bool more = at < n1;
+        int j = 0, born = 0, tid = 0, lived = 0;
+        if (waiting[1] >= 64 || (!more && waiting[0] == 0)) {   /* the remaining generations */
+            const int m = min(waiting[1], 64);
+            if (m == 0) break;
+            const bool valid = lane < m;
+            if (valid) {
+                const uint2 e = sq.q[1][(head[1] + lane) & (SPAN_QUEUE - 1)];
+                j = (int)(e.x & 0x3fffffu);
+                born = (int)(e.x >> 22);
+                tid = (int)e.y;
+            }
+            head[1] += m;
+            waiting[1] -= m;
+            const int from = min(philox_base(born + 1, g0) + 8, K);
+            int base = philox_base(born + 1, g0) + 8;
+            for (int b = __builtin_amdgcn_readfirstlane(base); b < K; b += 4, base += 4)
+                drift_four<false>(j, lived, base, 0, K, false, 0.0f, g0, k0, k1, (uint32_t)tid, g0 + 1 + born, 0, C, jn, tab,
+                                  ncdf, etab);
+            if (valid) count(born, from - 1 + lived);
+            const bool keep = valid && (unsigned)(j - 1) < inner;
+            const uint64_t b = __ballot(keep);
+            if (keep) write(tid, g0 + 1 + born, j, out + rank_in(b));
+            out += (int)__popcll(b);
+        } else if (waiting[0] >= 64 || !more) {   /* one Philox block */
+            const int m = min(waiting[0], 64);
+            const bool valid = lane < m;
+            if (valid) {
+                const uint2 e = sq.q[0][(head[0] + lane) & (SPAN_QUEUE - 1)];
+                j = (int)(e.x & 0x3fffffu);
+                born = (int)(e.x >> 22);
+                tid = (int)e.y;
+            }
+            head[0] += m;
+            waiting[0] -= m;
+            const int base = philox_base(born + 1, g0) + 4;
+            drift_four<false>(j, lived, base, 0, K, false, 0.0f, g0, k0, k1, (uint32_t)tid, g0 + 1 + born, 0, C, jn, tab, ncdf,
+                              etab);
+            const bool stays = valid && (unsigned)(j - 1) < inner;
+            if (valid && !stays) count(born, base - 1 + lived);
+            push(1, stays, j, born, tid);
+        } else {   /* birth, and the rest of its Philox block */
+            const bool valid = at + lane < n1;
+            const int rel = at + lane + cum_base;
+            int before;
+            born = wave_birth(rows, K, rel, at + cum_base, t_at, before);
+            tid = rel - before + 1;
+            j = valid ? 1 : 0;
+            at += 64;
+            drift_four<true>(j, lived, philox_base(born + 1, g0), born + 1, K, false, 0.0f, g0, k0, k1, (uint32_t)tid,
+                             g0 + 1 + born, 0, C, jn, tab, ncdf, etab);
+            const bool stays = valid && (unsigned)(j - 1) < inner;
+            if (valid && !stays) count(born, born + lived);
+            push(0, stays, j, born, tid);
+        }
+    }
+    return out;
+}
+
+/* survivors in tile `k` of a span of which n are left, packed from its first slot */
+__device__ __forceinline__ unsigned int span_count(int n, int k) { return (unsigned int)min(max(n - k * WG, 0), WG); }
 
 /* count of a slot read from the state, and its frequency if the first
  * generation needs it (const_drift's x): any count strictly between 0 and Nc
@@ -177,11 +326,13 @@ static __global__ __launch_bounds__(POIS_BUILD) void k_pois_table(const GenRow<1
 }
 
 /* k_advance_fused for one population and a launch whose model rows are all
- * alike (same arguments, layout and results) */
+ * alike (same arguments, layout and results).  spans: tiles of new mutations a
+ * wave takes as one span, 0: new mutations have a slot per lane like the old
+ * ones. */
 static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_advance_const(const FusedLaunch F,
                                                                                               const SegLaunch<1> S,
                                                                                               const PoisTable *__restrict__ ptab,
-                                                                                              int mid, int first_freq) {
+                                                                                              int mid, int first_freq, int spans) {
     const int lane = threadIdx.x & 63;
     const int w = wave_index();
     __shared__ unsigned int sh_wcount[WG / 64];
@@ -189,11 +340,12 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
     __shared__ NcdfSeg sh_ncdf[GF_NCDF_SEGMENTS];
     __shared__ ExpSeg sh_eneg[GF_EXPNEG_SEGMENTS];
     __shared__ uint4 sh_pois[POIS_ROWS * POIS_ROW_VECS];
+    __shared__ SpanQueues sh_span[WG / 64];
     load_draw_tables(sh_ncdf, sh_eneg);   /* published by the tile loop's first barrier */
     if (threadIdx.x < POIS_ROWS * POIS_ROW_VECS) sh_pois[threadIdx.x] = ptab->v[threadIdx.x];
     if (threadIdx.x <= KMAX) sh_diff[threadIdx.x] = 0;
     const int jn = as_const(ptab)->jn;
-    const int M0 = *F.M_in;
+    const int M0 = __builtin_amdgcn_readfirstlane(*F.M_in);
     const int Mend = M0 + F.new_in_block;
     const int need_tiles = (Mend + WG - 1) / WG;
     const int T_in = F.dense ? 0 : *F.T_in;
@@ -203,9 +355,39 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
     const ConstModel C{R.Nc[0], R.fN[0], R.newfreq[0], R.sa[0], R.sb[0], R.c1[0], R.c2[0], R.neutral_mask & 1, mid};
     const int K = S.K;
     const int last_tile = need_tiles < F.ntiles ? need_tiles : F.ntiles;
-    for (int tile = (int)blockIdx.x;; tile += (int)gridDim.x) {
+    /* the tiles that hold only new slots go in spans, ahead of the others */
+    const int old_tiles = spans ? min((M0 + WG - 1) / WG, last_tile) : last_tile;
+    const int per_item = spans * (WG / 64);
+    const int groups = spans ? (last_tile - old_tiles + per_item - 1) / per_item : 0;
+    auto store = [&](int64_t o, int j, int tid, int ogen, int opop, int rest) {
+        __builtin_nontemporal_store(quot_count((float)j, C.N, C.r), &F.freq_out[o]);
+        if (F.preserve) tid = -(tid < 0 ? -tid : tid);
+        typedef int i4v __attribute__((ext_vector_type(4)));
+        const i4v v = {ogen, opop, tid, rest};
+        __builtin_nontemporal_store(v, reinterpret_cast<i4v *>(&F.ids_out[o]));
+    };
+    /* per-generation live counts as a difference array: +1 at the start for
+     * an old slot, -1 after a slot's last generation; the births, whose
+     * numbers the rows hold, are added at the end */
+    auto count = [&](int, int last) {
+        if (last + 1 < K) atomicAdd(&sh_diff[last + 1], -1);
+    };
+    for (int item = (int)blockIdx.x;; item += (int)gridDim.x) {
         __syncthreads();
-        if (tile >= last_tile) break;
+        if (item >= groups + old_tiles) break;
+        if (item < groups) {
+            const int first = old_tiles + item * per_item + w * spans;   /* tile */
+            const int tiles = min(last_tile - first, spans);
+            if (tiles > 0) {
+                const int64_t slot = (int64_t)first * WG;
+                const int n = drift_span(first * WG - M0, min((first + tiles) * WG, Mend) - M0, rows, S.cum_base, K, S.g0, S.k0, S.k1,
+                                         C, jn, sh_pois, sh_ncdf, sh_eneg, sh_span[w], count,
+                                         [&](int tid, int ogen, int j, int pos) { store(slot + pos, j, tid, ogen, 0, 0); });
+                if (lane < tiles) F.cnt_out[first + lane] = span_count(n, lane);
+            }
+            continue;
+        }
+        const int tile = item - groups;
         const int li = tile * WG + (int)threadIdx.x;
         const bool valid = li < Mend;
         const int first = tile * WG + w * 64;   /* the wave's first index */
@@ -213,55 +395,45 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
         if (!F.dense && first < M0) src = frag_slot(li, first, tile, F.src0_in, F.pre_in, T_in);
         float x = 0.0f;
         int j = 0, born = -1;
-        uint32_t tid = 0;
         gf_mutid id;
         id.origin_generation = 0; id.origin_population = 0; id.origin_threadID = 0; id.reserved = 0;
-        if (valid) {
-            if (li < M0) {
-                x = F.freq_in[src];
-                id = F.ids_in[src];
-                tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
-                j = const_count(x, first_freq, C);
-            } else {
-                const int rel = li - M0 + S.cum_base;
-                int tb, pb;
-                find_birth<1>(rows, K, rel, tb, pb);
+        if (li < M0) {
+            x = F.freq_in[src];
+            id = F.ids_in[src];
+            j = const_count(x, first_freq, C);
+        }
+        if (first + 63 >= M0 && first < Mend) {
+            const int first_rel = max(first - M0, 0) + S.cum_base;
+            int t_at = first_birth(rows, K, first_rel), before;
+            const int tb = wave_birth(rows, K, li - M0 + S.cum_base, first_rel, t_at, before);
+            if (li >= M0 && valid) {
                 born = tb;
-                tid = (uint32_t)(rel - rows[tb].newcum[0] + 1);
                 id.origin_generation = S.g0 + 1 + tb;
-                id.origin_threadID = (int32_t)tid;
+                id.origin_threadID = li - M0 + S.cum_base - before + 1;
                 j = 1;
             }
         }
-        int klast;
-        const_drift(j, klast, x, first_freq, born, K, S.g0, S.k0, S.k1, tid, id.origin_generation, id.origin_population,
-                    C, jn, sh_pois, sh_ncdf, sh_eneg);
-        if (id.origin_threadID < 0) klast = K - 1;   /* preserved: kept in every generation */
-        /* per-generation live counts as a difference array: +1 at the first
-         * generation a slot is kept, -1 after its last one */
-        const uint64_t old = __ballot(klast >= 0 && born < 0);
+        const uint32_t tid = (uint32_t)(id.origin_threadID < 0 ? -id.origin_threadID : id.origin_threadID);
+        int lived = 0, base = philox_base(born + 1, S.g0);
+        int b = __builtin_amdgcn_readfirstlane(base);   /* the earliest: births ascend over the lanes */
+        drift_four<true>(j, lived, base, born + 1, K, first_freq, x, S.g0, S.k0, S.k1, tid, id.origin_generation,
+                         id.origin_population, C, jn, sh_pois, sh_ncdf, sh_eneg);
+        for (b += 4, base += 4; b < K; b += 4, base += 4)
+            drift_four<false>(j, lived, base, 0, K, false, 0.0f, S.g0, S.k0, S.k1, tid, id.origin_generation,
+                              id.origin_population, C, jn, sh_pois, sh_ncdf, sh_eneg);
+        /* the last generation the slot is kept in; preserved: every one */
+        const int last = !valid ? -1 : (id.origin_threadID < 0 ? K - 1 : born + lived);
+        const uint64_t old = __ballot(last >= 0 && born < 0);
         if (lane == 0 && old) atomicAdd(&sh_diff[0], (int)__popcll(old));
-        if (born >= 0) atomicAdd(&sh_diff[born], 1);
-        if (klast >= 0 && klast + 1 < K) atomicAdd(&sh_diff[klast + 1], -1);
-        const bool keep = F.compact ? klast == K - 1 : valid;
+        if (last >= 0 && last + 1 < K) atomicAdd(&sh_diff[last + 1], -1);
+        const bool keep = F.compact ? last == K - 1 : valid;
         /* tile-local stable packing */
         const uint64_t kb = __ballot(keep);
         if (lane == 0) sh_wcount[w] = (unsigned int)__popcll(kb);
         __syncthreads();
         unsigned int pos = 0;
         for (int k = 0; k < w; k++) pos += sh_wcount[k];
-        pos += __builtin_amdgcn_mbcnt_hi((uint32_t)(kb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kb, 0u));
-        if (keep) {
-            const int64_t o = (int64_t)tile * WG + pos;
-            __builtin_nontemporal_store(quot_count((float)j, C.N, C.r), &F.freq_out[o]);
-            if (F.preserve) {
-                const int z = id.origin_threadID;
-                id.origin_threadID = -(z < 0 ? -z : z);
-            }
-            typedef int i4v __attribute__((ext_vector_type(4)));
-            const i4v v = {id.origin_generation, id.origin_population, id.origin_threadID, id.reserved};
-            __builtin_nontemporal_store(v, reinterpret_cast<i4v *>(&F.ids_out[o]));
-        }
+        if (keep) store((int64_t)tile * WG + pos + rank_in(kb), j, id.origin_threadID, id.origin_generation, id.origin_population, id.reserved);
         if (threadIdx.x == 0) {
             unsigned int c = 0;
             for (int k = 0; k < WG / 64; k++) c += sh_wcount[k];
@@ -271,11 +443,13 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
     __syncthreads();
     if (w == 0) {   /* prefix of the difference array: lane t holds generation t */
         int run = lane < K ? sh_diff[lane] : 0;
+        const int births = blockIdx.x == 0 && lane < K ? rows[lane].newcum[1] - S.cum_base : 0;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) {
             const int y = __shfl_up(run, off);
             if (lane >= off) run += y;
         }
+        run += births;
         if (lane < K && run) atomicAdd(&S.live[(size_t)(S.t0 + lane) * 64 + (blockIdx.x & 63)], (unsigned long long)run);
     }
 }

@@ -546,6 +546,20 @@ struct PlainRun {
         return true;
     }
 
+    /* Tiles of new mutations a wave takes as one span (drift_span), 0: none.
+     * A span's stages follow one another, so they pay where the new tiles
+     * alone give every SIMD a wave (1,000 generations, in ms, a slot per lane
+     * / a tile / two tiles a wave: 8.4e4 live, 6.4e4 to 1.3e5 new per launch
+     * 1.60 / 1.62 / 2.10; 1.7e5 live, 5e5 new 1.85 / 1.69 / -; 2.5e5 live,
+     * 7.7e5 new 2.22 / 1.86 / 2.47; 8.4e5 live, 1.9e6 new 5.0 / 3.6 / 4.1),
+     * and two tiles a wave, with fuller late stages, where they give
+     * it eight (2.0e6 live, 4e6 new, 2,000 generations 20.4 / 15.1 / 14.2). */
+    int span_tiles(const FusedLaunch &F) const {
+        const int64_t wave_each = (int64_t)num_cus() * 4 * WG;
+        if (!F.compact || F.new_in_block < wave_each) return 0;
+        return F.new_in_block < 8 * wave_each ? 1 : 2;
+    }
+
     int advance_const(const FusedLaunch &F, const SegLaunch<P> &sl, int t_first, int grid) {
         if constexpr (P == 1) {
             const gf_pop_gen &pg = d->params[t_first];
@@ -558,7 +572,7 @@ struct PlainRun {
             }
             const int Nc_prev = t_first > 1 ? rows[t_first - 1].Nc[0] : nchrom(d->params[0].N, d->params[0].F);
             hipLaunchKernelGGL(k_advance_const, dim3(grid), dim3(WG), 0, st, F, sl, d_pois.p,
-                               mid, Nc_prev == rows[t_first].Nc[0] ? 0 : 1);
+                               mid, Nc_prev == rows[t_first].Nc[0] ? 0 : 1, span_tiles(F));
         }
         return GF_OK;
     }
@@ -712,24 +726,36 @@ struct PlainRun {
         /* generations per launch, unless the caller set it.  One population
          * compacts at every launch: a longer launch saves launch overhead
          * (a scan and two gaps, 13 us) but carries the slots lost inside it
-         * to its end.  By the slots in use, measured best (ms per run of
-         * 1,000 generations, live mutations at the end): 8.4e4: 64 (32 2.11,
-         * 48 1.93, 64 1.84); 2.5e5: 48 (16 2.82, 32 2.46, 48 2.44); 8.4e5:
-         * 20 (10 5.35, 16 4.89, 20 4.84, 32 5.07); 2.0e6: 16 (2,000
-         * generations: 10 19.6, 14 18.9, 16 18.9, 24 19.8); 2.6e7: 12 to 20
-         * alike.  Several populations end launches at the
-         * compaction interval anyway: up to 2e6 slots a launch runs to it
-         * (two populations, N = 1e4, 1,000 generations, interval 35: 20
-         * generations per launch 3.73 / 5.82 / 21.9 ms at 1.4e4 / 1.4e5 /
-         * 1.4e6 live, up to the interval 3.35 / 4.95 / 19.6 ms), 20
-         * generations beyond (three populations of 2e4-2e5 over 2,000
-         * generations: 16 per launch 158 ms, 20 146 ms, 24 146 ms). */
+         * to its end, except those born in it where they go in spans
+         * (k_advance_const).  By the slots in use, measured best in ms: with
+         * spans, 2.5e5: 64 (1,000 generations: 32 2.2, 48 2.2, 64 2.1);
+         * 8.4e5: 48 (32 4.22, 48 4.10, 64 4.08); 2.0e6: 40 (2,000
+         * generations: 24 15.9, 32 15.3, 40 14.2, 48 15.1); 2.6e7: 24 (200
+         * generations: 16 24.7, 24 24.7, 32 24.5).  Without (a model that
+         * changes), per 1,000 generations: 8.4e4: 64 (32 2.11, 48 1.93, 64
+         * 1.84); 2.5e5: 48 (16 2.82, 32 2.46, 48 2.44); 8.4e5: 20 (10 5.35,
+         * 16 4.89, 20 4.84, 32 5.07); 2.0e6: 16 (2,000: 10 19.6, 14 18.9, 16
+         * 18.9, 24 19.8); 2.6e7: 12 to 20 alike.  Several populations end
+         * launches at the compaction interval anyway: up to 2e6 slots a
+         * launch runs to it (two populations, N = 1e4, 1,000 generations,
+         * interval 35: 20 generations per launch 3.73 / 5.82 / 21.9 ms at
+         * 1.4e4 / 1.4e5 / 1.4e6 live, up to the interval 3.35 / 4.95 / 19.6
+         * ms), 20 generations beyond (three populations of 2e4-2e5 over
+         * 2,000 generations: 16 per launch 158 ms, 20 146 ms, 24 146 ms).
+         * One population's launches end with a Philox block (2.0e6: 15.7 ->
+         * 15.5 ms). */
         const int k_user = generations_per_launch(0);
-        auto launch_length = [&]() {
+        auto launch_length = [&](int t) {
             int k;
             if (k_user > 0) k = k_user;
-            else if (P == 1) k = M_seen <= 150000 ? 64 : (M_seen <= 400000 ? 48 : (M_seen <= 1200000 ? 20 : 16));
-            else k = M_bound <= 2000000 ? 64 : 20;
+            else if (P == 1) {
+                k = M_seen <= 400000 ? 64 : (M_seen <= 1200000 ? 48 : (M_seen <= 4000000 ? 40 : 24));
+                if (interval <= 0 || !const_model(t + 1, std::min(k, G - t)))
+                    k = M_seen <= 150000 ? 64 : (M_seen <= 400000 ? 48 : (M_seen <= 1200000 ? 20 : 16));
+                if (t + k < G) k -= (start + t + k + 1) & 3;
+                /* far from the slot limit and the device's memory */
+                if (M_bound + rows[std::min(t + k, G)].newcum[P] - rows[t + 1].newcum[0] > 200000000) k = std::min(k, 10);
+            } else k = M_bound <= 2000000 ? 64 : 20;
             return std::max(1, std::min(KMAX, k));
         };
         /* one population: a lost or fixed mutation never changes again, so
@@ -737,7 +763,7 @@ struct PlainRun {
         const bool compact_every_launch = (P == 1 && interval > 0);
         int rc = GF_OK;
         while (t < G) {
-            const int kpl = launch_length();
+            const int kpl = launch_length(t);
             int K = 0;
             for (;;) {
                 K++;
