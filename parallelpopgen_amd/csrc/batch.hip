@@ -320,21 +320,23 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
             x = quot_count((float)jc, C.N, C.r);
         } else {
             const auto *crows = as_const(rows);
-            u32x4 rc[1];
             keep = false;
             int kfirst = KMAX, klast = -1;
-            for (int t = 0; t < S.Kb; t++) {
-                const auto &R = crows[t];
-                const int g = S.g + 1 + t;
-                if (valid && born < t) {
-                    const bool refresh = ((g & 3) == 0) || (t == born + 1);
-                    generation_update<1>(&x, R, g, refresh, rc, S.k0, S.k1, tid, id.origin_generation, 0, LinearSel(),
-                                         sh_ncdf, sh_eneg);
+            for (int pb = philox_base(0, S.g); pb < S.Kb; pb += 4) {
+                u32x4 rc = {0, 0, 0, 0};
+                if (valid && born < pb + 3) rc = drift_block(S.k0, S.k1, tid, id.origin_generation, 0, 0, S.g + 1 + pb);
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    const int t = pb + i;
+                    if (t < 0 || t >= S.Kb) continue;
+                    const auto &R = crows[t];
+                    const uint32_t bits = lane_of(rc, i);
+                    if (valid && born < t) generation_update<1, false>(&x, R, S.g + 1 + t, &bits, LinearSel(), sh_ncdf, sh_eneg);
+                    keep = valid && born <= t && keep_rule<1>(&x, R.present_mask, false);
+                    /* one population: kept over one run of generations (lost
+                     * and fixed are absorbing) */
+                    if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
                 }
-                keep = valid && born <= t && keep_rule<1>(&x, R.present_mask, false);
-                /* one population: kept over one run of generations (lost and
-                 * fixed are absorbing) */
-                if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
             }
             if (klast >= 0) live += (uint64_t)(klast - kfirst + 1);
         }

@@ -124,11 +124,6 @@ GF_HD int pois_lookup(const uint4 *tab, int row, uint32_t bits) {
     return 5 * c + (int)(bits > b.x) + (int)(bits > b.y) + (int)(bits > b.z) + (int)(bits > b.w);
 }
 
-/* Philox block that generation index t of a block of generations after g0
- * belongs to: the index of its first generation (negative where the block
- * began before g0 + 1) */
-__device__ __forceinline__ int philox_base(int t, int g0) { return t - ((g0 + 1 + t) & 3); }
-
 /* One Philox block, four generations, of one slot per lane: generation
  * indices base .. base + 3 (base: philox_base of any of them; lanes need not
  * agree on it), those before `start` (FIRST) and from K on left out.  j: the

@@ -143,23 +143,22 @@ GF_HD bool mid_selection(float sa, float sb, float F, float h) {
  * populations), selection (Eq. 13 of the reference's model, with F and h)
  * and an approximate binomial(N, x') drift draw, clamped to [0, N].
  *
- * rc[p] caches the lane's Philox block for generations 4b..4b+3 (the
- * reference's float4 packing, go_fish_impl.cuh:107).  It is fetched when
- * `refresh` is set (at a block boundary, or in the first generation a slot
- * is drifted in this launch), also for a population that is empty in this
- * generation, so that it is current if the population is founded later in
- * the same block.  ncdf and etab are the workgroup's LDS copies of the
- * inverse normal's and exp(-m)'s segment tables (load_draw_tables). */
-template <int P, typename Row, typename Sel>
-__device__ __forceinline__ void generation_update(float *x, const Row &R, int g, bool refresh, u32x4 *rc,
-                                                  uint32_t k0, uint32_t k1, uint32_t tid, int ogen, int opop,
-                                                  const Sel &sel, const NcdfSeg *ncdf, const ExpSeg *etab) {
+ * bits[p] is the lane's random word for population p (also where it is empty).
+ * ncdf and etab are the workgroup's LDS copies of the inverse normal's and
+ * exp(-m)'s segment tables (load_draw_tables).
+ *
+ * SIMPLE (simple_rows): selection does not depend on the frequency (sa = 0,
+ * with sb clamped by the host), Eq. 13 stays in div_mid's range, and the
+ * chromosome numbers lie in [100, 2^22]: 12 vector instructions fewer per
+ * population and generation, of about 100. */
+template <int P, bool SIMPLE, typename Row, typename Sel>
+__device__ __forceinline__ void generation_update(float *x, const Row &R, int g, const uint32_t *bits, const Sel &sel,
+                                                  const NcdfSeg *ncdf, const ExpSeg *etab) {
     GF_STRICT_FP
     float nx[P];
 #pragma unroll
     for (int p = 0; p < P; p++) {
         const int Nc = R.Nc[p];
-        if (refresh) rc[p] = drift_block(k0, k1, tid, ogen, opop, p, g);
         if (Nc <= 0) { nx[p] = 0.0f; continue; }
         /* one population: the migration weight is 1 (conservative
          * migration), and 0 + 1 * x == x */
@@ -171,6 +170,8 @@ __device__ __forceinline__ void generation_update(float *x, const Row &R, int g,
         float xs;
         if (R.neutral_mask & (1 << p)) {
             xs = im;   /* s == 0: Eq. 13 reduces exactly to x */
+        } else if (SIMPLE) {
+            xs = selected_freq(im, R.sb[p], R.c1[p], R.c2[p], true);
         } else {
             float s = sel(p, g, im, R);
             s = s > -1.0f ? s : -1.0f;
@@ -179,17 +180,37 @@ __device__ __forceinline__ void generation_update(float *x, const Row &R, int g,
         const float N = R.fN[p];
         const float mean = xs * N;
         const float var = (1.0f - xs) * mean;
-        const int j = binom_count(lane_of(rc[p], g & 3), mean, var, N, Nc, ncdf, etab);
-        /* (float)j / N, correctly rounded: up to N = 2^22 in three float
-         * operations with r = RN(1/N), the row's newfreq (quot_count),
-         * above through double (invN); the test is on the integer Nc, a
-         * scalar comparison */
-        const float fj = (float)j;
-        nx[p] = Nc <= 4194304 ? quot_count(fj, N, R.newfreq[p]) : (float)((double)fj * R.invN[p]);
+        if (SIMPLE) {
+            const float u = u01(bits[p]);
+            const bool lo = mean <= 6.0f;
+            float fj;
+            if (lo || mean >= N - 6.0f) {
+                const float m = lo ? mean : N - mean;
+                const int k = m != 0.0f ? poiscdfinv_tail<true>(u, m, etab) : 0;
+                const int d = lo ? k : f2i_sat(N - (float)k);
+                fj = (float)min(max(d, 0), Nc);
+            } else {
+                fj = (float)round_count(binom_normal(u, mean, var, ncdf), N);
+            }
+            nx[p] = quot_count(fj, N, R.newfreq[p]);
+        } else {
+            const int j = binom_count(bits[p], mean, var, N, Nc, ncdf, etab);
+            /* (float)j / N, correctly rounded: up to N = 2^22 in three float
+             * operations with r = RN(1/N), the row's newfreq (quot_count),
+             * above through double (invN); the test is on the integer Nc, a
+             * scalar comparison */
+            const float fj = (float)j;
+            nx[p] = Nc <= 4194304 ? quot_count(fj, N, R.newfreq[p]) : (float)((double)fj * R.invN[p]);
+        }
     }
 #pragma unroll
     for (int p = 0; p < P; p++) x[p] = nx[p];
 }
+
+/* Philox block that generation index t of a launch after generation g0
+ * belongs to: the index of its first generation (negative where the block
+ * began before g0 + 1) */
+__device__ __forceinline__ int philox_base(int t, int g0) { return t - ((g0 + 1 + t) & 3); }
 
 /* copies the inverse normal's and exp(-m)'s segment tables into LDS (all
  * threads of the workgroup; the caller's next barrier publishes them) */
@@ -301,7 +322,7 @@ __device__ __forceinline__ int64_t frag_slot(int li, int first, int tile, const 
 /* the wave's index in its workgroup, as a scalar */
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
 
-template <int P, typename Sel>
+template <int P, typename Sel, bool SIMPLE = false>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_advance_fused(const FusedLaunch F, const SegLaunch<P> S,
                                                                                           const Sel sel) {
     const int lane = threadIdx.x & 63;
@@ -377,24 +398,37 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
             }
         }
         const auto *crows = as_const(rows);
-        u32x4 rc[P];
         bool keep = false;
         int kfirst = KMAX, klast = -1;
-        for (int t = 0; t < S.K; t++) {
-            const auto &R = crows[t];
-            const int g = S.g0 + 1 + t;
-            if (valid && born < t) {
-                const bool refresh = ((g & 3) == 0) || (t == born + 1);
-                generation_update<P>(x, R, g, refresh, rc, S.k0, S.k1, tid, ogen, opop, sel, sh_ncdf, sh_eneg);
+        /* four generations at a time, one Philox block per population, whose
+         * words are then in fixed registers */
+        for (int base = philox_base(0, S.g0); base < S.K; base += 4) {
+            u32x4 rc[P];
+            if (valid && born < base + 3) {
+#pragma unroll
+                for (int p = 0; p < P; p++) rc[p] = drift_block(S.k0, S.k1, tid, ogen, opop, p, S.g0 + 1 + base);
             }
-            keep = valid && born <= t && keep_rule<P>(x, R.present_mask, preserved);
-            if constexpr (P == 1) {
-                /* one population: a slot is kept over one run of generations
-                 * (lost and fixed are absorbing), recorded by its ends */
-                if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
-            } else {
-                const uint64_t b = __ballot(keep);
-                if (lane == t) cnt += (uint64_t)__popcll(b);
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const int t = base + i;
+                if (t < 0 || t >= S.K) continue;
+                const auto &R = crows[t];
+                if (valid && born < t) {
+                    uint32_t bits[P];
+#pragma unroll
+                    for (int p = 0; p < P; p++) bits[p] = lane_of(rc[p], i);
+                    generation_update<P, SIMPLE>(x, R, S.g0 + 1 + t, bits, sel, sh_ncdf, sh_eneg);
+                }
+                keep = valid && born <= t && keep_rule<P>(x, R.present_mask, preserved);
+                if constexpr (P == 1) {
+                    /* one population: a slot is kept over one run of
+                     * generations (lost and fixed are absorbing), recorded by
+                     * its ends */
+                    if (keep) { kfirst = t < kfirst ? t : kfirst; klast = t; }
+                } else {
+                    const uint64_t b = __ballot(keep);
+                    if (lane == t) cnt += (uint64_t)__popcll(b);
+                }
             }
         }
         if constexpr (P == 1) {

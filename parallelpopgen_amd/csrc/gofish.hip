@@ -252,6 +252,8 @@ struct PlainRun {
                 const float F = pg[p].F, h = pg[p].h;
                 r.sa[p] = pg[p].sel_slope;
                 r.sb[p] = pg[p].sel_intercept;
+                /* sa = 0: the model's clamp s >= -1 once, here */
+                if (r.sa[p] == 0.0f && !(r.sb[p] > -1.0f)) r.sb[p] = -1.0f;
                 r.c1[p] = (F + h) - (h * F);
                 r.c2[p] = (F + (2.0f * h)) - ((2.0f * h) * F);
                 for (int k = 0; k < P; k++) r.mig[k][p] = mig[k * P + p];
@@ -534,6 +536,29 @@ struct PlainRun {
                a.c1[0] == b.c1[0] && a.c2[0] == b.c2[0];
     }
 
+    /* whether generations t_first .. t_first+K-1 are generation_update's
+     * SIMPLE: in every row selection without slope in mid_selection's range,
+     * 100 to 2^22 chromosomes in every population that is drifted, and
+     * frequencies after migration that are 0 or at least 2^-79 (counts of at
+     * most 2^31 chromosomes, weights of at least 2^-40; not the caller's
+     * frequencies) */
+    bool simple_rows(int t_first, int K) const {
+        if (hooks || (t_first == 1 && d->init_mode == GF_INIT_PREV)) return false;
+        for (int t = t_first; t < t_first + K; t++) {
+            const GenRow<P> &r = rows[t];
+            const gf_pop_gen *pg = d->params + (size_t)t * P;
+            for (int p = 0; p < P; p++) {
+                if (r.Nc[p] <= 0) continue;
+                if (r.Nc[p] < 100 || r.Nc[p] > (1 << 22) || r.sa[p] != 0.0f ||
+                    !mid_selection(0.0f, r.sb[p], pg[p].F, pg[p].h))
+                    return false;
+                for (int k = 0; k < P; k++)
+                    if (!(r.mig[k][p] == 0.0f || r.mig[k][p] >= 0x1p-40f)) return false;
+            }
+        }
+        return true;
+    }
+
     /* whether generations t_first .. t_first+K-1 run as k_advance_const: one
      * population, the library's own selection form, one model throughout,
      * and a state counted in some number of chromosomes (every state but a
@@ -623,6 +648,8 @@ struct PlainRun {
             if (rc != GF_OK) { set_error("run_sim: selection advance hook failed"); return rc; }
         } else if (const_model(t_first, K)) {
             GF_TRY(advance_const(F, sl, t_first, grid));
+        } else if (simple_rows(t_first, K)) {
+            hipLaunchKernelGGL((k_advance_fused<P, LinearSel, true>), dim3(grid), dim3(WG), 0, st, F, sl, LinearSel());
         } else {
             hipLaunchKernelGGL((k_advance_fused<P, LinearSel>), dim3(grid), dim3(WG), 0, st, F, sl, LinearSel());
         }
