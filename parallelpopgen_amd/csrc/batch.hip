@@ -235,7 +235,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         }
         const int gt = (int)at + __builtin_ctzll(todo) * (int)gridDim.x;
         todo &= todo - 1;
-        __syncthreads();
+        sync_lds();
         const int s = *as_const(B.tile_sim + gt);
         const BSim S = load_bsim(sims + s);
         const int j = gt - S.t0;
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         const GenRow<1> *rows = B.rows + (size_t)s * BK_MAX;
         const int first = j * WG + w * 64;   /* the wave's first index */
         if constexpr (CONST) {
-            __syncthreads();   /* sh_pois */
+            sync_lds();   /* sh_pois */
             const ConstModel C{S.Nc, S.fN, S.newfreq, 0.0f, S.s, S.c1, S.c2, S.neutral, S.mid};
             const int old_tiles = (M0 + WG - 1) / WG;
             if (j >= old_tiles && S.tiles - old_tiles >= B.spans) {
@@ -343,7 +343,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         /* tile-local stable packing into the other buffer */
         const uint64_t kb = __ballot(keep);
         if (lane == 0) sh_wcount[w] = (unsigned int)__popcll(kb);
-        __syncthreads();
+        sync_lds();
         if (keep) {
             unsigned int pos = 0;
             for (int k = 0; k < w; k++) pos += sh_wcount[k];

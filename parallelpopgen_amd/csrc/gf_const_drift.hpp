@@ -187,21 +187,6 @@ __device__ __forceinline__ int wave_birth(const GenRow<1> *rows, int K, int rel,
     return t;
 }
 
-/* the generation of first_rel by a binary search, for wave_birth's t_at */
-__device__ __forceinline__ int first_birth(const GenRow<1> *rows, int K, int first_rel) {
-    const auto *c = as_const(rows);
-    int lo = 0, hi = K - 1;          /* last t with newcum[0] <= first_rel */
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (c[mid].newcum[0] <= first_rel) lo = mid; else hi = mid - 1;
-    }
-    return lo;
-}
-
-__device__ __forceinline__ int rank_in(uint64_t mask) {
-    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-}
-
 /* ---------------- the mutations born in a block ----------------
  * More than half of a block's new mutations are lost within two
  * generations, three quarters within four; in a slot per lane they left 40 %
@@ -368,7 +353,7 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
         if (last + 1 < K) atomicAdd(&sh_diff[last + 1], -1);
     };
     for (int item = (int)blockIdx.x;; item += (int)gridDim.x) {
-        __syncthreads();
+        sync_lds();
         if (item >= groups + old_tiles) break;
         if (item < groups) {
             const int first = old_tiles + item * per_item + w * spans;   /* tile */
@@ -425,7 +410,7 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
         /* tile-local stable packing */
         const uint64_t kb = __ballot(keep);
         if (lane == 0) sh_wcount[w] = (unsigned int)__popcll(kb);
-        __syncthreads();
+        sync_lds();
         unsigned int pos = 0;
         for (int k = 0; k < w; k++) pos += sh_wcount[k];
         if (keep) store((int64_t)tile * WG + pos + rank_in(kb), j, id.origin_threadID, id.origin_generation, id.origin_population, id.reserved);
@@ -435,7 +420,7 @@ static __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) 
             F.cnt_out[tile] = c;
         }
     }
-    __syncthreads();
+    sync_lds();
     if (w == 0) {   /* prefix of the difference array: lane t holds generation t */
         int run = lane < K ? sh_diff[lane] : 0;
         const int births = blockIdx.x == 0 && lane < K ? rows[lane].newcum[1] - S.cum_base : 0;

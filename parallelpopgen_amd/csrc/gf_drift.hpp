@@ -319,8 +319,37 @@ __device__ __forceinline__ int64_t frag_slot(int li, int first, int tile, const 
     return (int64_t)s * WG + (li - at);
 }
 
+/* __syncthreads with this wave's LDS writes done first.  Said in so many
+ * words: the compiler (ROCm 7.2) left the wait out before some barriers that
+ * a loop's back edge or a long branch-free stretch led to, and another wave
+ * then read the old words now and then. */
+__device__ __forceinline__ void sync_lds() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#endif
+    __syncthreads();
+}
+
 /* the wave's index in its workgroup, as a scalar */
 __device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); }
+
+/* Birth generation of the block's new mutation rel: the last row whose newcum
+ * is at most rel (scalar loads: rel is uniform) */
+template <int P>
+__device__ __forceinline__ int first_birth(const GenRow<P> *rows, int K, int rel) {
+    const auto *c = as_const(rows);
+    int lo = 0, hi = K - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (c[mid].newcum[0] <= rel) lo = mid; else hi = mid - 1;
+    }
+    return lo;
+}
+
+/* set bits of `mask` below the lane */
+__device__ __forceinline__ int rank_in(uint64_t mask) {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
 
 template <int P, typename Sel, bool SIMPLE = false>
 __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_advance_fused(const FusedLaunch F, const SegLaunch<P> S,
@@ -349,13 +378,13 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
      * tile (the cost of a tile varies with the populations its slots hold). */
     const int last_tile = need_tiles < F.ntiles ? need_tiles : F.ntiles;
     for (int it = 0;; it++) {
-        __syncthreads();
+        sync_lds();
         int tile;
         if constexpr (P == 1) {
             tile = (int)blockIdx.x + it * (int)gridDim.x;
         } else {
             if (threadIdx.x == 0) sh_tile = (int)atomicAdd(F.ticket, 1u);
-            __syncthreads();
+            sync_lds();
             tile = __builtin_amdgcn_readfirstlane(sh_tile);
         }
         if (tile >= last_tile) break;
@@ -444,7 +473,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
         /* tile-local stable packing */
         const uint64_t kb = __ballot(keep);
         if (lane == 0) sh_wcount[w] = (unsigned int)__popcll(kb);
-        __syncthreads();
+        sync_lds();
         unsigned int pos = 0;
         for (int k = 0; k < w; k++) pos += sh_wcount[k];
         pos += __builtin_amdgcn_mbcnt_hi((uint32_t)(kb >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)kb, 0u));
@@ -470,7 +499,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     }
     /* per-generation live counts: lane t of every wave holds generation t */
     if constexpr (P == 1) {
-        __syncthreads();
+        sync_lds();
         if (threadIdx.x == 0) {   /* prefix of the difference array */
             long long run = 0;
             for (int t = 0; t < S.K; t++) {
@@ -481,7 +510,7 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     } else {
         if (cnt) atomicAdd(&sh_live[lane], (unsigned long long)cnt);
     }
-    __syncthreads();
+    sync_lds();
     if ((int)threadIdx.x < S.K && sh_live[threadIdx.x])
         atomicAdd(&S.live[(size_t)(S.t0 + threadIdx.x) * 64 + (blockIdx.x & 63)], sh_live[threadIdx.x]);
 }

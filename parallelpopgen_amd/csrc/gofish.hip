@@ -12,6 +12,7 @@
  */
 #include "gf_kernels.hpp"
 #include "gf_const_drift.hpp"
+#include "gf_packed_drift.hpp"
 #include "gf_runtime.hpp"
 #include "gf_spectrum.hpp"
 
@@ -559,6 +560,20 @@ struct PlainRun {
         return true;
     }
 
+    /* Tiles of a chunk of k_advance_packed, 0: k_advance_fused.  Two to four
+     * populations, and tiles enough for four chunks of two per workgroup the
+     * device holds: a chunk's batches follow one another (three populations
+     * over 2,000 generations, 35 a launch, in ms, by the tiles a chunk tile
+     * needs at least: never packed 83.6, 2,048 62.3, 4,096 60.2, 8,192 56.3,
+     * 16,384 56.0; the same without preserved mutations 34.9, 45.1, 40.9,
+     * 31.6, 34.9, and on three times the sites 95.0, 85.3, 84.7, 82.9,
+     * 104.3; two populations of 3,000 tiles in chunks of 1, 2, 4: 4.3, 5.2,
+     * 7.7). */
+    int packed_tiles(int ntiles) const {
+        const int c = ntiles / (num_cus() * 32);
+        return P < 2 || P > 4 || c < 2 ? 0 : std::min(c, PACK_TILES);
+    }
+
     /* whether generations t_first .. t_first+K-1 run as k_advance_const: one
      * population, the library's own selection form, one model throughout,
      * and a state counted in some number of chromosomes (every state but a
@@ -648,6 +663,14 @@ struct PlainRun {
             if (rc != GF_OK) { set_error("run_sim: selection advance hook failed"); return rc; }
         } else if (const_model(t_first, K)) {
             GF_TRY(advance_const(F, sl, t_first, grid));
+        } else if (const int chunk = packed_tiles(ntiles)) {
+            if constexpr (P >= 2 && P <= 4) {
+                const int pgrid = std::max(1, std::min((ntiles + chunk - 1) / chunk, num_cus() * 8));
+                if (simple_rows(t_first, K))
+                    hipLaunchKernelGGL((k_advance_packed<P, true>), dim3(pgrid), dim3(WG), 0, st, F, sl, chunk);
+                else
+                    hipLaunchKernelGGL((k_advance_packed<P, false>), dim3(pgrid), dim3(WG), 0, st, F, sl, chunk);
+            }
         } else if (simple_rows(t_first, K)) {
             hipLaunchKernelGGL((k_advance_fused<P, LinearSel, true>), dim3(grid), dim3(WG), 0, st, F, sl, LinearSel());
         } else {
@@ -767,11 +790,15 @@ struct PlainRun {
          * launch runs to it (two populations, N = 1e4, 1,000 generations,
          * interval 35: 20 generations per launch 3.73 / 5.82 / 21.9 ms at
          * 1.4e4 / 1.4e5 / 1.4e6 live, up to the interval 3.35 / 4.95 / 19.6
-         * ms), 20 generations beyond (three populations of 2e4-2e5 over
-         * 2,000 generations: 16 per launch 158 ms, 20 146 ms, 24 146 ms).
+         * ms), at most 35 generations beyond (three populations of 2e4-2e5
+         * over 2,000 generations, interval 35: 12 72.8, 18 64.9, 20 64.5, 35
+         * 56.3).
          * One population's launches end with a Philox block (2.0e6: 15.7 ->
          * 15.5 ms). */
         const int k_user = generations_per_launch(0);
+        auto slots_after = [&](int t, int k) {
+            return M_bound + rows[std::min(t + k, G)].newcum[P] - rows[t + 1].newcum[0];
+        };
         auto launch_length = [&](int t) {
             int k;
             if (k_user > 0) k = k_user;
@@ -781,8 +808,11 @@ struct PlainRun {
                     k = M_seen <= 150000 ? 64 : (M_seen <= 400000 ? 48 : (M_seen <= 1200000 ? 20 : 16));
                 if (t + k < G) k -= (start + t + k + 1) & 3;
                 /* far from the slot limit and the device's memory */
-                if (M_bound + rows[std::min(t + k, G)].newcum[P] - rows[t + 1].newcum[0] > 200000000) k = std::min(k, 10);
-            } else k = M_bound <= 2000000 ? 64 : 20;
+                if (slots_after(t, k) > 200000000) k = std::min(k, 10);
+            } else {
+                k = M_bound <= 2000000 ? 64 : 35;
+                if (k == 35 && slots_after(t, k) > 200000000) k = 20;
+            }
             return std::max(1, std::min(KMAX, k));
         };
         /* one population: a lost or fixed mutation never changes again, so
