@@ -375,15 +375,16 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(8))) void k_
     /* Tile order.  One population: a fixed stride over the tiles (their
      * costs are alike, and a ticket's atomic round trip was measured to cost
      * more than the imbalance).  Several populations: an atomic ticket per
-     * tile (the cost of a tile varies with the populations its slots hold). */
+     * tile (the cost of a tile varies with the populations its slots hold)
+     * after the first, which is the workgroup's own, if there are any left:
+     * 2,048 tickets drawn at once from one word took about 20 us (two
+     * populations over 1,001 generations, 34 launches: 4.32 -> 3.60 ms). */
     const int last_tile = need_tiles < F.ntiles ? need_tiles : F.ntiles;
     for (int it = 0;; it++) {
         sync_lds();
-        int tile;
-        if constexpr (P == 1) {
-            tile = (int)blockIdx.x + it * (int)gridDim.x;
-        } else {
-            if (threadIdx.x == 0) sh_tile = (int)atomicAdd(F.ticket, 1u);
+        int tile = (int)blockIdx.x + it * (int)gridDim.x;
+        if (P > 1 && it > 0 && last_tile > (int)gridDim.x) {
+            if (threadIdx.x == 0) sh_tile = (int)(gridDim.x + atomicAdd(F.ticket, 1u));
             sync_lds();
             tile = __builtin_amdgcn_readfirstlane(sh_tile);
         }

@@ -123,9 +123,9 @@ __global__ __launch_bounds__(WG) __attribute__((amdgpu_waves_per_eu(6))) void k_
     };
 
     int parity = 0;
-    for (;;) {
+    for (bool own = true;; own = false) {   /* its own chunk, then tickets */
         sync_lds();
-        if (threadIdx.x == 0) sh_chunk = (int)atomicAdd(F.ticket, 1u);
+        if (threadIdx.x == 0) sh_chunk = (int)(own ? blockIdx.x : gridDim.x + atomicAdd(F.ticket, 1u));
         if (threadIdx.x < PACK_TILES * (WG / 32)) L.keep[threadIdx.x] = L.gone[threadIdx.x] = 0;
         sync_lds();
         const int chunk = __builtin_amdgcn_readfirstlane(sh_chunk) * tiles_per_chunk;   /* its first tile */
