@@ -12,7 +12,7 @@ live (segregating or preserved) mutations after each generation's update,
 divided by the wall time of the step.
 
 Prints ONE JSON line (rank 0, N = 1).  Also reports:
-  roofline      the drift kernel (k_advance_fused) against MI355X HBM peak, with
+  roofline      the drift kernel (k_advance_const) against MI355X HBM peak, with
                 8 algorithmic bytes per mutation-generation (4 B read + 4 B
                 written state), timed with HIP events on the library stream;
                 traffic = measured HBM bytes per launch from rocprofv3
@@ -470,7 +470,7 @@ def main():
             "traffic": traffic,
             "traffic_source": "FETCH_SIZE + WRITE_SIZE per launch of this kernel on this workload, from "
                               "rocprofv3 --pmc runs (profiles/advance_traffic.json), not measured in this run",
-            "kernel": "k_advance_fused (migration_selection_drift + add_new_mutations + tile-local compaction, "
+            "kernel": "k_advance_const (migration_selection_drift + add_new_mutations + tile-local compaction, "
                       "%.1f generations per launch)" % (a.generations * a.steps / max(adv_launch, 1)),
             "avg_launch_ms": avg_launch_ms,
             "timed_launches": adv_timed,

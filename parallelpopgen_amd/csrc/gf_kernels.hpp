@@ -1,8 +1,9 @@
 /*
  * gf_kernels.hpp -- library-only gfx950 kernels of the GO_Fish hot path:
  * stream compaction (batched path and initial counts), the
- * mutation-selection-equilibrium start and scans.  The drift kernel and the
- * shared types are in gf_drift.hpp.
+ * mutation-selection-equilibrium start and scans.  The drift kernels and the
+ * shared types are in gf_drift.hpp, gf_const_drift.hpp and
+ * gf_packed_drift.hpp.
  */
 #ifndef GF_KERNELS_HPP_
 #define GF_KERNELS_HPP_
