@@ -680,20 +680,20 @@ struct PlainRun {
         t_adv.end(ev);
         /* survivors per tile -> prefix, slot count, next launch's source tiles */
         const int slot = (int)(launches % RING);
-        /* more than two chunks of tiles: sum the chunks, then scan them in
-         * parallel (one workgroup walking 14 chunks took 110 us) */
-        const int nchunks = (int)((ntiles + SCAN_CHUNK - 1) / SCAN_CHUNK);
-        const bool chunked = nchunks > 2;
-        if (chunked) {
+        int *pre_out = d_pre.p + (par ^ 1) * pre_half, *src0_out = d_src0.p + (par ^ 1) * src_half;
+        if (ntiles <= SCAN_SELF) {
+            hipLaunchKernelGGL(k_tile_scan<4>, dim3(std::max(1, (ntiles + SCAN_SELF_CHUNK - 1) / SCAN_SELF_CHUNK)), dim3(1024), 0, st, d_cnt.p,
+                               d_M.p + mcur, (int)new_in_block, pre_out, src0_out, d_M.p + (mcur ^ 1), d_T.p + (par ^ 1),
+                               &h_ring.p[slot], (const int *)nullptr);
+        } else {
+            const int nchunks = (int)((ntiles + SCAN_CHUNK - 1) / SCAN_CHUNK);
             if ((size_t)nchunks > d_chunk.n) { set_error("tile scan: chunk buffer smaller than the launch"); return GF_ERR_DEVICE; }
             hipLaunchKernelGGL(k_tile_chunk_sums, dim3(nchunks), dim3(1024), 0, st, d_cnt.p, d_M.p + mcur,
                                (int)new_in_block, d_chunk.p);
             GF_HIP(hipGetLastError());
+            hipLaunchKernelGGL(k_tile_scan<16>, dim3(nchunks), dim3(1024), 0, st, d_cnt.p, d_M.p + mcur, (int)new_in_block,
+                               pre_out, src0_out, d_M.p + (mcur ^ 1), d_T.p + (par ^ 1), &h_ring.p[slot], (const int *)d_chunk.p);
         }
-        hipLaunchKernelGGL(k_tile_scan, dim3(chunked ? nchunks : 1), dim3(1024), 0, st, d_cnt.p, d_M.p + mcur,
-                           (int)new_in_block, d_pre.p + (par ^ 1) * pre_half, d_src0.p + (par ^ 1) * src_half,
-                           d_M.p + (mcur ^ 1), d_T.p + (par ^ 1), &h_ring.p[slot],
-                           chunked ? (const int *)d_chunk.p : (const int *)nullptr);
         GF_HIP(hipGetLastError());
         freqA.swap(freqB);
         idsA.swap(idsB);

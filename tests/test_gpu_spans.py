@@ -58,3 +58,16 @@ def test_batch_spans(gpu, K):
         assert np.array_equal(a["ids"], ids), k
         live += int(a["live"][1:].sum())
     assert live == b["live_mutation_generations"]
+
+
+# the tile scan's two forms: around one chunk (4,096 tiles), several, and the
+# last count that a workgroup adds up itself (65,536)
+@pytest.mark.parametrize("L", [3.1e10, 3.4e10, 1.6e11, 5.5e11])
+def test_tile_scan_sizes(gpu, oracle, L):
+    d = S.constant(N=1000, L=L, G=3, s=-0.001, compact_interval=1)
+    gpu.set_generations_per_launch(1)
+    try:
+        a = gpu.run(d)
+    finally:
+        gpu.set_generations_per_launch(0)
+    assert_same(a, oracle.run(d), L)
