@@ -75,7 +75,11 @@ __device__ __forceinline__ void sfs_add_mutation(float pf, int n, int half_n, co
         };
         auto add = [&](int k, float t) {
             if (t < -23.0f) return;
-            const unsigned long long v = (unsigned long long)(exp_f(t) * 4294967296.0f);
+            /* t is finite and below 1, where exp_f_mid is exp_f; below 2^32
+             * the 32-bit conversion is the 64-bit one */
+            const float f = exp_f_mid(t) * 4294967296.0f;
+            unsigned long long v = (uint32_t)f;
+            if (f >= 4294967296.0f) v = (unsigned long long)f;
             if (v) {
                 if (LDS) atomicAdd(&sh[k], v);
                 else atomicAdd(&out[k], v);
