@@ -116,8 +116,10 @@ __global__ void k_sfs_prep(int n, int half_n, float *__restrict__ lc, unsigned l
  * words) added to the global ones once: a workgroup per 256 mutations spent
  * most of a small row's time on clearing and adding its sums.  Bound by the
  * exponentials and LDS additions of a few dozen levels per mutation.  A row
- * of 1.4e7 mutations, n = 50: 652 -> 104 us (one workgroup per 256 -> this);
- * 2.0e6, n = 1,000: 163 -> 112; 2e5, n = 100: 44 -> 40. */
+ * of 1.4e7 mutations, n = 50: 652 -> 104 us (one workgroup per 256 -> this)
+ * -> 86 with exp_f_mid; 2.0e6, n = 1,000: 163 -> 112 -> 88; 2e5, n = 100: 44
+ * -> 40 -> 33.  Two lanes a mutation, one for either side of its mode: 8.4e3
+ * mutations 15 -> 11, but 1.4e7 86 -> 131. */
 constexpr int SFS_ROW_WGS = 4;
 template <bool LDS>
 __global__ __launch_bounds__(WG) void k_sfs_row(const float *__restrict__ freq, int M, int n, int half_n,
