@@ -77,6 +77,12 @@ GF_HD float const_mean(int j, const ConstModel &C) {
     return const_selected(quot_count((float)j, C.N, C.r), C) * C.N;
 }
 
+/* whether a fixed mutation stays fixed, as the count form takes for granted
+ * (drift_four leaves a count of Nc alone): not where Eq. 13 is no number at a
+ * frequency of 1, whose draw is 0 (s(1) <= -1: 0/0).  A lost one stays lost in
+ * every model: 0, or no number, there.  (A batch drops both at every block.) */
+GF_HD bool const_keeps_fixed(const ConstModel &C) { return const_selected(1.0f, C) == 1.0f; }
+
 /* T[k] of the row with mean `mean` in [0, 6] */
 GF_HD uint32_t pois_threshold(float mean, int k) {
     GF_STRICT_FP

@@ -574,13 +574,19 @@ struct PlainRun {
         return P < 2 || P > 4 || c < 2 ? 0 : std::min(c, PACK_TILES);
     }
 
+    static ConstModel model_of(const GenRow<P> &r, int mid) {
+        return ConstModel{r.Nc[0], r.fN[0], r.newfreq[0], r.sa[0], r.sb[0], r.c1[0], r.c2[0], r.neutral_mask & 1, mid};
+    }
+
     /* whether generations t_first .. t_first+K-1 run as k_advance_const: one
-     * population, the library's own selection form, one model throughout,
-     * and a state counted in some number of chromosomes (every state but a
-     * previous run's, whose frequencies are the caller's) */
+     * population, the library's own selection form, one model throughout
+     * that keeps fixed mutations fixed (those preserved, or never compacted,
+     * are in the state), and a state counted in some number of chromosomes
+     * (every state but a previous run's, whose frequencies are the caller's) */
     bool const_model(int t_first, int K) const {
         if (P != 1 || hooks || (t_first == 1 && d->init_mode == GF_INIT_PREV)) return false;
         if (!const_drift_range(rows[t_first].Nc[0]) || !(rows[t_first].present_mask & 1)) return false;
+        if (!const_keeps_fixed(model_of(rows[t_first], 0))) return false;
         for (int t = t_first + 1; t < t_first + K; t++)
             if (!same_model(rows[t], rows[t_first])) return false;
         return true;
