@@ -282,7 +282,11 @@ static __global__ __launch_bounds__(JW_WG) void k_joint_sfs_wave(const float *__
         float pf = 0.5f;
         if (mine < nm) pf = (lane < JW_BATCH ? fa : fb)[m0 + mine];
         const bool inner = pf > 0.0f && pf < 1.0f;
-        const float lp = inner ? log_f(pf) : 0.0f, lq = inner ? log_f(1.0f - pf) : 0.0f;
+        float lp = inner ? log_f(pf) : 0.0f, lq = inner ? log_f(1.0f - pf) : 0.0f;
+        if (pf != pf) {   /* no number: a frequency between, every level of which vanishes */
+            pf = 0.5f;
+            lp = lq = -1e30f;
+        }
         for (int m = 0; m < nm; m++) {
             const float pa = level(pf, lp, lq, m, na, ca);
             const float pb = level(pf, lp, lq, m + JW_BATCH, nb, cb) * 4294967296.0f;
