@@ -75,9 +75,12 @@ __device__ __forceinline__ void sfs_add_mutation(float pf, int n, int half_n, co
         };
         auto add = [&](int k, float t) {
             if (t < -23.0f) return;
-            /* t is finite and below 1, where exp_f_mid is exp_f; below 2^32
-             * the 32-bit conversion is the 64-bit one */
-            const float f = exp_f_mid(t) * 4294967296.0f;
+            /* samples whose sums fit LDS: t is finite and below 1, where
+             * exp_f_mid is exp_f.  (From 1.5e6 chromosomes up the rounding
+             * errors of the table's float sum take t past 88, where exp_f
+             * overflows and exp_f_mid is no exponential.)  Below 2^32 the
+             * 32-bit conversion is the 64-bit one. */
+            const float f = (LDS ? exp_f_mid(t) : exp_f(t)) * 4294967296.0f;
             unsigned long long v = (uint32_t)f;
             if (f >= 4294967296.0f) v = (unsigned long long)f;
             if (v) {
