@@ -313,7 +313,12 @@ int32_t gf_sg_forward(gf_sg_model *model, const float *x, int32_t n, float *logi
  *   DIV        in0 / in1 (float)                             out: float
  *   BINOM_DRAW in0 uint32 bits, in1 mean, in2 var, in3 N     out: int32
  *   POIS_DRAW  in0 uint32 bits, in1 mean, in2 N              out: int32
- *   COPY       in0 float                                     out: float */
+ *   COPY       in0 float                                     out: float
+ * and the drift kernels' own forms, which have no host counterpart:
+ *   SQRT_POS    in0 float >= 2^-96                           out: float
+ *   DIV_MID     in0 / in1 (float, operands within 2^+-20)    out: float
+ *   ROUND_COUNT in0 float, in1 float (the largest count)     out: int32
+ *   BINOM_COUNT in0 uint32 bits, in1 mean, in2 var, in3 N    out: int32 in [0, N] */
 #define GF_MATH_PHILOX      0
 #define GF_MATH_U01         1
 #define GF_MATH_EXP         2
@@ -326,6 +331,10 @@ int32_t gf_sg_forward(gf_sg_model *model, const float *x, int32_t n, float *logi
 #define GF_MATH_ROUND_AWAY  9
 #define GF_MATH_COPY       10   /* out = in0 (float): a plain copy kernel for counter calibration */
 #define GF_MATH_F2I        11   /* out (int32) = saturating float -> int conversion of in0 */
+#define GF_MATH_SQRT_POS   12
+#define GF_MATH_DIV_MID    13
+#define GF_MATH_ROUND_COUNT 14
+#define GF_MATH_BINOM_COUNT 15
 int32_t gf_device_math(int32_t op, const void *in0, const void *in1, const void *in2, const void *in3,
                        void *out, int64_t n, int32_t device);
 

@@ -1,7 +1,9 @@
 /*
  * diag.hip -- gf_device_math: evaluates the device implementations of the
  * random-number and elementary functions on arrays, so their bit-exact
- * agreement with the host restatement can be checked function by function.
+ * agreement with the host restatement can be checked function by function:
+ * the general forms and, where the drift kernels have shorter ones of their
+ * own (sqrt_pos, div_mid, round_count, binom_count), those as well.
  */
 #include "gf_math.hpp"
 #include "gf_runtime.hpp"
@@ -36,6 +38,14 @@ static __global__ void k_math(int op, const void *in0, const void *in1, const vo
         case GF_MATH_ROUND_AWAY: fo[i] = round_away(f0[i]); break;
         case GF_MATH_COPY: fo[i] = f0[i]; break;
         case GF_MATH_F2I: io[i] = f2i_sat(f0[i]); break;
+        case GF_MATH_SQRT_POS: fo[i] = sqrt_pos(f0[i]); break;
+        case GF_MATH_DIV_MID: fo[i] = div_mid(f0[i], f1[i]); break;
+        case GF_MATH_ROUND_COUNT: io[i] = round_count(f0[i], f1[i]); break;
+        case GF_MATH_BINOM_COUNT: {
+            const float N = ((const float *)in3)[i];
+            io[i] = binom_count(u0[i], f1[i], f2[i], N, f2i_sat(N), ncdf_table(), expneg_table());
+            break;
+        }
         default: break;
         }
     }
@@ -46,13 +56,13 @@ static __global__ void k_math(int op, const void *in0, const void *in1, const vo
 extern "C" int32_t gf_device_math(int32_t op, const void *in0, const void *in1, const void *in2, const void *in3,
                                   void *out, int64_t n, int32_t device) {
     using namespace gf;
-    if (n <= 0 || !in0 || !out || op < 0 || op > GF_MATH_F2I) { set_error("gf_device_math: bad arguments"); return GF_ERR_ARG; }
+    if (n <= 0 || !in0 || !out || op < 0 || op > GF_MATH_BINOM_COUNT) { set_error("gf_device_math: bad arguments"); return GF_ERR_ARG; }
     GF_TRY(select_device(device));
     const size_t in_bytes = op == GF_MATH_PHILOX ? 24 : 4;
     const size_t out_bytes = op == GF_MATH_PHILOX ? 16 : 4;
     DevBuf<char> d0, d1, d2, d3, dout;
     GF_TRY(d0.alloc(n * in_bytes));
-    const bool extra = op == GF_MATH_DIV || op == GF_MATH_BINOM_DRAW || op == GF_MATH_POIS_DRAW;
+    const bool extra = op == GF_MATH_DIV || op == GF_MATH_BINOM_DRAW || op == GF_MATH_POIS_DRAW || op >= GF_MATH_DIV_MID;
     GF_TRY(d1.alloc(extra ? n * 4 : 1));
     GF_TRY(d2.alloc(extra ? n * 4 : 1));
     GF_TRY(d3.alloc(extra ? n * 4 : 1));

@@ -156,7 +156,8 @@ GF_HD float pow_f(float a, float b) {
  * reciprocal root g, s = x g, one Newton step s + (x - s s) g / 2 with the
  * residual in a fused multiply-add: five operations where the compiler's
  * expansion without its tiny-input scaling takes nine.  Equal to the IEEE
- * root for every float from 2^-96 up (all of them compared on the device);
+ * root for every finite float from 2^-96 up (tests/test_gpu_drift_math.py
+ * compares all of them on the device);
  * the host's sqrtf is correctly rounded. */
 GF_HD float sqrt_pos(float x) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -171,7 +172,9 @@ GF_HD float sqrt_pos(float x) {
 /* num / den, correctly rounded, for num = 0 or 2^-80 <= |num| <= 2^20 and
  * 2^-20 <= |den| <= 2^20: the compiler's expansion (reciprocal, one Newton
  * step, two residual steps) without the scaling and the special cases, which
- * do nothing in that range: 8 operations instead of 11. */
+ * do nothing in that range: 8 operations instead of 11 (compared on the
+ * device at random operands, the range's edges and quotients next to a
+ * rounding midpoint by tests/test_gpu_drift_math.py). */
 GF_HD float div_mid(float num, float den) {
 #if defined(__HIP_DEVICE_COMPILE__)
     float r = __builtin_amdgcn_rcpf(den);
@@ -462,8 +465,8 @@ GF_HD float binom_normal(float u, float mean, float var, const NcdfSeg *ncdf) {
 /* v rounded half away from zero and clamped to [0, top], NaN to 0, for an
  * integer top in [0, 2^31 - 128]: the clamp first, then floor(v + 1/2), which
  * v_cvt_rpi_i32_f32 computes without rounding v + 1/2 (equal to round half
- * away for every float >= 0, all of them compared on the device): two
- * operations instead of six. */
+ * away for every float >= 0; tests/test_gpu_drift_math.py compares all of
+ * them on the device): two operations instead of six. */
 GF_HD int round_count(float v, float top) {
     GF_STRICT_FP
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -491,7 +494,8 @@ GF_HD int binom_tail(float u, float mean, bool lo, float N, const ExpSeg *etab) 
  * (or binomial, N < 100) tails share one CDF inversion; the rest is the
  * rounded normal approximation.  The result equals the reference's draw wherever that is
  * >= 0; where the normal approximation goes below 0 it is some value <= 0
- * (round_away_nonneg), and the caller clamps the result to [0, N]. */
+ * (round_away_nonneg), and the caller clamps the result to [0, N].  The form
+ * that checks compare with; the kernels draw by binom_count. */
 GF_HD int binom_draw(uint32_t bits, float mean, float var, float N, const NcdfSeg *ncdf = ncdf_table(),
                      const ExpSeg *etab = expneg_table()) {
     GF_STRICT_FP
