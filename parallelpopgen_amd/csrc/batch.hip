@@ -394,7 +394,7 @@ static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims,
             if (lane >= off) x += y;
         }
         if (lane == 63) sh_w[w] = x;
-        __syncthreads();
+        sync_lds();
         int before = 0, round = 0;
 #pragma unroll
         for (int k = 0; k < 4; k++) {
@@ -413,7 +413,7 @@ static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims,
             }
         }
         carry += round;
-        __syncthreads();
+        sync_lds();
     }
     if (threadIdx.x == 0) {
         for (int k = 0; k < PRE_PAD; k++) pre[T + k] = carry;
@@ -425,7 +425,7 @@ static __global__ __launch_bounds__(256) void k_bt_scan(BSim *__restrict__ sims,
         if (r.g >= r.G) r.status = BS_DONE;
         __threadfence_block();
     }
-    __syncthreads();
+    sync_lds();
     if (w == 0) next_rows(sims, s, B);
 }
 
@@ -445,7 +445,7 @@ static __global__ __launch_bounds__(1024) void k_bt_status(const BSim *__restric
         st += __shfl_xor(st, off);
     }
     if ((threadIdx.x & 63) == 0) { sh_a[threadIdx.x >> 6] = a; sh_st[threadIdx.x >> 6] = st; }
-    __syncthreads();
+    sync_lds();
     if (threadIdx.x == 0) {
         int ta = 0, ts = 0;
         for (int k = 0; k < (int)blockDim.x / 64; k++) { ta += sh_a[k]; ts += sh_st[k]; }
@@ -514,13 +514,13 @@ static __global__ __launch_bounds__(WG) void k_bt_final(const BFin *__restrict__
     float *sh_lc = reinterpret_cast<float *>(sh_fin + n + 2);
     if (LDS)
         for (int k = threadIdx.x; k < half_n; k += WG) sh_lc[k] = lc[k];
-    __syncthreads();
+    sync_lds();
     const int per = (ntiles + (int)gridDim.x - 1) / (int)gridDim.x;
     const int g0 = (int)blockIdx.x * per, g1 = g0 + per < ntiles ? g0 + per : ntiles;
     const int w = wave_index();
     int sim = -1;
     auto flush = [&]() {   /* the sums of simulation `sim` */
-        __syncthreads();
+        sync_lds();
         if (LDS && sim >= 0) {
             unsigned long long *out = acc + (size_t)sim * (n + 2);
             for (int k = threadIdx.x; k < n + 2; k += WG)
@@ -541,7 +541,7 @@ static __global__ __launch_bounds__(WG) void k_bt_final(const BFin *__restrict__
             sim = lo;
             if (LDS) {
                 for (int k = threadIdx.x; k < n + 2; k += WG) sh_fin[k] = 0;   /* each its own words of the flush */
-                __syncthreads();
+                sync_lds();
             }
         }
         /* a lane per compacted index: half of the lanes would idle over the

@@ -27,6 +27,7 @@
 #define GF_DRIFT_HPP_
 
 #include "gf_math.hpp"
+#include "gf_sync.hpp"
 #include "../../include/gofish_capi.h"
 
 namespace gf {
@@ -317,17 +318,6 @@ __device__ __forceinline__ int64_t frag_slot(int li, int first, int tile, const 
         if (v[PRE_PAD - 1] > first + 63) break;
     }
     return (int64_t)s * WG + (li - at);
-}
-
-/* __syncthreads with this wave's LDS writes done first.  Said in so many
- * words: the compiler (ROCm 7.2) left the wait out before some barriers that
- * a loop's back edge or a long branch-free stretch led to, and another wave
- * then read the old words now and then. */
-__device__ __forceinline__ void sync_lds() {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#endif
-    __syncthreads();
 }
 
 /* the wave's index in its workgroup, as a scalar */

@@ -50,7 +50,7 @@ static __global__ __launch_bounds__(1024) void k_tile_chunk_sums(const unsigned 
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off);
     if ((threadIdx.x & 63) == 0) sh_w[threadIdx.x >> 6] = sum;
-    __syncthreads();
+    sync_lds();
     if (threadIdx.x == 0) {
         int t = 0;
         for (int k = 0; k < 16; k++) t += sh_w[k];
@@ -109,7 +109,7 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const unsigned int *__restri
             if (lane >= off) x += y;
         }
         if (lane == 63) sh_w[w] = x;
-        __syncthreads();
+        sync_lds();
         if (w == 0) {
             int t = lane < 16 ? sh_w[lane] : 0;
 #pragma unroll
@@ -119,7 +119,7 @@ __global__ __launch_bounds__(1024) void k_tile_scan(const unsigned int *__restri
             }
             if (lane < 16) sh_w[lane] = t;
         }
-        __syncthreads();
+        sync_lds();
         carry = 0;
 #pragma unroll
         for (int k = 0; k < 16; k++) carry += sh_before[k];
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(WG) void k_flag(const float *__restrict__ freq, int
         masks[(size_t)tile * (WG / 64) + w] = b;
         sh[w] = (unsigned int)__popcll(b);
     }
-    __syncthreads();
+    sync_lds();
     if (threadIdx.x == 0) {
         unsigned int c = 0;
         for (int k = 0; k < WG / 64; k++) c += sh[k];
@@ -248,12 +248,12 @@ static __global__ __launch_bounds__(1024) void k_scan_tiles(const unsigned int *
     unsigned int sum = 0;
     for (int k = b; k < e; k++) sum += tile_counts[first + k];
     sh[threadIdx.x] = sum;
-    __syncthreads();
+    sync_lds();
     for (int off = 1; off < T; off <<= 1) {
         unsigned int v = threadIdx.x >= (unsigned)off ? sh[threadIdx.x - off] : 0u;
-        __syncthreads();
+        sync_lds();
         sh[threadIdx.x] += v;
-        __syncthreads();
+        sync_lds();
     }
     unsigned int run = sh[threadIdx.x] - sum;
     for (int k = b; k < e; k++) {
@@ -461,10 +461,10 @@ static __global__ __launch_bounds__(256) void k_scan_partial(const int *__restri
     for (int64_t k = b + threadIdx.x; k < e; k += blockDim.x) s += in[k];
     __shared__ int64_t sh[256];
     sh[threadIdx.x] = s;
-    __syncthreads();
+    sync_lds();
     for (int o = 128; o > 0; o >>= 1) {
         if ((int)threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-        __syncthreads();
+        sync_lds();
     }
     if (threadIdx.x == 0) block_sums[blockIdx.x] = sh[0];
 }
@@ -477,12 +477,12 @@ static __global__ __launch_bounds__(1024) void k_scan_sums(int64_t *__restrict__
     int64_t s = 0;
     for (int k = b; k < e; k++) s += sums[k];
     sh[threadIdx.x] = s;
-    __syncthreads();
+    sync_lds();
     for (int off = 1; off < T; off <<= 1) {
         int64_t v = threadIdx.x >= (unsigned)off ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
+        sync_lds();
         sh[threadIdx.x] += v;
-        __syncthreads();
+        sync_lds();
     }
     int64_t run = sh[threadIdx.x] - s;
     for (int k = b; k < e; k++) { int64_t t = sums[k]; sums[k] = run; run += t; }
@@ -501,16 +501,16 @@ static __global__ __launch_bounds__(256) void k_scan_final(const int *__restrict
         const int64_t k = r + threadIdx.x;
         const int64_t v = k < e ? in[k] : 0;
         sh[threadIdx.x] = v;
-        __syncthreads();
+        sync_lds();
         for (int off = 1; off < 256; off <<= 1) {
             int64_t t = threadIdx.x >= (unsigned)off ? sh[threadIdx.x - off] : 0;
-            __syncthreads();
+            sync_lds();
             sh[threadIdx.x] += t;
-            __syncthreads();
+            sync_lds();
         }
         if (k < e) out[k] = run + sh[threadIdx.x] - v;
         const int64_t tot = sh[255];
-        __syncthreads();
+        sync_lds();
         run += tot;
     }
 }

@@ -39,7 +39,7 @@ static __global__ __launch_bounds__(HIST_WG) void k_pop_hist(const float *__rest
     const int b0 = (int)blockIdx.y * chunk;
     const int nb = Nc - b0 < chunk ? Nc - b0 : chunk;
     for (int k = threadIdx.x; k < nb; k += HIST_WG) sh_hist[k] = 0;
-    __syncthreads();
+    sync_lds();
     /* 64-bit index: i + stride must not wrap for M near INT_MAX */
     for (int64_t i = (int64_t)blockIdx.x * HIST_WG + threadIdx.x; i < M; i += (int64_t)gridDim.x * HIST_WG) {
         int idx = f2i_sat(round_away((float)Nc * freq[i]));
@@ -47,7 +47,7 @@ static __global__ __launch_bounds__(HIST_WG) void k_pop_hist(const float *__rest
         const unsigned int r = (unsigned int)(idx - b0);
         if (idx >= 0 && r < (unsigned int)nb) atomicAdd(&sh_hist[r], 1u);
     }
-    __syncthreads();
+    sync_lds();
     for (int k = threadIdx.x; k < nb; k += HIST_WG)
         if (sh_hist[k]) atomicAdd(&hist[b0 + k], sh_hist[k]);
 }
@@ -132,14 +132,14 @@ __global__ __launch_bounds__(WG) void k_sfs_row(const float *__restrict__ freq, 
     if (LDS) {
         for (int k = threadIdx.x; k < n + 2; k += WG) sh_sfs[k] = 0;
         for (int k = threadIdx.x; k < half_n; k += WG) sh_lc[k] = lc[k];
-        __syncthreads();
+        sync_lds();
     }
     for (int64_t i = (int64_t)blockIdx.x * WG + threadIdx.x; i < M; i += (int64_t)gridDim.x * WG) {
         if (LDS) sfs_add_mutation<LDS>(freq[i], n, half_n, sh_lc, sh_sfs, acc);
         else sfs_add_mutation<LDS>(freq[i], n, half_n, lc, sh_sfs, acc);
     }
     if (LDS) {
-        __syncthreads();
+        sync_lds();
         for (int k = threadIdx.x; k < n + 2; k += WG)
             if (sh_sfs[k]) atomicAdd(&acc[k], sh_sfs[k]);
     }
@@ -210,7 +210,7 @@ static __global__ __launch_bounds__(WG) void k_joint_sfs(const float *__restrict
     const int m_end = m_begin + JS_MUT_PER_WG < M ? m_begin + JS_MUT_PER_WG : M;
     for (int mb = m_begin; mb < m_end; mb += batch) {
         const int nm = m_end - mb < batch ? m_end - mb : batch;
-        __syncthreads();
+        sync_lds();
         for (int idx = threadIdx.x; idx < nm * (na + 1); idx += WG) {
             const int m = idx / (na + 1), k = idx % (na + 1);
             sa[idx] = sample_prob(fa[mb + m], na, k, la, half_a);
@@ -219,7 +219,7 @@ static __global__ __launch_bounds__(WG) void k_joint_sfs(const float *__restrict
             const int m = idx / (nb + 1), k = idx % (nb + 1);
             sb[idx] = sample_prob(fb[mb + m], nb, k, lb, half_b);
         }
-        __syncthreads();
+        sync_lds();
         for (int m = 0; m < nm; m++) {
             const float *pa = sa + (size_t)m * (na + 1);
             const float *pb = sb + (size_t)m * (nb + 1);
@@ -265,7 +265,7 @@ static __global__ __launch_bounds__(JW_WG) void k_joint_sfs_wave(const float *__
     extern __shared__ unsigned long long sh_bins[];   /* [na + 1][nb + 1] */
     const int B = (na + 1) * (nb + 1);
     for (int k = threadIdx.x; k < B; k += JW_WG) sh_bins[k] = 0;
-    __syncthreads();
+    sync_lds();
     const int lane = threadIdx.x & 63;
     const int waves = (int)gridDim.x * (JW_WG / 64);
     const int first = (int)blockIdx.x * (JW_WG / 64) + __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
@@ -308,7 +308,7 @@ static __global__ __launch_bounds__(JW_WG) void k_joint_sfs_wave(const float *__
             }
         }
     }
-    __syncthreads();
+    sync_lds();
     for (int k = threadIdx.x; k < B; k += JW_WG)
         if (sh_bins[k]) atomicAdd(&acc[k], sh_bins[k]);
 }

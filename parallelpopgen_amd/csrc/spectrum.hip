@@ -89,7 +89,7 @@ __global__ void k_sfs_prep(int n, int half_n, float *__restrict__ lc, unsigned l
     for (int k = threadIdx.x; k < n + 2; k += blockDim.x) acc[k] = 0ull;
     for (int k = 1 + (int)threadIdx.x; k < half_n; k += blockDim.x)
         lc[k] = log_f(((float)n + 1.0f - (float)k) / (float)k);
-    __syncthreads();
+    sync_lds();
     if (threadIdx.x == 0) {
         float a = 0.0f;
         lc[0] = 0.0f;

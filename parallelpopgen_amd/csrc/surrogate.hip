@@ -16,6 +16,7 @@
  *                    their Adam update in one kernel
  */
 #include "gf_runtime.hpp"
+#include "gf_sync.hpp"
 
 #include <cmath>
 #include <cstring>
@@ -226,16 +227,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void 
 #pragma unroll
                     for (int k = 0; k < 4; k++) pk[i][j][q][k] = (bf16)gelu(acc[i][j][4 * q + k] + bv[k]);
             }
-        __syncthreads();   /* every wave has read this layer's inputs */
+        sync_lds();   /* every wave has read this layer's inputs */
 #pragma unroll
         for (int i = 0; i < RB; i++)
 #pragma unroll
             for (int j = 0; j < JB; j++)
 #pragma unroll
                 for (int q = 0; q < 4; q++) *(bf16x4 *)&act[i * 32 + fr][32 * (JB * w + j) + 8 * q + 4 * hi] = pk[i][j][q];
-        __syncthreads();
+        sync_lds();
     };
-    __syncthreads();
+    sync_lds();
     /* layer 1: one k-step holds all six inputs */
     clear();
     rows(0, 0);
@@ -368,7 +369,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
     for (int i = 0; i <= NHID; i++)
         if (i < NHID || t < OUT_PAD) bias[i * HID + t] = bv[i];
-    __syncthreads();
+    sync_lds();
     if (z == 0 && w < 2) {   /* the inputs' batch fragments: 2 column blocks */
         bf16x8 v;
 #pragma unroll
@@ -406,14 +407,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         *(bf16x4 *)(base + ((int64_t)cb * cs + tile) * 512 + (fr + 32 * q) * 8 + 4 * hi) = v;
     };
     auto to_act = [&](const bf16x4 (&v)[2][2]) {
-        __syncthreads();   /* every wave has read this layer's rows */
+        sync_lds();   /* every wave has read this layer's rows */
 #pragma unroll
         for (int j = 0; j < 2; j++)
 #pragma unroll
             for (int q = 0; q < 2; q++)
 #pragma unroll
                 for (int k = 0; k < 4; k++) act[8 * q + 4 * hi + k][64 * w + 32 * j + fr] = v[j][q][k];
-        __syncthreads();
+        sync_lds();
     };
     auto activate = [&](int l) {
         bf16x4 v[2][2];
@@ -468,7 +469,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
     static_assert(OS <= TDEPTH, "the output layer's contraction is prefetched whole");
 #pragma unroll
     for (int u = 0; u < OS; u++) fetch(down(NHID, OS), u, OS, u);
-    __syncthreads();
+    sync_lds();
     {   /* softmax cross-entropy + w_tot (log-total - target)^2: 32 threads per row */
         float lv[4], mx = lg[lr][0];
 #pragma unroll
@@ -481,7 +482,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
 #pragma unroll
         for (int i = 0; i < 4; i++)
             if (lc + 32 * i < NBINS) ex[lr][lc + 32 * i] = __expf(lv[i] - mx);
-        __syncthreads();
+        sync_lds();
         float ls = 0.0f;
         if (lc == 0) {   /* the sum in bin order */
             float sum = 0.0f;
@@ -512,7 +513,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void k
         for (int off = 32; off > 0; off >>= 1) ce += __shfl_xor(ce, off);
         if (lane == 0) wloss[w] = ce;
     }
-    __syncthreads();
+    sync_lds();
     if (t == 0) {
         float sum = 0.0f;
         for (int k = 0; k < 8; k++) sum += wloss[k];
