@@ -358,9 +358,15 @@ const char *gf_last_error(void);
 int32_t gf_set_kernel_timing(int32_t enable);
 /* Number of generations the drift kernel advances per launch at most
  * (temporal blocking depth); 1 gives one generation per launch, 0 restores
- * the default (one population: 64 while at most 1.5e5 slots are in use, 48 up
- * to 4e5, 20 up to 1.2e6, 16 beyond; several: 64 up to 2e6 slots, 20 beyond, a launch
- * ending at each compaction generation either way; batches: 16). */
+ * the default.  One population whose model stays the same over the launch:
+ * 64 while at most 4e5 slots are in use, 48 up to 1.2e6, 40 up to 4e6, 24
+ * beyond; one whose model changes, or a run that never compacts: 64 up to
+ * 1.5e5, 48 up to 4e5, 20 up to 1.2e6, 16 beyond; in either case up to 3 fewer,
+ * so that the launch ends with a block of random words, and 10 at most where
+ * it would end with more than 2e8 slots.  Several: 64 up to 2e6 slots, 35
+ * beyond (20 above 2e8), a launch ending at each compaction generation.
+ * Batches: the length of 8 to 32 that their tuner measures as the best, or up
+ * to 3 fewer. */
 int32_t gf_set_generations_per_launch(int32_t k);
 int32_t gf_device_count(int32_t *out);
 

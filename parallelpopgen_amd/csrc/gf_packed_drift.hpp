@@ -18,8 +18,9 @@
  * one another.  Three populations over 2,000 generations, 1.4e7 slots in the
  * end: 90.9 -> 64.4 ms with 20 generations a launch, 56.7 with 35 (83.6
  * without packing).  Packing within each tile alone gave 80: one busy wave in
- * a workgroup of four.  Six waves per SIMD (72 VGPRs), not eight with spills:
- * 66.8 -> 64.3.
+ * a workgroup of four.  Six waves per SIMD (80 VGPRs, of which two
+ * populations with simple rows spill none, three 7, four 19), not eight with
+ * more spills: 66.8 -> 64.3.
  */
 #ifndef GF_PACKED_DRIFT_HPP_
 #define GF_PACKED_DRIFT_HPP_

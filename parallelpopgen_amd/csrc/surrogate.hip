@@ -9,7 +9,8 @@
  * forward, backward and Adam kernels.  Every matrix product runs on the
  * gfx950 matrix cores (v_mfma_f32_32x32x16_bf16) from operands kept in
  * fragment order, so that a wave's load is one contiguous KB:
- *   k_mlp            prediction: the whole network in one kernel
+ *   k_mlp            prediction: the whole network, inputs to logits, in one
+ *                    kernel (k_predict_stats: the ensemble's statistics)
  *   k_train_rows     training: forward, loss and the backward chain of 16
  *                    rows in one kernel
  *   k_train_weights  training: every layer's weight and bias gradients and
@@ -309,8 +310,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(EU))) void 
  * instead of 32 halve the vector work of a CU for the same stream, and 16
  * k-steps in flight instead of 8: 62 -> 49 us.  Rounding points and the order
  * of every sum (products by k, the softmax sum by bin) are those of the
- * layer-by-layer kernels it replaces: the same gradients bit for bit; the
- * loss, which those summed with one atomic per row, differs in its last bits.
+ * layer-by-layer kernels it replaced: compared with them, the gradients were
+ * the same bits; the loss, which those summed with one atomic per row, differs
+ * in its last bits.
  * One step (512 rows, 4 members) was 14 products of 6 to 20 us, loss 15,
  * column sums 5 x 4.6, Adam 17, gather and packing 9, together 300 us; now
  * this kernel and k_train_weights, 80 us. */
